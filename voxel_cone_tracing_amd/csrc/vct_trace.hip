@@ -124,20 +124,12 @@ struct Pair<VCT_RGBA8> {
   static constexpr bool kOn = true;
   using Raw = uint2;
   static __device__ __forceinline__ Raw make(uint32_t a, uint32_t b) { return pair_pack(a, b); }
-  static __device__ __forceinline__ float4 first(Raw v) { return Tex<VCT_RGBA8>::decode(v.x); }
-  static __device__ __forceinline__ float4 second(Raw v) { return Tex<VCT_RGBA8>::decode(v.y); }
 };
 template <int DT>
 struct Pair16 {
   static constexpr bool kOn = true;
   using Raw = uint4;
   static __device__ __forceinline__ Raw make(uint2 a, uint2 b) { return pair_pack(a, b); }
-  static __device__ __forceinline__ float4 first(Raw v) {
-    return Tex<DT>::decode(make_uint2((v.x & 0xffffu) | (v.y << 16), (v.z & 0xffffu) | (v.w << 16)));
-  }
-  static __device__ __forceinline__ float4 second(Raw v) {
-    return Tex<DT>::decode(make_uint2((v.x >> 16) | (v.y & 0xffff0000u), (v.z >> 16) | (v.w & 0xffff0000u)));
-  }
 };
 template <>
 struct Pair<VCT_FP16> : Pair16<VCT_FP16> {};
@@ -145,6 +137,10 @@ template <>
 struct Pair<VCT_BF16> : Pair16<VCT_BF16> {};
 
 __device__ __forceinline__ float4 f4(float x) { return make_float4(x, x, x, x); }
+// The four bytes of an RGBA8 texel as floats (v_cvt_f32_ubyte0..3).
+__device__ __forceinline__ float4 bytes4(uint32_t v) {
+  return make_float4((float)(v & 255u), (float)((v >> 8) & 255u), (float)((v >> 16) & 255u), (float)(v >> 24));
+}
 __device__ __forceinline__ float4 operator+(float4 a, float4 b) {
   return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
 }
@@ -302,9 +298,16 @@ struct PairWeights<VCT_BF16> {
   }
 };
 
-// Blend of the eight corners of one paired map: per channel, one FP32
-// two-term dot product (v_dot2_f32_f16 / _bf16) per corner pair for 16-bit
-// storage; RGBA8 decodes both texels and accumulates in FP32.
+// What a blended texel is multiplied by once its corners are summed: an RGBA8
+// texel counts in steps of 1/255 (unorm8), the others are stored as values.
+template <int DT>
+constexpr float kTexScale = DT == VCT_RGBA8 ? 1.0f / 255.0f : 1.0f;
+
+// Blend of the eight corners of one paired map, before kTexScale: per
+// channel, one FP32 two-term dot product (v_dot2_f32_f16 / _bf16) per corner
+// pair for 16-bit storage; RGBA8 converts each byte and accumulates in FP32
+// (the 1/255 is applied to the sum, so a byte costs one conversion and one
+// fused multiply-add).
 template <int DT>
 __device__ __forceinline__ float4 blend4(const PairWeights<DT>& W, const typename Pair<DT>::Raw (&r)[4]) {
   float4 acc = f4(0.0f);
@@ -327,7 +330,7 @@ __device__ __forceinline__ float4 blend4(const PairWeights<DT>& W, const typenam
   } else {
 #pragma unroll
     for (int k = 0; k < 4; ++k)
-      acc = acc + W.w[2 * k] * Pair<DT>::first(r[k]) + W.w[2 * k + 1] * Pair<DT>::second(r[k]);
+      acc = acc + W.w[2 * k] * bytes4(r[k].x) + W.w[2 * k + 1] * bytes4(r[k].y);
   }
   return acc;
 }
@@ -340,10 +343,24 @@ __device__ __forceinline__ float4 blend8(const Corners& c, const typename Tex<DT
   return acc;
 }
 
+__device__ __forceinline__ float4 fma4(float s, float4 a, float4 c) {
+  return make_float4(__builtin_fmaf(s, a.x, c.x), __builtin_fmaf(s, a.y, c.y), __builtin_fmaf(s, a.z, c.z),
+                     __builtin_fmaf(s, a.w, c.w));
+}
+
 // One level of sample_voxel: level 0 is the one map shared by all directions
 // (|d.x| + |d.y| + |d.z| times one trilinear fetch), a higher level blends
-// the three directional maps mx, my, mz.
-template <int DT>
+// the three directional maps mx, my, mz.  `ad` is |d| times kTexScale.
+//
+// Paired storage fetches the first map alike at every level (every map of
+// level 0 starts at offset 0) and lanes above level 0 add the other two:
+// most waves mix lanes of both kinds, and a path of its own for level 0
+// costs the wave a blend, four more loads and one more wait on memory per
+// sample (2560x1440 soup, the trace alone: FP16 2.18 -> 2.14 ms; RGBA8, with
+// the 1/255 out of the corner sums, 2.58 -> 2.23 ms).  FP32 storage has twice
+// the loads per map and no registers for a map held over the others: there
+// the two paths stay apart (one path measured 0.43 -> 0.58 ms at 1001x563).
+template <int DT, bool kMaybeLevel0>
 __device__ __forceinline__ float4 sample_level(const TraceArgs& A, const SamplerLds* S, float3 p, float3 ad, int mx,
                                                int my, int mz, int l) {
   Corners c;
@@ -351,19 +368,23 @@ __device__ __forceinline__ float4 sample_level(const TraceArgs& A, const Sampler
   if constexpr (Pair<DT>::kOn) {
     using PRaw = typename Pair<DT>::Raw;
     const PairWeights<DT> W(c);
-    if (l == 0) {
-      PRaw r[4];
-      gather4<DT>(A.vol, 0u, c, r);
-      return (ad.x + ad.y + ad.z) * blend4<DT>(W, r);
-    }
-    PRaw rx[4], ry[4], rz[4];
+    float ax = ad.x;
+    float4 yy = f4(0.0f), bz = f4(0.0f);
+    PRaw rx[4];
     gather4<DT>(A.vol, S->off[l][mx], c, rx);
-    gather4<DT>(A.vol, S->off[l][my], c, ry);
-    gather4<DT>(A.vol, S->off[l][mz], c, rz);
-    return ad.x * blend4<DT>(W, rx) + ad.y * blend4<DT>(W, ry) + ad.z * blend4<DT>(W, rz);
+    if (!kMaybeLevel0 || l > 0) {
+      PRaw ry[4], rz[4];
+      gather4<DT>(A.vol, S->off[l][my], c, ry);
+      gather4<DT>(A.vol, S->off[l][mz], c, rz);
+      yy = ad.y * blend4<DT>(W, ry);
+      bz = blend4<DT>(W, rz);
+    } else {
+      ax = ad.x + ad.y + ad.z;
+    }
+    return fma4(ad.z, bz, fma4(ax, blend4<DT>(W, rx), yy));
   }
   using Raw = typename Tex<DT>::Raw;
-  if (l == 0) {
+  if (kMaybeLevel0 && l == 0) {
     Raw r[8];
     gather8<DT>(A.vol, 0u, c, r);
     return (ad.x + ad.y + ad.z) * blend8<DT>(c, r);
@@ -388,8 +409,9 @@ __device__ __forceinline__ float4 sample_voxel(const TraceArgs& A, const Sampler
   lod = fminf(fmaxf(lod, 0.0f), lmax);
   const int l0 = (int)floorf(lod);
   const float t = lod - (float)l0;
-  float4 acc = sample_level<DT>(A, S, p, ad, mx, my, mz, l0);
-  if (t > 0.0f) acc = (1.0f - t) * acc + t * sample_level<DT>(A, S, p, ad, mx, my, mz, l0 + 1);
+  ad = make_float3(ad.x * kTexScale<DT>, ad.y * kTexScale<DT>, ad.z * kTexScale<DT>);
+  float4 acc = sample_level<DT, true>(A, S, p, ad, mx, my, mz, l0);
+  if (t > 0.0f) acc = (1.0f - t) * acc + t * sample_level<DT, false>(A, S, p, ad, mx, my, mz, l0 + 1);
   return acc;
 }
 
@@ -517,13 +539,18 @@ __device__ __forceinline__ bool cone_alive(const Cone& k, float3 origin, float m
            (sp.z < -margin && k.dir.z <= 0.0f) || (sp.z >= 1.0f + margin && k.dir.z >= 0.0f));
 }
 
+// log2 of a cone's diameter in voxels by the hardware instruction alone: the
+// diameter is at least 3 * 0.0174533 voxels (three voxels out, the narrowest
+// aperture), so log2f's scaling of subnormal arguments never applies.
+__device__ __forceinline__ float log2_of(float x) { return __builtin_amdgcn_logf(x); }
+
 template <int DT>
 __device__ __forceinline__ void cone_step(const TraceArgs& A, const SamplerLds* S, Cone& k, float3 origin, float vs,
                                           float fres) {
   const float3 sp = make_float3(k.dir.x * k.dist + origin.x, k.dir.y * k.dist + origin.y,
                                 k.dir.z * k.dist + origin.z);
   const float diam = k.dist * k.ap;
-  const float mip = fmaxf(log2f(diam * fres), 0.0f);
+  const float mip = fmaxf(log2_of(diam * fres), 0.0f);
   // face_indices (voxel_cone_tracing.frag:71-78): the map of each axis by the sign of dir
   const float3 ad = make_float3(fabsf(k.dir.x), fabsf(k.dir.y), fabsf(k.dir.z));
   const float4 s = sample_voxel<DT>(A, S, sp, ad, k.dir.x < 0.0f ? 0 : 1, k.dir.y < 0.0f ? 2 : 3,
