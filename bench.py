@@ -324,9 +324,10 @@ def main():
     achieved = amount / t_launch / 1e9
     load_peak = ctx.load_peak_gbps()
     log(f"bench: L1-hit 16-byte load ceiling {load_peak:.0f} GB/s")
-    # up to 9 diffuse cones without shadow lights: the 128-pixel (16x8) block shape
-    kname = f"trace_frame_kernel<{dt},Shape<128,2>>"
-    grid = (wl.width + 15) // 16 * 256 * ((wl.height + 7) // 8)
+    # blocks of 192 pixels (24x8) for the 16-bit types, 128 (16x8) for the others
+    px = 192 if dt in (L.FP16, L.BF16) else 128
+    kname = f"trace_frame_kernel<{dt},Shape<{px},2>>"
+    grid = (wl.width + px // 8 - 1) // (px // 8) * 256 * ((wl.height + 7) // 8)
     traffic = l2_hit = None
     from voxel_cone_tracing_amd.profile_summary import read_summary, read_traffic, summary_is_current
 

@@ -456,6 +456,38 @@ def test_trace_ragged_viewport_matches_oracle(gpu_available, orc):
     assert err <= 2e-3
 
 
+@pytest.mark.parametrize("dtype", [L.RGBA8, L.FP16, L.BF16, L.FP32])
+def test_trace_wide_blocks_ragged_viewport_matches_oracle(gpu_available, orc, dtype):
+    """A viewport past the small block shape (over 2^18 pixels) that no block
+    width divides (521 = 21 x 24 + 17 = 32 x 16 + 9; 509 = 63 x 8 + 5): the
+    wide shape of each storage type, its partial blocks on both edges and the
+    block rows past a multiple of 8.  A block's pixels are queued in sorted
+    order, so a pixel dropped or taken twice by the sort shows up as well."""
+    say(f"trace parity, ragged 521x509 viewport, dtype={dtype}")
+    W, H, res = 521, 509, 64
+    sc = SceneSpec("cornell", res=res, W=W, H=H, glass=True, phases=(True, True, True, True))
+    with Context(W, H) as ctx:
+        sc.build(ctx, dtype)
+        ctx.render()
+        img = ctx.download_image()
+        gp, gn = ctx.download_gbuffer()
+        l0 = decode_level(ctx.download_level(0), dtype)
+        mips = {(l, d): decode_level(ctx.download_level(l, d), dtype) for l in range(1, 7) for d in range(6)}
+    edge = np.zeros((H, W), bool)
+    edge[-6:, :] = True
+    edge[:, -18:] = True
+    edge[248:256, 240:288] = True  # two whole 24-pixel blocks, three 16-pixel ones
+    edge.reshape(-1)[np.random.default_rng(3).choice(W * H, 2000, replace=False)] = True
+    cov = gp[..., 3] != 0
+    pix = np.flatnonzero(edge & cov).astype(np.int64)
+    assert pix.size > 10000
+    want, _ = orc.trace(np.float32, res, 7, l0, mips, gp, gn, sc.mat_records, sc.lights, sc.cam, sc.cube_size,
+                        cone_set=sc.cone_set, phases=sc.phases, pixels=pix)
+    err = np.abs(img.reshape(-1, 4)[pix, :3] - want[:, :3]).max()
+    say(f"  {pix.size} pixels, max-abs vs FP32 oracle = {err:.3e}")
+    assert err <= 2e-3
+
+
 @pytest.mark.parametrize("view_dir,lod,extra,dtype", [
     (0, 0.0, {}, L.RGBA8), (3, 1.5, {}, L.RGBA8), (5, 4.0, {}, L.FP16),
     # the camera inside the box: clipped walls drawn as fans, in draw order

@@ -18,10 +18,10 @@
 // level and all 24 corner loads of a level are issued before the first is
 // used; level 0 is shared by all maps, so it is fetched once per step.
 //
-// Work mapping: a workgroup of 4 waves shades an 8x8 pixel block (lane =
-// pixel); the cones of a pixel are dealt over the 4 waves, and all lanes of
-// a wave march the same cone at the same time over neighbouring surface
-// points, so their texel fetches fall on the same bricks and L2 lines.
+// Work mapping: a workgroup of 4 waves shades a block of 64 to 192 pixels
+// whose cones form one queue for its lanes (shade_block), ordered so that the
+// lanes of a wave march like cones over neighbouring surface points and their
+// texel fetches fall on the same cache lines.
 // Accumulation is FP32 for every storage type.
 #include <algorithm>
 #include <cmath>
@@ -450,28 +450,63 @@ __device__ __forceinline__ float3 refract3(float3 I, float3 N, float eta) {
 // in LDS as soon as its cone ends, so lanes do not idle while the longest cone
 // of a wave finishes.  The same waves then compose their pixels in the
 // reference's order (voxel_cone_tracing.frag:246-275).
+//
+// What bounds the march is the number of cache lines a wave's load touches,
+// not its instructions (cones set up 64 at a time for the idle lanes to take,
+// which raises the lanes in use, measured no faster), so the queue takes the
+// block's pixels sorted by the octant of their normal and their position:
+// the lanes of a wave then read the same maps around the same place (128
+// pixels, 2560x1440 soup: FP16 2.08 -> 1.94 ms, RGBA8 2.18 -> 2.13;
+// pixel-major items instead of job-major ones 3.1 ms).
 // job codes: 0..15 diffuse cone k, then:
 constexpr int kJobSpecular = 16, kJobRefraction = 17, kJobShadow = 18;  // kJobShadow + light
 constexpr int kMaxJobs = kJobShadow + VCT_MAX_LIGHTS;
 // idle lanes of a wave that trigger a refill: a refill costs the whole wave
-// its set-up; measured on the 1M-triangle soup with 128-pixel blocks: 8 ->
-// 2.69 ms, 16 -> 2.60 ms, 24 -> 2.55 ms, 32 -> 2.59 ms, 48 -> 2.77 ms
-constexpr int kRefillMin = 24;
+// its set-up; measured on the 1M-triangle soup at 2560x1440, FP16 / RGBA8:
+// 16 -> 1.90 / 2.02 ms, 24 -> 1.90 / 2.06, 32 -> 1.96 / 2.11, 40 -> 2.04 / 2.21
+constexpr int kRefillMin = 16;
 
 // Block shapes: pixels per workgroup and the shadow-light slots in LDS.
 // Cones are short in cluttered scenes (6.2 steps per cone of a covered pixel
-// on a 1M-triangle soup), so a queue of 64 pixels x 10 cones gives each of the 256 lanes only
-// 2.5 items and the drain at its end leaves a third of the lanes idle; more
-// pixels per workgroup shorten the drain relative to the work.  The wide
-// shape holds shadow results of up to 2 lights; more lights use the full one.
+// on a 1M-triangle soup), so a queue of 64 pixels x 10 cones gives each of the
+// 256 lanes only 2.5 items and the drain at its end leaves a third of the
+// lanes idle; more pixels per workgroup shorten the drain relative to the
+// work.  The full shape holds shadow results of every light, the others of up
+// to 2.
 template <int NPIX_, int NSHADOW_>
 struct Shape {
   static constexpr int NPIX = NPIX_, NSHADOW = NSHADOW_, NSUB = NPIX_ / 64;
-  static constexpr int BX = NSUB >= 2 ? 2 : 1;  // sub-blocks side by side (BX x NSUB/BX of 8x8)
+  static constexpr int BX = NSUB == 3 ? 3 : (NSUB >= 2 ? 2 : 1);  // sub-blocks side by side (BX x NSUB/BX of 8x8)
+  static_assert(NSUB <= 4, "one set-up wave per sub-block; pixel numbers are bytes");
 };
-using ShapeWide = Shape<128, 2>;
 using ShapeFull = Shape<128, VCT_MAX_LIGHTS>;
-using ShapeSmall = Shape<64, 2>;  // small viewports (see launch_trace)
+using ShapeTile = Shape<128, 2>;  // 32x32 tiles and long pixel lists
+using ShapeSmall = Shape<64, 2>;  // small viewports and lists (see launch_trace)
+// Whole viewports of the 16-bit types: 31 KB of LDS per 192 pixels let 5
+// workgroups share a CU, as many as their registers do, and a longer run of
+// sorted pixels shares more of its fetches (2560x1440 soup, FP16: 1.96 ms
+// with 128 pixels, 1.89 with 192; 256 fit 4 workgroups only, 1.92).  RGBA8
+// runs 6 waves per SIMD, which 128 pixels fit and 192 do not (2.08 against
+// 2.18 ms with 256), and FP32 measures alike.
+template <int DT>
+struct WideOf {
+  using type = ShapeTile;
+};
+template <>
+struct WideOf<VCT_FP16> {
+  using type = Shape<192, 2>;
+};
+template <>
+struct WideOf<VCT_BF16> {
+  using type = Shape<192, 2>;
+};
+
+// Waves per SIMD the kernels are compiled for, and what measured (2560x1440
+// soup, RGBA8: 6 waves in 79 registers 2.08 ms, 5 waves 2.13; 1001x563,
+// FP32: 4 waves in 126 registers 0.367 ms, 5 waves and 24 bytes of scratch
+// 0.398; the 16-bit types hold 12 paired loads in flight and spill past 5).
+template <int DT>
+constexpr int kTraceWaves = DT == VCT_RGBA8 ? 6 : (DT == VCT_FP32 ? 4 : 5);
 
 // 32.32 fixed point of a non-negative cone colour channel (< 2^31): sums of
 // these are exact, so the diffuse cones of a pixel may finish in any order.
@@ -487,9 +522,7 @@ struct ShadeLds {
   float spec_ap[SH::NPIX], eta[SH::NPIX];
   unsigned long long refr_mask[SH::NSUB];  // shading pixels with a transmissive material, per sub-block
   int sub_count[SH::NSUB];                 // shading pixels per sub-block
-  // each set-up thread's G-buffer index (~0: none) and output index, kept
-  // here over the cone queue instead of in registers
-  uint32_t gidx[SH::NPIX], oidx[SH::NPIX];
+  uint32_t key[SH::NPIX];  // order of the block's pixels in the queue
   int npx, njobs, next_item;
   uint8_t px_of[SH::NPIX];  // the block's shading pixels, compacted
   int8_t jobs[kMaxJobs];
@@ -577,17 +610,23 @@ __device__ __forceinline__ float3 light_dir(const TraceArgs& A, int li, float3 p
 template <int N>
 __device__ __forceinline__ float3 ld3(const float (*a)[N], int p) { return make_float3(a[0][p], a[1][p], a[2][p]); }
 
-// Shades the block's pixels; (px, py, oidx, valid) are the thread's pixel in
-// sub-block (wave index mod NSUB).  L->next_item must be 0 and visible to the
-// workgroup on entry.
-template <int DT, class SH>
-__device__ __forceinline__ void shade_block(const TraceArgs& A, int px, int py, size_t oidx, bool valid,
-                                            ShadeLds<SH>* L, const SamplerLds* S) {
+// Shades the block's pixels; where(sub, lane, px, py, oidx, valid) gives the
+// pixel of a lane of sub-block `sub`, where its result goes and whether it is
+// traced.  L->next_item must be 0 and visible to the workgroup on entry.
+template <int DT, class SH, class Where>
+__device__ __forceinline__ void shade_block(const TraceArgs& A, Where&& where, ShadeLds<SH>* L, const SamplerLds* S) {
   const int lane = threadIdx.x & 63;
   const int grp = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // wave-uniform: a scalar register
   const int me = grp * 64 + lane;  // the thread's pixel in the block (set-up and composition waves)
-  valid = valid && px < A.W && py < A.H;
-  size_t idx = valid ? (size_t)py * A.W + px : 0;
+  size_t idx = 0, oidx = 0;
+  bool valid = false;
+  auto locate = [&](int ln) {
+    int px, py;
+    where(grp, ln, px, py, oidx, valid);
+    valid = valid && px < A.W && py < A.H;
+    idx = valid ? (size_t)py * A.W + px : 0;
+  };
+  if (grp < SH::NSUB) locate(lane);
   const float sqrt3 = 1.73205080757f;
   const int nd = A.en_diffuse ? A.cones.n : 0;
   const bool do_spec = A.en_specular != 0;
@@ -609,16 +648,13 @@ __device__ __forceinline__ void shade_block(const TraceArgs& A, int px, int py, 
     }
   };
   unsigned long long shade = 0ull;
-  int smode = 0;
+  uint32_t mykey = ~0u;
   if (grp < SH::NSUB) {
-    L->gidx[me] = valid ? (uint32_t)idx : ~0u;
-    L->oidx[me] = (uint32_t)oidx;
     float4 gp, gn;
     const DevMaterial* m;
     float3 pos;
     int mode;
     pixel(gp, gn, m, pos, mode);
-    smode = mode;
     const float3 n = make_float3(gn.x, gn.y, gn.z);
     const float3 cam = make_float3(A.cam[0], A.cam[1], A.cam[2]);
     const float3 vd = normalize3(make_float3(gp.x - cam.x, gp.y - cam.y, gp.z - cam.z));
@@ -643,6 +679,15 @@ __device__ __forceinline__ void shade_block(const TraceArgs& A, int px, int py, 
       dst[q][2][me] = vals[q].z;
     }
     shade = __ballot(mode == 3);
+    // the pixel's place in the queue's order: the octant of its normal, then
+    // its position in cells of two voxels along the Morton curve
+    {
+      const float sc = 0.5f * (float)min(A.res, 256);
+      auto cell = [&](float v) { return (uint32_t)min(max((int)(v * sc), 0), 127); };
+      const uint32_t oct = (n.x < 0.0f ? 1u : 0u) | (n.y < 0.0f ? 2u : 0u) | (n.z < 0.0f ? 4u : 0u);
+      mykey = mode == 3 ? (((oct << 21) | morton3(cell(pos.x), cell(pos.y), cell(pos.z))) << 8) | (uint32_t)me : ~0u;
+      L->key[me] = mykey;
+    }
     const unsigned long long refr = __ballot(mode == 3 && do_spec && illum_transmissive(m->illum));
     if (lane == 0) {
       L->sub_count[grp] = __popcll(shade);
@@ -652,15 +697,17 @@ __device__ __forceinline__ void shade_block(const TraceArgs& A, int px, int py, 
   __syncthreads();
   if (grp < SH::NSUB) {
     // the block's shading pixels, compacted in sub-block order
-    int base = 0, total = 0;
+    int total = 0;
     bool refr = false;
 #pragma unroll
     for (int w = 0; w < SH::NSUB; ++w) {
-      base += w < grp ? L->sub_count[w] : 0;
       total += L->sub_count[w];
       refr = refr || L->refr_mask[w] != 0ull;
     }
-    if (smode == 3) L->px_of[base + __popcll(shade & ((1ull << lane) - 1ull))] = (uint8_t)me;
+    uint32_t rank = 0;  // keys are distinct: a pixel's place is the number of smaller ones
+#pragma unroll 8
+    for (int q = 0; q < SH::NPIX; ++q) rank += L->key[q] < mykey ? 1u : 0u;
+    if (mykey != ~0u) L->px_of[rank] = (uint8_t)me;
     if (me == 0) {
       L->npx = total;
       int nj = 0;  // longest kinds first
@@ -678,8 +725,8 @@ __device__ __forceinline__ void shade_block(const TraceArgs& A, int px, int py, 
   const float margin = 0.5f * (float)(1u << (A.levels - 1)) * vs;
   const int npx = L->npx;
   const int nitems = npx * L->njobs;
-  // it / npx as (it * ceil(2^20 / npx)) >> 20: exact for it < kMaxJobs * 128 and npx <= 128
-  const uint32_t npx_inv = npx ? (1u << 20) / (uint32_t)npx + (((1u << 20) % (uint32_t)npx) ? 1u : 0u) : 0u;
+  // it / npx as (it * ceil(2^22 / npx)) >> 22: exact for it < kMaxJobs * npx and npx <= 256
+  const uint32_t npx_inv = npx ? (1u << 22) / (uint32_t)npx + (((1u << 22) % (uint32_t)npx) ? 1u : 0u) : 0u;
   // the lane's cone: job << 8 | pixel while it marches, -1 while it idles
   int cur = -1;
   unsigned long long wave_steps = 0;  // cone steps of the wave (uniform)
@@ -719,7 +766,7 @@ __device__ __forceinline__ void shade_block(const TraceArgs& A, int px, int py, 
         drained = true;
         continue;
       }
-      const int j = (int)(((uint32_t)it * npx_inv) >> 20);
+      const int j = (int)(((uint32_t)it * npx_inv) >> 22);
       const int job = L->jobs[j];
       const int pix = L->px_of[it - j * npx];
       if (job == kJobRefraction && !((L->refr_mask[pix >> 6] >> (pix & 63)) & 1ull)) continue;  // opaque: no item
@@ -764,15 +811,13 @@ __device__ __forceinline__ void shade_block(const TraceArgs& A, int px, int py, 
   __syncthreads();
   // ---- composition (waves 0..NSUB-1, lane = pixel) -----------------------------------
   if (grp >= SH::NSUB) return;
-  // the thread's slot again, from the scalar wave index and the hardware lane
-  // id: nothing per lane is held over the cone queue
-  const int lane_c = (int)__lane_id(), me_c = grp * 64 + lane_c;
-  {
-    const uint32_t g = ((const volatile uint32_t*)L->gidx)[me_c];
-    valid = g != ~0u;
-    idx = valid ? (size_t)g : 0;
-    oidx = ((const volatile uint32_t*)L->oidx)[me_c];
-  }
+  // the thread's pixel again, from the scalar wave index and a lane id the
+  // compiler cannot match with the first: nothing per lane is held over the
+  // cone queue
+  int lane_c = (int)__lane_id();
+  asm volatile("" : "+v"(lane_c));
+  const int me_c = grp * 64 + lane_c;
+  locate(lane_c);
   float4 gp, gn;
   const DevMaterial* mp;
   float3 pos;
@@ -874,10 +919,9 @@ __device__ __forceinline__ void shade_block(const TraceArgs& A, int px, int py, 
 // FP32 path keeps 20 bytes per lane in scratch at this occupancy): the 12
 // paired loads of a three-map level are in flight together.
 template <int DT, class SH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void trace_frame_kernel(TraceArgs A) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kTraceWaves<DT>))) void trace_frame_kernel(TraceArgs A) {
   __shared__ ShadeLds<SH> s_shade;
   __shared__ SamplerLds s_sampler;
-  const int lane = threadIdx.x & 63, sub = (int)(threadIdx.x >> 6) % SH::NSUB;
   sampler_init<DT>(A, &s_sampler);
   if (threadIdx.x == 0) s_shade.next_item = 0;
   __syncthreads();
@@ -895,9 +939,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void t
     b = ((q / gx) * 8u + (b & 7u)) * gx + q % gx;
   }
   const int bx = (int)(b % gx), by = (int)(b / gx);
-  const int px = bx * (8 * SH::BX) + (sub % SH::BX) * 8 + (lane & 7);
-  const int py = by * (8 * (SH::NSUB / SH::BX)) + (sub / SH::BX) * 8 + (lane >> 3);
-  shade_block<DT, SH>(A, px, py, (size_t)py * A.W + px, true, &s_shade, &s_sampler);
+  shade_block<DT, SH>(
+      A,
+      [&](int sub, int lane, int& px, int& py, size_t& oidx, bool& valid) {
+        px = bx * (8 * SH::BX) + (sub % SH::BX) * 8 + (lane & 7);
+        py = by * (8 * (SH::NSUB / SH::BX)) + (sub / SH::BX) * 8 + (lane >> 3);
+        oidx = (size_t)py * A.W + px;
+        valid = true;
+      },
+      &s_shade, &s_sampler);
 }
 
 // Chunks (npix pixels each) of a list launch.
@@ -942,18 +992,19 @@ __device__ __forceinline__ void list_chunk(const TraceArgs& A, uint32_t c, uint3
 // (A fixed grid striding over the chunks measured slower: the loop costs the
 // kernel registers and spills at 4 waves per SIMD.)
 template <int DT, class SH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void trace_list_kernel(TraceArgs A) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kTraceWaves<DT>))) void trace_list_kernel(TraceArgs A) {
   __shared__ ShadeLds<SH> s_shade;
   __shared__ SamplerLds s_sampler;
   if (blockIdx.x >= list_chunks(A, SH::NPIX)) return;
   sampler_init<DT>(A, &s_sampler);
   if (threadIdx.x == 0) s_shade.next_item = 0;
   __syncthreads();
-  int px, py;
-  size_t oidx;
-  bool valid;
-  list_chunk(A, blockIdx.x, SH::NSUB, (threadIdx.x >> 6) % SH::NSUB, threadIdx.x & 63, px, py, oidx, valid);
-  shade_block<DT, SH>(A, px, py, oidx, valid, &s_shade, &s_sampler);
+  shade_block<DT, SH>(
+      A,
+      [&](int sub, int lane, int& px, int& py, size_t& oidx, bool& valid) {
+        list_chunk(A, blockIdx.x, SH::NSUB, (uint32_t)sub, lane, px, py, oidx, valid);
+      },
+      &s_shade, &s_sampler);
 }
 
 // Builds the x-paired copy of every (level, map) of the volume in one launch:
@@ -1215,7 +1266,8 @@ static int launch_trace(vct_context* ctx, const TraceArgs& A, const TraceSelect&
   // 3.257 -> 3.244 ms for the frame.
   if (wide && !sel.tile_list && (sel.pix_list ? (size_t)sel.npix_list : (size_t)W * H) <= (1u << 18))
     launch_shape<DT, ShapeSmall>(ctx, A, sel, W, H);
-  else if (wide) launch_shape<DT, ShapeWide>(ctx, A, sel, W, H);
+  else if (wide && (sel.pix_list || sel.tile_list)) launch_shape<DT, ShapeTile>(ctx, A, sel, W, H);
+  else if (wide) launch_shape<DT, typename WideOf<DT>::type>(ctx, A, sel, W, H);
   else launch_shape<DT, ShapeFull>(ctx, A, sel, W, H);
   return VCT_OK;
 }
@@ -1278,7 +1330,7 @@ int vct_trace_select(vct_context* ctx, const float4* gpos, const float4* gnrm, f
   A.lights.count = n;
   // the wide shape holds the shadows of up to 2 lights
   const int nshadow = (ctx->en_direct && ctx->en_shadow) ? n : 0;
-  const bool wide = nshadow <= ShapeWide::NSHADOW;
+  const bool wide = nshadow <= ShapeTile::NSHADOW;
   switch (ctx->dtype) {
     case VCT_RGBA8: rc = launch_trace<VCT_RGBA8>(ctx, A, sel, W, H, wide); break;
     case VCT_FP16: rc = launch_trace<VCT_FP16>(ctx, A, sel, W, H, wide); break;
