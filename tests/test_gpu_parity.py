@@ -316,6 +316,54 @@ def test_gbuffer_many_models(gpu_available, orc):
     assert np.array_equal(bits(gn), bits(n32))
 
 
+def large_triangles(n, seed):
+    """Triangles of 0.01 to 3 world units around and across the grid, every
+    fourth a sliver, every fifth flat in a coordinate plane."""
+    rng = np.random.default_rng(seed)
+    size = np.exp(rng.uniform(np.log(0.01), np.log(3.0), (n, 1, 1)))
+    p = rng.uniform(-1.3, 1.3, (n, 1, 3)) + size * rng.standard_normal((n, 3, 3)) * 0.5
+    k = np.arange(n)
+    sl = k % 4 == 0
+    p[sl, 2] = p[sl, 0] + (p[sl, 1] - p[sl, 0]) * rng.uniform(0, 1, (sl.sum(), 1)) + \
+        1e-3 * rng.standard_normal((sl.sum(), 3))
+    for a in range(3):
+        f = (k % 5 == 0) & (k % 3 == a)
+        p[f, :, a] = p[f, :1, a]
+    nrm = np.cross(p[:, 1] - p[:, 0], p[:, 2] - p[:, 0])
+    nrm /= np.maximum(np.linalg.norm(nrm, axis=1, keepdims=True), 1e-12)
+    return (np.ascontiguousarray(p.reshape(n, 9).astype(np.float32)),
+            np.ascontiguousarray(np.repeat(nrm[:, None], 3, 1).reshape(n, 9).astype(np.float32)))
+
+
+@pytest.mark.parametrize("n,res,W,H", [(1, 64, 40, 40), (65, 128, 700, 500), (4096, 64, 333, 190), (4097, 32, 64, 64),
+                                       (20000, 128, 200, 120)])
+def test_large_triangles_bit_exact(gpu_available, orc, n, res, W, H):
+    """The set-up and list kernels take 64, 32 (4097 triangles) or 8 lanes per
+    triangle here; boxes of more than 8 bricks or tiles go to the whole wave,
+    which drops bricks and tiles the triangle cannot reach.  Level 0 in both
+    averaging modes and the G-buffer must not notice."""
+    say(f"large triangles n={n} res={res} {W}x{H}")
+    sc = SceneSpec("soup", ntri=n, res=res, W=W, H=H)
+    sc.pos, sc.nrm = large_triangles(n, n)
+    want = orc.voxelize(res, sc.cube_size, sc.M, sc.pos, sc.nrm, sc.tri_mat, sc.mat_records, sc.lights,
+                        want=("q32", "ref"))
+    p32, n32, _, _, _ = orc.gbuffer(W, H, sc.view, sc.proj, [(sc.M, sc.pos, sc.nrm, sc.tri_mat)])
+    with Context(W, H) as ctx:
+        sc.build(ctx, L.FP16, L.AVG_EXACT)
+        for _ in range(2):  # the second frame sizes its lists from the first one's count
+            ctx.voxelize()
+            got = ctx.download_level(0)
+            assert np.array_equal(bits(got), bits(encode_level(want["q32"], L.FP16)))
+        ctx.gbuffer()
+        gp, gn = ctx.download_gbuffer()
+        ctx.set_grid(res, 6, L.RGBA8, L.AVG_REFERENCE)
+        ctx.voxelize()
+        ref = ctx.download_level(0)
+    assert np.array_equal(ref, want["ref"])
+    assert np.array_equal(bits(gp), bits(p32))
+    assert np.array_equal(bits(gn), bits(n32))
+
+
 # ---- trace (kernel c) ----------------------------------------------------------------
 @pytest.mark.parametrize("kind,dtype,res,ntri", [("cornell", L.RGBA8, 64, 34), ("cornell", L.FP16, 64, 34),
                                                  ("soup", L.FP16, 64, 4000), ("soup", L.BF16, 64, 4000),

@@ -341,6 +341,46 @@ __device__ __forceinline__ TileRange tile_range(const GRec& r) {
   return t;
 }
 
+// A box of few tiles is listed whole, lane by lane with one atomic per
+// distinct tile of the wave.  Larger ones would hold their wave for a round
+// trip per tile, so the wave takes them one after another, its lanes over the
+// triangle's tiles, and drops the tiles that lie outside an edge (4,000
+// triangles at 1001x563: bin count 28 and list write 41 us before, the 34
+// triangles of the Cornell box at 512x512: 80 and 130 us).
+constexpr int kSmallRange = 8;
+
+// The fields of a wave lane's record that its tiles depend on, in every lane
+// (scalar registers: `lead` is uniform).
+__device__ __forceinline__ GRec g_rec_of_lane(const GRec& r, int lead) {
+  GRec u;
+  auto rl = [lead](int v) { return __builtin_amdgcn_readlane(v, lead); };
+  for (int v = 0; v < 3; ++v) {
+    u.X[v] = rl(r.X[v]);
+    u.Y[v] = rl(r.Y[v]);
+  }
+  u.i0 = (int16_t)rl(r.i0);
+  u.j0 = (int16_t)rl(r.j0);
+  u.i1 = (int16_t)rl(r.i1);
+  u.j1 = (int16_t)rl(r.j1);
+  u.swap = (uint32_t)rl((int)r.swap);
+  u.area = 0;
+  return u;
+}
+
+// False only where no pixel of the triangle's box in tile (tx, ty) is inside
+// all three edges (exact integers: the largest edge value over the box's
+// corner pixels is negative).
+__device__ __forceinline__ bool g_tile_reached(const GRec& r, int tx, int ty) {
+  const int i0 = max((int)r.i0, tx * kTile), i1 = min((int)r.i1, tx * kTile + kTile - 1);
+  const int j0 = max((int)r.j0, ty * kTile), j1 = min((int)r.j1, ty * kTile + kTile - 1);
+  GEdges e;
+  g_edges(g_setup_of(r), i0, j0, e);
+  for (int k = 0; k < 3; ++k)
+    if (e.w[k] + max((int64_t)0, e.di[k] * (int64_t)(i1 - i0)) + max((int64_t)0, e.dj[k] * (int64_t)(j1 - j0)) < 0)
+      return false;
+  return true;
+}
+
 __device__ __forceinline__ void g_rec_from(const GSetup& s, GRec& r) {
 #pragma clang fp contract(off)
   r.area = s.area;
@@ -385,22 +425,28 @@ __device__ __noinline__ GRec g_fan_record(const GParams& p, uint32_t t, uint32_t
   return r;
 }
 
-// 1. setup (lane per stored triangle): clip, snap, bounding box; count the
-//    triangle into every 32x32 tile its bounding box overlaps.  A triangle that
+// 1. setup (1 << lsh lanes per stored triangle, the first of them sets it up):
+//    clip, snap, bounding box; count the triangle into the 32x32 tiles its
+//    bounding box overlaps.  A triangle that
 //    needs clipping is only flagged and listed here: its fans are counted and
 //    written by g_fan_count_kernel / g_fan_write_kernel, so that the polygon
 //    code (private arrays, calls) stays out of this kernel.
 __global__ __launch_bounds__(256) void g_bin_count_kernel(GParams p, GRec* __restrict__ recs, uint32_t* tile_count,
-                                                          int tiles_x, uint32_t* clip_list, uint32_t* clip_count) {
+                                                          int tiles_x, uint32_t* clip_list, uint32_t* clip_count,
+                                                          int lsh) {
 #pragma clang fp contract(off)
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t t = gid >> lsh;
+  const bool own = (gid & ((1u << lsh) - 1u)) == 0u && t < p.ntri;
+  const int lane = threadIdx.x & 63;
   GRec r;
+  memset(&r, 0, sizeof(r));
   r.i0 = 1;
   r.i1 = 0;
   r.j0 = 1;
   r.j1 = 0;
   bool clipped = false;
-  if (t < p.ntri) {
+  if (own) {
     const int d = g_find_draw(p, t);
     const GDraw& dr = p.draws[d];
     float clip[3][4];
@@ -423,10 +469,19 @@ __global__ __launch_bounds__(256) void g_bin_count_kernel(GParams p, GRec* __res
   const uint32_t slot = wave_add_one(clip_count, 0u, clipped);
   if (clipped) clip_list[slot] = t;
   const TileRange tr = tile_range(r);
-  for (int k = 0; __ballot(k < tr.n) != 0ull; ++k) {
-    const bool act = k < tr.n;
+  const int nsmall = tr.n <= kSmallRange ? tr.n : 0;
+  for (int k = 0; __ballot(k < nsmall) != 0ull; ++k) {
+    const bool act = k < nsmall;
     const uint32_t key = act ? (uint32_t)((tr.ty0 + k / tr.tw) * tiles_x + tr.tx0 + k % tr.tw) : 0u;
     wave_add_one(tile_count, key, act);
+  }
+  for (unsigned long long big = __ballot(tr.n > kSmallRange); big; big &= big - 1ull) {
+    const GRec u = g_rec_of_lane(r, __ffsll((long long)big) - 1);
+    const TileRange ur = tile_range(u);
+    for (int k = lane; k < ur.n; k += 64) {
+      const int tx = ur.tx0 + k % ur.tw, ty = ur.ty0 + k / ur.tw;
+      if (g_tile_reached(u, tx, ty)) atomicAdd(tile_count + ty * tiles_x + tx, 1u);
+    }
   }
 }
 
@@ -456,18 +511,35 @@ __global__ __launch_bounds__(256) void g_fan_count_kernel(GParams p, GRec* __res
 //    tile's list (clipped triangles have no tiles here).
 __global__ __launch_bounds__(256) void g_bin_write_kernel(uint32_t ntri, const GRec* __restrict__ recs,
                                                           const uint32_t* __restrict__ tile_off, uint32_t* cursor,
-                                                          int tiles_x, uint32_t* __restrict__ list) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+                                                          int tiles_x, uint32_t* __restrict__ list, int lsh) {
+  const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t t = gid >> lsh;
+  const bool own = (gid & ((1u << lsh) - 1u)) == 0u && t < ntri;
+  const int lane = threadIdx.x & 63;
   GRec r;
+  memset(&r, 0, sizeof(r));
   r.i0 = 1;
   r.i1 = 0;
-  if (t < ntri) r = recs[t];
+  if (own) r = recs[t];
   const TileRange tr = tile_range(r);
-  for (int k = 0; __ballot(k < tr.n) != 0ull; ++k) {
-    const bool act = k < tr.n;
+  const int nsmall = tr.n <= kSmallRange ? tr.n : 0;
+  for (int k = 0; __ballot(k < nsmall) != 0ull; ++k) {
+    const bool act = k < nsmall;
     const uint32_t key = act ? (uint32_t)((tr.ty0 + k / tr.tw) * tiles_x + tr.tx0 + k % tr.tw) : 0u;
     const uint32_t slot = wave_add_one(cursor, key, act);
     if (act) list[tile_off[key] + slot] = t;
+  }
+  for (unsigned long long big = __ballot(tr.n > kSmallRange); big; big &= big - 1ull) {
+    const int lead = __ffsll((long long)big) - 1;
+    const GRec u = g_rec_of_lane(r, lead);
+    const uint32_t ut = (uint32_t)__builtin_amdgcn_readlane((int)t, lead);
+    const TileRange ur = tile_range(u);
+    for (int k = lane; k < ur.n; k += 64) {
+      const int tx = ur.tx0 + k % ur.tw, ty = ur.ty0 + k / ur.tw;
+      if (!g_tile_reached(u, tx, ty)) continue;
+      const uint32_t key = (uint32_t)(ty * tiles_x + tx);
+      list[tile_off[key] + atomicAdd(cursor + key, 1u)] = ut;
+    }
   }
 }
 
@@ -1129,6 +1201,7 @@ int vct_launch_gbuffer_phase(vct_context* ctx, int phase) {
   uint32_t* tile_count = (uint32_t*)ctx->g_count.p;
   uint32_t* cursor = tile_count + ntiles;
   uint32_t* tile_off = (uint32_t*)ctx->g_off.p;
+  const int lsh = vct_lanes_log2(p.ntri);
   if (phase & 1) {
     hipLaunchKernelGGL(fill_u32_kernel, dim3((2 * ntiles + 255) / 256), dim3(256), 0, ctx->stream, tile_count,
                        2 * ntiles, 0u);
@@ -1139,8 +1212,8 @@ int vct_launch_gbuffer_phase(vct_context* ctx, int phase) {
       if ((rc = vct_ensure(ctx->g_recs, (size_t)ntri * sizeof(GRec), ctx))) return rc;
       if ((rc = vct_ensure(ctx->g_clip, (size_t)ntri * 4, ctx))) return rc;
       hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, ctx->stream, counters + 5, 2u, 0u);
-      hipLaunchKernelGGL(g_bin_count_kernel, dim3((ntri + 255) / 256), dim3(256), 0, ctx->stream, p,
-                         (GRec*)ctx->g_recs.p, tile_count, tiles_x, (uint32_t*)ctx->g_clip.p, counters + 6);
+      hipLaunchKernelGGL(g_bin_count_kernel, dim3(vct_lane_blocks(p.ntri, lsh)), dim3(256), 0, ctx->stream, p,
+                         (GRec*)ctx->g_recs.p, tile_count, tiles_x, (uint32_t*)ctx->g_clip.p, counters + 6, lsh);
       hipLaunchKernelGGL(g_fan_count_kernel, dim3(kFanGrid), dim3(256), 0, ctx->stream, p, (GRec*)ctx->g_recs.p,
                          (const uint32_t*)ctx->g_clip.p, (const uint32_t*)(counters + 6), tile_count, tiles_x,
                          counters + 5);
@@ -1163,9 +1236,9 @@ int vct_launch_gbuffer_phase(vct_context* ctx, int phase) {
   GFan* fans = (GFan*)((char*)ctx->g_fans.p + (size_t)nfans * sizeof(GRec));
   if (total) {
     if ((rc = vct_ensure(ctx->g_list, (size_t)total * 4 + (size_t)total / 4 * 4, ctx))) return rc;
-    hipLaunchKernelGGL(g_bin_write_kernel, dim3((p.ntri + 255) / 256), dim3(256), 0, ctx->stream, p.ntri,
+    hipLaunchKernelGGL(g_bin_write_kernel, dim3(vct_lane_blocks(p.ntri, lsh)), dim3(256), 0, ctx->stream, p.ntri,
                        (const GRec*)ctx->g_recs.p, (const uint32_t*)tile_off, cursor, tiles_x,
-                       (uint32_t*)ctx->g_list.p);
+                       (uint32_t*)ctx->g_list.p, lsh);
     if (nfans)
       hipLaunchKernelGGL(g_fan_write_kernel, dim3(kFanGrid), dim3(256), 0, ctx->stream, p, (const GRec*)ctx->g_recs.p,
                          (const uint32_t*)ctx->g_clip.p, (const uint32_t*)(counters + 6), (const uint32_t*)tile_off,

@@ -345,6 +345,16 @@ inline int vct_pass_event(vct_context* ctx, int slot, bool end, hipStream_t s) {
   return VCT_OK;
 }
 
+// Lanes per triangle (log2) of the set-up and list kernels: few triangles are
+// spread until 2^18 lanes (4096 waves) run, so that each wave has few large
+// triangles to take one after another; from 2^18 triangles on, one lane each.
+inline int vct_lanes_log2(uint32_t ntri) {
+  int l = 0;
+  while (l < 6 && ((uint64_t)ntri << (l + 1)) <= (1ull << 18)) ++l;
+  return l;
+}
+inline uint32_t vct_lane_blocks(uint32_t ntri, int lsh) { return (uint32_t)((((uint64_t)ntri << lsh) + 255) / 256); }
+
 // kernels launchers
 int vct_launch_mip(vct_context* ctx);
 int vct_ensure_pairs(vct_context* ctx);  // x-paired copy of the volume for the marcher
