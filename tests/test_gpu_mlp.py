@@ -50,6 +50,41 @@ def test_forward_matches_oracle(gpu_available, orc, n):
     assert np.abs(y - want).mean() < 2e-3 * max(1.0, np.abs(want).mean())
 
 
+@pytest.mark.parametrize("n", [1, 15, 17, 32, 33, 129, 32769, 65793, 262144])
+def test_forward_row_groups_match_oracle(gpu_available, orc, n):
+    """Edges of the forward kernel's 16-row tiles, 32-row groups and grid
+    (256 workgroups of 128 rows, then two to four groups per wave), from BF16
+    rows and from float rows at an address that is only 4-byte aligned."""
+    from test_zz_no_alloc import DeviceBuffer
+
+    say(f"mlp forward rows n={n}")
+    rng = np.random.default_rng(n)
+    x = (rng.random((n, 34)) * 2 - 0.5).astype(np.float32)
+    p = _params(3)
+    with Context(16, 16) as ctx:
+        ctx.mlp_set_params(p)
+        ctx.sync()
+        y = ctx.mlp_forward(x)
+        dx, dy = DeviceBuffer(n * 136 + 4), DeviceBuffer(n * 12 + 16)
+        try:
+            dx.put(np.concatenate([np.zeros(1, np.float32), x.reshape(-1)]))
+            dy.put(np.full(n * 3 + 4, np.nan, np.float32))
+            L.check(ctx.lib.vct_mlp_forward_noalloc(ctx.h, dx.p.value + 4, n, dy.p.value + 4, None))
+            ctx.sync()
+            raw = dy.get(np.zeros(n * 3 + 4, np.float32))
+        finally:
+            dx.free()
+            dy.free()
+    assert np.array_equal(raw[1:-3].reshape(n, 3).view(np.uint32), y.view(np.uint32))
+    assert np.isnan(raw[[0, -3, -2, -1]]).all(), "wrote outside the n rows"
+    k = np.unique(np.concatenate([np.arange(min(n, 300)), np.arange(max(0, n - 300), n),
+                                  rng.integers(0, n, min(n, 4000))]))
+    want = orc.mlp_forward(p, x[k], bf16=True)
+    err = np.abs(y[k] - want)
+    say(f"  max-abs {err.max():.2e}, max |y| {np.abs(want).max():.2f}")
+    assert np.all(err <= 2e-2 + 2e-2 * np.abs(want))
+
+
 @pytest.mark.parametrize("n", [64, 1000, 8192])
 def test_gradient_matches_oracle(gpu_available, orc, n):
     say(f"mlp gradient n={n}")

@@ -400,7 +400,4 @@ int vct_trace_into(vct_context* ctx, const float4* gpos, const float4* gnrm, flo
 int vct_launch_scan_u32(vct_context* ctx, const uint32_t* in, uint32_t* out, uint32_t n,
                         uint32_t* total_dev, VctBuf* tmp = nullptr);
 int vct_tex3d_mip_launch(vct_context* ctx, VctTex3D& t);
-// Device address of the no-allocation entry point's staging array, taken once
-// per device (the current one) at context creation.
-int vct_noalloc_setup(int device);
 int vct_tex3d_clear_launch(vct_context* ctx, VctTex3D& t, const float rgba[4]);

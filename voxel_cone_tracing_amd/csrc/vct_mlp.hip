@@ -17,9 +17,9 @@
 //   27..29 normal, 30 relative linear depth (d - d_low) / d_low, 31..33 albedo
 // The network predicts the demodulated indirect light; the image is
 // albedo * prediction.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <mutex>
 
 #include "vct_internal.h"
 
@@ -154,47 +154,129 @@ __device__ int pixel_features(const FeatArgs& F, int px, int py, float* f, float
   return kFeatures;
 }
 
-// Row stride (BF16 elements) of the activations a wave keeps in LDS: 64
-// values padded to 72, so the 16 rows one MFMA operand load reads start 16
-// banks apart instead of all on the same bank (a 128-byte stride put the
-// inference kernel at 30 LDS bank conflicts per LDS instruction).
-constexpr int kXS = 72;
+// Row stride (BF16 elements) of the feature rows a wave stages in LDS: the 34
+// features padded with zeros to 40, a stride of 20 banks that spreads the 16
+// rows of an operand load over the banks.
+constexpr int kXS = 40;
 
-// ---- forward of one wave's 64 samples held in LDS ---------------------------------
-// xs: [64 samples][kXS] BF16 (features zero padded to 64).  Layers 1 and 2 are
-// computed per 16-sample column tile and written back over that tile's own
-// input rows, which no other tile reads (the tile's MFMAs have consumed them
-// before the write; one wave, in order).  Returns y (C layout of the 16-row
-// output tile) for the wave's four 16-sample column tiles.
-__device__ __forceinline__ void forward_wave(const MlpDev& P, uint16_t* xs, floatx4 (&y)[4]) {
+// ---- the network in registers ---------------------------------------------------
+// A C tile of one layer (rows: units, columns: samples) holds the very values
+// that the next layer's B operand needs, in other lanes of the same column:
+// lane group q = lane / 16 has units 16 mt + 4 q + i and needs units
+// 32 s + 8 q + j.  Two swaps per register move them (v_permlane32_swap,
+// v_permlane16_swap), so activations pass from layer to layer without LDS,
+// in the same k order as from memory.
+__device__ __forceinline__ bf16x8 ld_frag(const uint16_t* base, int ld) {
   const int lane = threadIdx.x & 63;
-  const int col = lane & 15, rq = (lane >> 4) * 4;
+  return *reinterpret_cast<const bf16x8*>(base + (lane & 15) * ld + (lane >> 4) * 8);
+}
+
+__device__ __forceinline__ floatx4 mfma32(bf16x8 a, bf16x8 b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint2 pack4(floatx4 v) {
+  return make_uint2(__builtin_bit_cast(uint32_t, bf16x2{(__bf16)v[0], (__bf16)v[1]}),
+                    __builtin_bit_cast(uint32_t, bf16x2{(__bf16)v[2], (__bf16)v[3]}));
+}
+
+// B operand of units 32 s .. 32 s + 31 from the packed C tiles mt = 2 s (lo)
+// and 2 s + 1 (hi).
+__device__ __forceinline__ bf16x8 next_frag(uint2 lo, uint2 hi) {
+  uint32_t w[4];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const auto a = __builtin_amdgcn_permlane32_swap(k ? lo.y : lo.x, k ? hi.y : hi.x, false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap(a[0], a[1], false, false);
+    w[k] = b[0];
+    w[2 + k] = b[1];
+  }
+  return __builtin_bit_cast(bf16x8, make_uint4(w[0], w[1], w[2], w[3]));
+}
+
+// The three layers' A operands and the lane's biases.
+struct NetRegs {
+  bf16x8 w1[4][2], w2[4][2], w3[2];
+  floatx4 b1[4], b2[4], b3;
+  __device__ __forceinline__ void load(const MlpDev& P) {
+    const int q = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        w1[mt][s] = ld_frag(P.packed + kPW1 + mt * 16 * 64 + 32 * s, 64);
+        w2[mt][s] = ld_frag(P.packed + kPW2 + mt * 16 * 64 + 32 * s, 64);
+      }
+      b1[mt] = *reinterpret_cast<const floatx4*>(P.b1 + mt * 16 + q * 4);
+      b2[mt] = *reinterpret_cast<const floatx4*>(P.b2 + mt * 16 + q * 4);
+    }
+    w3[0] = ld_frag(P.packed + kPW3, 64);
+    w3[1] = ld_frag(P.packed + kPW3 + 32, 64);
+    b3 = *reinterpret_cast<const floatx4*>(P.b3 + q * 4);  // zero past the outputs
+  }
+};
+
+// bias, ReLU and BF16 rounding of a C tile
+__device__ __forceinline__ uint2 relu_pack(floatx4 acc, floatx4 bias) {
+  floatx4 h;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) h[i] = fmaxf(acc[i] + bias[i], 0.0f);
+  return pack4(h);
+}
+
+// Output tile (rows 0..2 in lanes 0..15) of 16 samples from their features'
+// B operands (k 0..31 and 32..63).
+__device__ __forceinline__ floatx4 net_forward(const NetRegs& N, bf16x8 x0, bf16x8 x1) {
+  const floatx4 z = {0.f, 0.f, 0.f, 0.f};
+  uint2 p[4];
+#pragma unroll
+  for (int mt = 0; mt < 4; ++mt) p[mt] = relu_pack(mfma32(N.w1[mt][1], x1, mfma32(N.w1[mt][0], x0, z)), N.b1[mt]);
+  bf16x8 h0 = next_frag(p[0], p[1]), h1 = next_frag(p[2], p[3]);
+#pragma unroll
+  for (int mt = 0; mt < 4; ++mt) p[mt] = relu_pack(mfma32(N.w2[mt][1], h1, mfma32(N.w2[mt][0], h0, z)), N.b2[mt]);
+  h0 = next_frag(p[0], p[1]);
+  h1 = next_frag(p[2], p[3]);
+  return mfma32(N.w3[1], h1, mfma32(N.w3[0], h0, z)) + N.b3;
+}
+
+// The network over the 64 samples of a wave, their features in LDS rows xs
+// ([64][kXS] BF16): each weight operand is read once for
+// the four 16-sample tiles, and activations stay in registers.  Returns the
+// output tiles (rows 0..2 in lanes 0..15).
+__device__ __forceinline__ void forward_wave(const MlpDev& P, const uint16_t* xs, floatx4 (&y)[4]) {
+  const floatx4 z = {0.f, 0.f, 0.f, 0.f};
+  const int q = (threadIdx.x & 63) >> 4;
+  bf16x8 x[4][2];
+#pragma unroll
+  for (int nt = 0; nt < 4; ++nt) {
+    x[nt][0] = ld_frag(xs + nt * 16 * kXS, kXS);
+    uint4 c = make_uint4(0, 0, 0, 0);  // k = 32 + 8 q: features 32, 33 in q = 0, zeros past them
+    if (q == 0) c = *reinterpret_cast<const uint4*>(xs + (nt * 16 + (threadIdx.x & 15)) * kXS + 32);
+    x[nt][1] = __builtin_bit_cast(bf16x8, c);
+  }
+#pragma unroll
   for (int layer = 0; layer < 2; ++layer) {
     const uint16_t* Wp = P.packed + (layer == 0 ? kPW1 : kPW2);
     const float* bias = layer == 0 ? P.b1 : P.b2;
+    uint2 p[4][4];
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+      const bf16x8 w0 = ld_frag(Wp + mt * 16 * 64, 64), w1 = ld_frag(Wp + mt * 16 * 64 + 32, 64);
+      const floatx4 b = *reinterpret_cast<const floatx4*>(bias + mt * 16 + q * 4);
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt) p[nt][mt] = relu_pack(mfma32(w1, x[nt][1], mfma32(w0, x[nt][0], z)), b);
+    }
+#pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
-      floatx4 acc[4];
-      for (int mt = 0; mt < 4; ++mt) {
-        acc[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
-        acc[mt] = mfma_tile(Wp + mt * 16 * 64, 64, xs + nt * 16 * kXS, kXS, 64, acc[mt]);
-      }
-      for (int mt = 0; mt < 4; ++mt) {
-        uint16_t o[4];
-        for (int i = 0; i < 4; ++i) {
-          const float h = fmaxf(acc[mt][i] + bias[mt * 16 + rq + i], 0.0f);
-          o[i] = bf16_bits(h);
-        }
-        uint2 pk = make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
-        *reinterpret_cast<uint2*>(xs + (nt * 16 + col) * kXS + mt * 16 + rq) = pk;
-      }
+      x[nt][0] = next_frag(p[nt][0], p[nt][1]);
+      x[nt][1] = next_frag(p[nt][2], p[nt][3]);
     }
   }
-  for (int nt = 0; nt < 4; ++nt) {
-    floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
-    acc = mfma_tile(P.packed + kPW3, 64, xs + nt * 16 * kXS, kXS, 64, acc);
-    for (int i = 0; i < 4; ++i) acc[i] += (rq + i < kOut) ? P.b3[rq + i] : 0.0f;
-    y[nt] = acc;
-  }
+  const bf16x8 w0 = ld_frag(P.packed + kPW3, 64), w1 = ld_frag(P.packed + kPW3 + 32, 64);
+  const floatx4 b = *reinterpret_cast<const floatx4*>(P.b3 + q * 4);  // zero past the outputs
+#pragma unroll
+  for (int nt = 0; nt < 4; ++nt) y[nt] = mfma32(w1, x[nt][1], mfma32(w0, x[nt][0], z)) + b;
 }
 
 // ---- inference: features + MLP + output for a 16x16 pixel tile per workgroup ------
@@ -216,8 +298,11 @@ struct InferArgs {
 
 // Each lane keeps its pixel's data in registers over the network and writes
 // its own pixel, taking the three outputs of its sample from the lane that
-// holds them (36 KB of LDS per workgroup: 4 workgroups per CU).
-__global__ __launch_bounds__(256) void mlp_infer_kernel(InferArgs A) {
+// holds them; only the features pass through LDS (20 KB per workgroup), the
+// activations from layer to layer in registers, and 94 registers hold it at 5
+// waves per SIMD (upsampling pass of the 2560x1440 learned frame, its probes
+// included: 245 us with all activations in LDS at 4 workgroups per CU, 198).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void mlp_infer_kernel(InferArgs A) {
   __shared__ __attribute__((aligned(16))) uint16_t s_x[256 * kXS];
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
   if (!A.pix_list && A.skip_tile &&
@@ -248,8 +333,10 @@ __global__ __launch_bounds__(256) void mlp_infer_kernel(InferArgs A) {
   }
   uint16_t* row = s_x + t * kXS;
   const bool feat = st == kFeatures;
-  for (int k = 0; k < 64; k += 8) {
+#pragma unroll
+  for (int k = 0; k < kXS; k += 8) {
     uint32_t w[4];
+#pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int k0 = k + 2 * q, k1 = k0 + 1;
       const uint32_t lo = (feat && k0 < kIn) ? bf16_bits(f[k0]) : 0u;
@@ -314,28 +401,84 @@ __global__ __launch_bounds__(256) void mlp_sample_kernel(FeatArgs F, const float
   valid[k] = ok ? 1u : 0u;
 }
 
-// ---- forward on given features (tests and evaluation) -------------------------------
-__global__ __launch_bounds__(256) void mlp_forward_kernel(MlpDev P, const uint16_t* __restrict__ X, uint32_t n,
-                                                          float* __restrict__ Y) {
-  __shared__ __attribute__((aligned(16))) uint16_t s_x[256 * kXS];
-  const int t = threadIdx.x;
-  const uint32_t base = blockIdx.x * 256u;
-  {
-    const uint32_t k = base + t;
-    const uint4* src = reinterpret_cast<const uint4*>(X + (size_t)k * 64);
-    uint4* dst = reinterpret_cast<uint4*>(s_x + t * kXS);
-    for (int q = 0; q < 8; ++q) dst[q] = k < n ? src[q] : make_uint4(0, 0, 0, 0);
+// ---- forward on given features ------------------------------------------------------
+// Each wave keeps the weights in registers and takes 32 rows at a time, its B
+// operands straight from the rows: BF16 rows of 64 (T = uint16_t) or the
+// caller's rows of 34 floats, rounded here (T = float; any 4-byte aligned
+// address).  Reads and writes are the rows' own bytes (148 B per row, 6 us at
+// the copy rate for 200,003 rows): 12 us, where a staging pass to BF16 rows
+// and a pass over those through LDS took 37.
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float float2u __attribute__((ext_vector_type(2), aligned(4)));
+
+__device__ __forceinline__ void row_frags(const uint16_t* X, uint32_t row, bool in, bf16x8& x0, bf16x8& x1) {
+  const int q = (threadIdx.x & 63) >> 4;
+  uint4 a = make_uint4(0, 0, 0, 0), b = a;
+  if (in) {
+    const uint4* p = reinterpret_cast<const uint4*>(X + (size_t)row * 64) + q;
+    a = p[0];
+    b = p[4];
   }
-  __syncthreads();
-  const int wave = t >> 6, lane = t & 63;
-  floatx4 y[4];
-  forward_wave(P, s_x + wave * 64 * kXS, y);
-  if (lane < 16)
-    for (int nt = 0; nt < 4; ++nt) {
-      const uint32_t k = base + wave * 64 + nt * 16 + lane;
-      if (k < n)
-        for (int o = 0; o < kOut; ++o) Y[(size_t)k * 3 + o] = y[nt][o];
+  x0 = __builtin_bit_cast(bf16x8, a);
+  x1 = __builtin_bit_cast(bf16x8, b);
+}
+
+__device__ __forceinline__ void row_frags(const float* X, uint32_t row, bool in, bf16x8& x0, bf16x8& x1) {
+  const int q = (threadIdx.x & 63) >> 4;
+  float4u a = {0.f, 0.f, 0.f, 0.f}, b = a;
+  float2u c = {0.f, 0.f};
+  if (in) {
+    const float* p = X + (size_t)row * kIn;
+    a = *reinterpret_cast<const float4u*>(p + 8 * q);
+    b = *reinterpret_cast<const float4u*>(p + 8 * q + 4);
+    if (q == 0) c = *reinterpret_cast<const float2u*>(p + 32);
+  }
+  x0 = bf16x8{(__bf16)a[0], (__bf16)a[1], (__bf16)a[2], (__bf16)a[3],
+              (__bf16)b[0], (__bf16)b[1], (__bf16)b[2], (__bf16)b[3]};
+  const __bf16 z = (__bf16)0.0f;
+  x1 = bf16x8{(__bf16)c[0], (__bf16)c[1], z, z, z, z, z, z};
+}
+
+constexpr uint32_t kRowsPerWave = 32;     // rows a wave takes at a time
+// Workgroups of 4 waves: a wave's weights (18 KB) cost as much as several of
+// its row groups, so from 256 workgroups on (one per CU) each wave takes two
+// groups before there are more, up to two workgroups per CU (65,536 rows:
+// 6.1 us with 256 workgroups, 7.7 with 512; 262,144: 14.8 and 13.7, 1024 16.3).
+constexpr uint32_t kForwardMin = 256, kForwardMax = 512;
+
+template <typename T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void mlp_forward_kernel(
+    MlpDev P, const T* __restrict__ X, uint32_t n, float* __restrict__ Y) {
+  const int lane = threadIdx.x & 63, col = lane & 15;
+  const uint32_t first = (blockIdx.x * 4u + (threadIdx.x >> 6)) * kRowsPerWave, step = gridDim.x * 4u * kRowsPerWave;
+  if (first >= n) return;
+  NetRegs N;
+  bf16x8 x[2][2];
+  auto rows = [&](uint32_t base) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const uint32_t row = base + 16u * t + (uint32_t)col;
+      row_frags(X, row, row < n, x[t][0], x[t][1]);
     }
+  };
+  rows(first);
+  N.load(P);
+  for (uint32_t base = first; base < n; base += step) {  // n + step stays below 2^32 (checked at the launch)
+    floatx4 y[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) y[t] = net_forward(N, x[t][0], x[t][1]);
+    if (base + step < n) rows(base + step);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const uint32_t row = base + 16u * t + (uint32_t)lane;
+      if (lane < 16 && row < n) {
+        float* o = Y + (size_t)row * 3;
+        o[0] = y[t][0];
+        o[1] = y[t][1];
+        o[2] = y[t][2];
+      }
+    }
+  }
 }
 
 // ---- training: forward + backward over chunks of 64 samples ------------------------
@@ -966,6 +1109,18 @@ int need_mlp(vct_context* ctx) {
   return VCT_OK;
 }
 
+// The forward pass of n rows on a stream; allocates nothing.
+template <typename T>
+int launch_forward(vct_context* ctx, const T* X, uint32_t n, float* Y, hipStream_t stream) {
+  const uint32_t groups = (uint32_t)(((uint64_t)n + 4 * kRowsPerWave - 1) / (4 * kRowsPerWave));
+  const uint32_t blocks = std::min(groups, std::max(kForwardMin, std::min(kForwardMax, groups / 2)));
+  // the kernel's row counter passes n by less than one step of all waves
+  if (n > 0xffffffffu - kForwardMax * 4 * kRowsPerWave) return vct_set_error(VCT_ERR_LIMIT, "too many rows");
+  hipLaunchKernelGGL(mlp_forward_kernel<T>, dim3(blocks), dim3(256), 0, stream, mlp_dev(ctx), X, n, Y);
+  VCT_HIP(hipGetLastError());
+  return VCT_OK;
+}
+
 // Training step over X/A/Y rows [off, off + n) already on the device.
 int mlp_train_on(vct_context* ctx, const uint16_t* X, const float* Alb, const float* Y, uint32_t n, float lr,
                  float* loss_host, float* grad_host) {
@@ -1334,50 +1489,6 @@ int vct_launch_lowres_gather(vct_context* ctx) { return launch_lowres_gather(ctx
     VCT_HIP(hipSetDevice((ctx)->device));                                     \
   } while (0)
 
-// ---- the forward pass that allocates nothing ----------------------------------------
-// The BF16 feature rows of vct_mlp_forward_noalloc are staged in this fixed
-// array: each GPU the library runs on holds its own copy until the process
-// ends, at its own address.  Host code never passes the array's name to a
-// kernel (on the host it is only a stand-in symbol): the device address comes
-// from hipGetSymbolAddress, taken once per device when a context is created.
-static __device__ __align__(256) uint16_t scratch[(size_t)VCT_MLP_NOALLOC_MAX_ROWS * 64];
-
-namespace {
-constexpr int kScratchDevices = 64;
-std::mutex g_scratch_mu;
-uint16_t* g_scratch_ptr[kScratchDevices];  // device address of `scratch` per device (null: not set up)
-}  // namespace
-
-// Sets up the device address of the staging array of the current device.
-int vct_noalloc_setup(int device) {
-  if (device < 0 || device >= kScratchDevices) return vct_set_error(VCT_ERR_LIMIT, "device index above 63");
-  std::lock_guard<std::mutex> lock(g_scratch_mu);
-  if (g_scratch_ptr[device]) return VCT_OK;
-  void* ptr = nullptr;
-  const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-  if (e != hipSuccess) return vct_hip_check(e, "hipGetSymbolAddress(scratch)");
-  if (!ptr) return vct_set_error(VCT_ERR_HIP, "hipGetSymbolAddress(scratch) returned null");
-  g_scratch_ptr[device] = (uint16_t*)ptr;
-  return VCT_OK;
-}
-
-// Feature rows (n x 34 floats) -> BF16 rows of 64 (columns 34..63 zero), the
-// layout the forward kernel reads; one thread per (row, 8 columns).
-__global__ __launch_bounds__(256) void mlp_stage_kernel(const float* __restrict__ features, uint32_t n,
-                                                        uint16_t* __restrict__ X) {
-  const uint64_t g = (uint64_t)blockIdx.x * 256u + threadIdx.x;
-  if (g >= (uint64_t)n * 8u) return;
-  const uint32_t row = (uint32_t)(g >> 3), q = (uint32_t)(g & 7u);
-  uint32_t w[4];
-  for (int e = 0; e < 8; e += 2) {
-    const int c0 = (int)q * 8 + e, c1 = c0 + 1;
-    const uint32_t lo = c0 < kIn ? f32_to_bf16(features[(size_t)row * kIn + c0]) : 0u;
-    const uint32_t hi = c1 < kIn ? f32_to_bf16(features[(size_t)row * kIn + c1]) : 0u;
-    w[e >> 1] = lo | (hi << 16);
-  }
-  reinterpret_cast<uint4*>(X + (size_t)row * 64)[q] = make_uint4(w[0], w[1], w[2], w[3]);
-}
-
 extern "C" {
 
 int vct_mlp_init(vct_ctx ctx, uint64_t seed) {
@@ -1435,9 +1546,7 @@ int vct_mlp_forward(vct_ctx ctx, const float* features, uint32_t n, float* out) 
   if ((rc = need_mlp(ctx))) return rc;
   if ((rc = upload_features(ctx, features, n, ctx->train_X))) return rc;
   if ((rc = vct_ensure(ctx->train_Y, (size_t)n * 12, ctx))) return rc;
-  hipLaunchKernelGGL(mlp_forward_kernel, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, mlp_dev(ctx),
-                     (const uint16_t*)ctx->train_X.p, n, (float*)ctx->train_Y.p);
-  VCT_HIP(hipGetLastError());
+  if ((rc = launch_forward(ctx, (const uint16_t*)ctx->train_X.p, n, (float*)ctx->train_Y.p, ctx->stream))) return rc;
   VCT_HIP(hipMemcpyAsync(out, ctx->train_Y.p, (size_t)n * 12, hipMemcpyDeviceToHost, ctx->stream));
   VCT_HIP(hipStreamSynchronize(ctx->stream));
   ctx->train_n = 0;  // the training set buffers were reused
@@ -1451,15 +1560,7 @@ int vct_mlp_forward_noalloc(vct_ctx ctx, const float* features, uint32_t n, floa
     return vct_set_error(VCT_ERR_LIMIT, "vct_mlp_forward_noalloc takes at most VCT_MLP_NOALLOC_MAX_ROWS rows");
   int rc;
   if ((rc = need_mlp(ctx))) return rc;
-  uint16_t* X = ctx->device < kScratchDevices ? g_scratch_ptr[ctx->device] : nullptr;
-  if (!X) return vct_set_error(VCT_ERR_STATE, "staging array of the device not set up");
-  hipStream_t st = stream ? (hipStream_t)stream : ctx->stream;
-  hipLaunchKernelGGL(mlp_stage_kernel, dim3((unsigned)(((uint64_t)n * 8u + 255u) / 256u)), dim3(256), 0, st,
-                     features, n, X);
-  hipLaunchKernelGGL(mlp_forward_kernel, dim3((n + 255) / 256), dim3(256), 0, st, mlp_dev(ctx),
-                     (const uint16_t*)X, n, out);
-  VCT_HIP(hipGetLastError());
-  return VCT_OK;
+  return launch_forward(ctx, features, n, out, stream ? (hipStream_t)stream : ctx->stream);
 }
 
 int vct_mlp_loss_grad(vct_ctx ctx, const float* features, const float* albedo, const float* target, uint32_t n,
