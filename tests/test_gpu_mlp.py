@@ -109,6 +109,58 @@ def test_gradient_matches_oracle(gpu_available, orc, n):
         assert r < 5e-2, (lo, hi, r)
 
 
+@pytest.mark.parametrize("n", [65, 127, 129, 32768 + 33])
+def test_gradient_sample_groups_match_oracle(gpu_available, orc, n):
+    """Edges of the training kernel's 16-sample tiles, 32-sample waves, 128-
+    sample workgroups and its grid (32,801 samples: a second turn of one
+    wave), in gradient and loss; same bars as test_gradient_matches_oracle."""
+    say(f"mlp gradient groups n={n}")
+    rng = np.random.default_rng(n)
+    x = rng.random((n, 34)).astype(np.float32)
+    a = rng.random((n, 3)).astype(np.float32)
+    t = rng.random((n, 3)).astype(np.float32)
+    p = _params(4)
+    with Context(16, 16) as ctx:
+        ctx.mlp_set_params(p)
+        loss, g = ctx.mlp_loss_grad(x, a, t)
+    wl, wg = orc.mlp_loss_grad(p, x, a, t, bf16=True)
+    rel = np.linalg.norm(g - wg) / np.linalg.norm(wg)
+    say(f"  loss {loss:.6f} vs {wl:.6f}; gradient relative error {rel:.2e}")
+    assert abs(loss - wl) <= 1e-3 * wl
+    assert rel < 2e-2
+
+
+def test_train_step_walks_the_shuffled_rows(gpu_available):
+    """One Adam step from zero moments moves every parameter by lr times the
+    sign of its gradient (where |g| >> eps), so a step over a whole shuffled
+    set and one over the same rows in order agree with the set's gradient; a
+    step on the first minibatch of another seed does not use the same rows."""
+    say("training step over shuffled rows")
+    rng = np.random.default_rng(9)
+    n = 192
+    x = rng.random((n, 34)).astype(np.float32)
+    a = rng.random((n, 3)).astype(np.float32)
+    t = rng.random((n, 3)).astype(np.float32)
+    p = _params(5)
+    lr = 1e-3
+    with Context(16, 16) as ctx:
+        ctx.mlp_set_params(p)
+        loss, g = ctx.mlp_loss_grad(x, a, t)
+        got = []
+        for batch, seed in [(n, 1), (n, 2), (64, 1), (64, 2)]:
+            ctx.mlp_set_params(p)
+            ctx.upsample_set_samples(x, a, t)
+            l = ctx.upsample_train(1, batch, lr, seed)
+            got.append((l, ctx.mlp_params()))
+    for l, q in got[:2]:  # any order of the whole set: its loss and gradient
+        assert abs(l - loss) <= 1e-5 * loss
+        big = np.abs(g) > 1e-5
+        assert big.sum() > 3000
+        assert np.allclose((p - q)[big], lr * np.sign(g[big]), atol=lr * 1e-2)
+    assert not np.array_equal(got[2][1], got[3][1])
+    assert got[2][0] != got[3][0]
+
+
 def test_training_fits_a_smooth_target(gpu_available):
     rng = np.random.default_rng(7)
     n = 16384

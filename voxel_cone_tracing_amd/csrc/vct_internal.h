@@ -298,7 +298,7 @@ struct vct_context {
   int mlp_step = 0;
   VctBuf low_gpos, low_gnrm, low_img, full_target, sample_pix;
   VctBuf train_X, train_A, train_Y, train_valid;
-  VctBuf train_perm, batch_X, batch_A, batch_Y;  // minibatch order and the gathered minibatch
+  VctBuf train_perm;  // minibatch order
   size_t train_n = 0, train_cap = 0;
   // per-tile fallback of the learned frame
   VctBuf probe_pix, probe_val, fb_list;  // fb_list: [count][tiles...]

@@ -47,22 +47,6 @@ constexpr int kPW1 = 0, kPW2 = kPW1 + 64 * 64, kPW3 = kPW2 + 64 * 64, kPW2T = kP
 
 __device__ __forceinline__ uint16_t bf16_bits(float f) { return f32_to_bf16(f); }
 
-// One 16x16x32 MFMA step; a and b point at the lane's 8 contiguous BF16.
-__device__ __forceinline__ floatx4 mfma_step(const uint16_t* a, const uint16_t* b, floatx4 c) {
-  const bf16x8 va = *reinterpret_cast<const bf16x8*>(a);
-  const bf16x8 vb = *reinterpret_cast<const bf16x8*>(b);
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, vb, c, 0, 0, 0);
-}
-
-// C tile += A[m0:m0+16][0:K] * B[n0:n0+16][0:K]^T, K a multiple of 32.
-__device__ __forceinline__ floatx4 mfma_tile(const uint16_t* A, int lda, const uint16_t* B, int ldb, int K,
-                                             floatx4 c) {
-  const int lane = threadIdx.x & 63;
-  const int r = lane & 15, kq = (lane >> 4) * 8;
-  for (int k0 = 0; k0 < K; k0 += 32) c = mfma_step(A + r * lda + k0 + kq, B + r * ldb + k0 + kq, c);
-  return c;
-}
-
 struct MlpDev {
   const uint16_t* packed;  // kPacked BF16
   const float* b1;
@@ -453,255 +437,332 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
   const uint32_t first = (blockIdx.x * 4u + (threadIdx.x >> 6)) * kRowsPerWave, step = gridDim.x * 4u * kRowsPerWave;
   if (first >= n) return;
   NetRegs N;
-  bf16x8 x[2][2];
-  auto rows = [&](uint32_t base) {
+  N.load(P);
+  for (uint32_t base = first; base < n; base += step) {  // n + step stays below 2^32 (checked at the launch)
+    bf16x8 x[2][2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const uint32_t row = base + 16u * t + (uint32_t)col;
       row_frags(X, row, row < n, x[t][0], x[t][1]);
     }
-  };
-  rows(first);
-  N.load(P);
-  for (uint32_t base = first; base < n; base += step) {  // n + step stays below 2^32 (checked at the launch)
-    floatx4 y[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) y[t] = net_forward(N, x[t][0], x[t][1]);
-    if (base + step < n) rows(base + step);
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
+      const floatx4 y = net_forward(N, x[t][0], x[t][1]);
       const uint32_t row = base + 16u * t + (uint32_t)lane;
       if (lane < 16 && row < n) {
         float* o = Y + (size_t)row * 3;
-        o[0] = y[t][0];
-        o[1] = y[t][1];
-        o[2] = y[t][2];
+        o[0] = y[0];
+        o[1] = y[1];
+        o[2] = y[2];
       }
     }
   }
 }
 
-// ---- training: forward + backward over chunks of 64 samples ------------------------
-// Per chunk (P = 64 samples, 4 waves of 16): every activation and gradient is
-// staged in LDS as BF16 in the K-contiguous layout its next product reads.
-// Gradients accumulate in FP32 matrix-core accumulators across the chunks of
-// the workgroup; partial sums go to `partial` [gridDim.x][kParams] and are
-// reduced in a fixed order by mlp_adam_kernel (deterministic).
+// ---- training: forward + backward, a wave per 32 samples --------------------------
+// The A and B operands of v_mfma_f32_16x16x32_bf16 have one layout, so
+// exchanging them yields the transposed tile: every activation and gradient
+// is computed as units x samples (whose packed tiles chain into the next
+// product through next_frag) and again as samples x units, whose packed C
+// tiles are at once the operands of the weight gradients: lane (unit, q) holds
+// samples 4 q + i of both 16-sample tiles, a K order that all of them share.
+// Nothing passes through LDS until the four waves of the workgroup add their
+// gradients up.  Partial sums go to `partial` [gridDim.x][kParams + 1] and
+// are reduced in a fixed order by mlp_adam_kernel (deterministic).  A step of
+// 8,192 samples (64 workgroups here) is one chain of dependent reads and
+// products per wave: 13.8 us, where every operand staged through LDS behind
+// ten barriers took 19.6 and the minibatch gather before it 5 (the weights
+// staged in LDS at once measured 13.0, the rows read ahead of them 14.5 with
+// spills).
 struct TrainArgs {
   MlpDev P;
-  const uint16_t* X;  // [n][64]
-  const float* Alb;   // [n][3]
-  const float* Y;     // [n][3] target
+  const uint16_t* X;  // [rows][64]
+  const float* Alb;   // [rows][3]
+  const float* Y;     // [rows][3] target
+  // minibatch sample k is row perm[(first + k) mod nset], or row k without perm
+  const uint32_t* perm;
+  uint32_t first, nset;  // first < nset, n <= nset
   uint32_t n;
   float scale;        // 2 / (3 * n): d(mean squared error) / dy
   float* partial;     // [gridDim.x][kParams + 1] (last: loss sum)
 };
 
-constexpr int kP = 64;
+constexpr uint32_t kTrainRows = 128;   // samples of a workgroup at a time, 32 per wave
+constexpr uint32_t kTrainBlocks = 256;
 
-__global__ __launch_bounds__(256) void mlp_train_kernel(TrainArgs A) {
-  __shared__ __attribute__((aligned(16))) uint16_t xs[kP * 64];    // [sample][in]
-  __shared__ __attribute__((aligned(16))) uint16_t xt[64 * kP];    // [in][sample]
-  __shared__ __attribute__((aligned(16))) uint16_t h1s[kP * 64];   // [sample][hid]
-  __shared__ __attribute__((aligned(16))) uint16_t h1t[64 * kP];   // [hid][sample]
-  __shared__ __attribute__((aligned(16))) uint16_t h2s[kP * 64];
-  __shared__ __attribute__((aligned(16))) uint16_t h2t[64 * kP];
-  __shared__ __attribute__((aligned(16))) uint16_t dys[kP * 32];   // [sample][out (pad 32)]
-  __shared__ __attribute__((aligned(16))) uint16_t dyt[16 * kP];   // [out (pad 16)][sample]
-  __shared__ __attribute__((aligned(16))) uint16_t dz2s[kP * 64];  // [sample][hid]
-  __shared__ __attribute__((aligned(16))) uint16_t dz2t[64 * kP];  // [hid][sample]
-  __shared__ __attribute__((aligned(16))) uint16_t dz1t[64 * kP];  // [hid][sample]
-  __shared__ float s_db[4][2 * 64 + 16];
-  __shared__ float s_loss[4];
-
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-  const int col = lane & 15, rq = (lane >> 4) * 4;
-  const uint16_t* pk = A.P.packed;
-
-  // zero the padded output columns once (rows 3..31 of dY stay zero)
-  for (int i = t; i < kP * 32; i += 256) dys[i] = 0;
-  for (int i = t; i < 16 * kP; i += 256) dyt[i] = 0;
-
-  // gradient tiles owned by this wave: 4 (W3) + 16 (W2) + 12 (W1, in < 48) = 32
-  floatx4 g[8];
-  for (int q = 0; q < 8; ++q) g[q] = floatx4{0.f, 0.f, 0.f, 0.f};
-  float db1[16], db2[16], db3[3] = {0.f, 0.f, 0.f};
-  for (int q = 0; q < 16; ++q) db1[q] = db2[q] = 0.f;
-  float loss = 0.f;
-
-  const uint32_t nchunks = (A.n + kP - 1) / kP;
-  for (uint32_t ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
-    const uint32_t base = ch * kP;
-    __syncthreads();
-    // stage X in both layouts
-    for (int i = t; i < kP * 8; i += 256) {
-      const int s = i >> 3, q = i & 7;
-      const uint32_t k = base + s;
-      const uint4 v = k < A.n ? reinterpret_cast<const uint4*>(A.X + (size_t)k * 64)[q] : make_uint4(0, 0, 0, 0);
-      *reinterpret_cast<uint4*>(xs + s * 64 + q * 8) = v;
-      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-      for (int e = 0; e < 8; ++e) xt[(q * 8 + e) * kP + s] = (uint16_t)(w[e >> 1] >> ((e & 1) * 16));
-    }
-    __syncthreads();
-    // forward layers 1 and 2 on the wave's 16-sample column tile
-    floatx4 h1[4], h2[4];
-    for (int mt = 0; mt < 4; ++mt) {
-      floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
-      acc = mfma_tile(pk + kPW1 + mt * 16 * 64, 64, xs + wave * 16 * 64, 64, 64, acc);
-      for (int i = 0; i < 4; ++i) acc[i] = fmaxf(acc[i] + A.P.b1[mt * 16 + rq + i], 0.f);
-      h1[mt] = acc;
-      uint16_t o[4];
-      for (int i = 0; i < 4; ++i) o[i] = bf16_bits(acc[i]);
-      const int s = wave * 16 + col;
-      *reinterpret_cast<uint2*>(h1s + s * 64 + mt * 16 + rq) =
-          make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
-      for (int i = 0; i < 4; ++i) h1t[(mt * 16 + rq + i) * kP + s] = o[i];
-    }
-    __syncthreads();
-    for (int mt = 0; mt < 4; ++mt) {
-      floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
-      acc = mfma_tile(pk + kPW2 + mt * 16 * 64, 64, h1s + wave * 16 * 64, 64, 64, acc);
-      for (int i = 0; i < 4; ++i) acc[i] = fmaxf(acc[i] + A.P.b2[mt * 16 + rq + i], 0.f);
-      h2[mt] = acc;
-      uint16_t o[4];
-      for (int i = 0; i < 4; ++i) o[i] = bf16_bits(acc[i]);
-      const int s = wave * 16 + col;
-      *reinterpret_cast<uint2*>(h2s + s * 64 + mt * 16 + rq) =
-          make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
-      for (int i = 0; i < 4; ++i) h2t[(mt * 16 + rq + i) * kP + s] = o[i];
-    }
-    __syncthreads();
-    // layer 3 and the output gradient
-    {
-      floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
-      acc = mfma_tile(pk + kPW3, 64, h2s + wave * 16 * 64, 64, 64, acc);
-      const int s = wave * 16 + col;
-      const uint32_t k = base + s;
-      if (lane < 16) {  // rows 0..3 of the output tile: outputs 0..2
-        for (int o = 0; o < kOut; ++o) {
-          float d = 0.f;
-          if (k < A.n) {
-            const float yv = acc[o] + A.P.b3[o];
-            const float a = A.Alb[(size_t)k * 3 + o];
-            const float e = a * (yv - A.Y[(size_t)k * 3 + o]);
-            loss += e * e;
-            d = A.scale * a * e;  // d(loss)/dy
-          }
-          db3[o] += d;
-          const uint16_t b = bf16_bits(d);
-          dys[s * 32 + o] = b;
-          dyt[o * kP + s] = b;
-        }
-      }
-    }
-    __syncthreads();
-    // dH2 = W3^T dY -> dZ2 = dH2 * [h2 > 0]
-    for (int mt = 0; mt < 4; ++mt) {
-      floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
-      acc = mfma_tile(pk + kPW3T + mt * 16 * 32, 32, dys + wave * 16 * 32, 32, 32, acc);
-      uint16_t o[4];
-      for (int i = 0; i < 4; ++i) {
-        const float dz = h2[mt][i] > 0.f ? acc[i] : 0.f;
-        db2[mt * 4 + i] += dz;
-        o[i] = bf16_bits(dz);
-      }
-      const int s = wave * 16 + col;
-      *reinterpret_cast<uint2*>(dz2s + s * 64 + mt * 16 + rq) =
-          make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
-      for (int i = 0; i < 4; ++i) dz2t[(mt * 16 + rq + i) * kP + s] = o[i];
-    }
-    __syncthreads();
-    // dH1 = W2^T dZ2 -> dZ1 = dH1 * [h1 > 0]
-    for (int mt = 0; mt < 4; ++mt) {
-      floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
-      acc = mfma_tile(pk + kPW2T + mt * 16 * 64, 64, dz2s + wave * 16 * 64, 64, 64, acc);
-      const int s = wave * 16 + col;
-      for (int i = 0; i < 4; ++i) {
-        const float dz = h1[mt][i] > 0.f ? acc[i] : 0.f;
-        db1[mt * 4 + i] += dz;
-        dz1t[(mt * 16 + rq + i) * kP + s] = bf16_bits(dz);
-      }
-    }
-    __syncthreads();
-    // weight gradients over the chunk's 64 samples (K = samples)
-    for (int q = 0; q < 8; ++q) {
-      const int tile = wave * 8 + q;  // 0..31
-      if (tile < 4) {                 // dW3 [16 x 64]: n tile = tile
-        g[q] = mfma_tile(dyt, kP, h2t + tile * 16 * kP, kP, kP, g[q]);
-      } else if (tile < 20) {         // dW2 [64 x 64]
-        const int tt = tile - 4, mt = tt >> 2, nt = tt & 3;
-        g[q] = mfma_tile(dz2t + mt * 16 * kP, kP, h1t + nt * 16 * kP, kP, kP, g[q]);
-      } else {                        // dW1 [64 x 48]
-        const int tt = tile - 20, mt = tt / 3, nt = tt % 3;
-        g[q] = mfma_tile(dz1t + mt * 16 * kP, kP, xt + nt * 16 * kP, kP, kP, g[q]);
-      }
-    }
-  }
-  // ---- write this workgroup's partial gradients --------------------------------------
-  float* out = A.partial + (size_t)blockIdx.x * (kParams + 1);
-  for (int q = 0; q < 8; ++q) {
-    const int tile = wave * 8 + q;
-    for (int i = 0; i < 4; ++i) {
-      const int m = rq + i;
-      if (tile < 4) {
-        if (m < kOut) out[kOffW3 + m * 64 + tile * 16 + col] = g[q][i];
-      } else if (tile < 20) {
-        const int tt = tile - 4, mt = tt >> 2, nt = tt & 3;
-        out[kOffW2 + (mt * 16 + m) * 64 + nt * 16 + col] = g[q][i];
-      } else {
-        const int tt = tile - 20, mt = tt / 3, nt = tt % 3;
-        const int in = nt * 16 + col;
-        if (in < kIn) out[kOffW1 + (mt * 16 + m) * kIn + in] = g[q][i];
-      }
-    }
-  }
-  // bias gradients: sum the 16 sample lanes of each row group, then the waves
-  for (int q = 0; q < 16; ++q) {
-    float a = db1[q], b = db2[q];
-    for (int o = 1; o < 16; o <<= 1) {
-      a += __shfl_xor(a, o, 64);
-      b += __shfl_xor(b, o, 64);
-    }
-    db1[q] = a;
-    db2[q] = b;
-  }
-  if (col == 0) {
-    for (int mt = 0; mt < 4; ++mt)
-      for (int i = 0; i < 4; ++i) {
-        s_db[wave][mt * 16 + rq + i] = db1[mt * 4 + i];
-        s_db[wave][64 + mt * 16 + rq + i] = db2[mt * 4 + i];
-      }
-  }
-  {
-    float l = loss;
-    for (int o = 1; o < 64; o <<= 1) l += __shfl_xor(l, o, 64);
-    if (lane == 0) s_loss[wave] = l;
-  }
-  for (int o = 0; o < kOut; ++o) {
-    float a = lane < 16 ? db3[o] : 0.f;
-    for (int q = 1; q < 16; q <<= 1) a += __shfl_xor(a, q, 64);
-    if (lane == 0) s_db[wave][128 + o] = a;
-  }
-  __syncthreads();
-  if (t < 64) {
-    out[kOffB1 + t] = ((s_db[0][t] + s_db[1][t]) + s_db[2][t]) + s_db[3][t];
-    out[kOffB2 + t] = ((s_db[0][64 + t] + s_db[1][64 + t]) + s_db[2][64 + t]) + s_db[3][64 + t];
-  }
-  if (t < kOut) out[kOffB3 + t] = ((s_db[0][128 + t] + s_db[1][128 + t]) + s_db[2][128 + t]) + s_db[3][128 + t];
-  if (t == 0) out[kParams] = ((s_loss[0] + s_loss[1]) + s_loss[2]) + s_loss[3];
+__device__ __forceinline__ bf16x8 join(uint2 a, uint2 b) {
+  return __builtin_bit_cast(bf16x8, make_uint4(a.x, a.y, b.x, b.y));
 }
 
-// Fixed-order reduction of the partials + Adam (FP32 master weights).
-// With lr == 0 it only reduces (gradient and loss read-back).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void mlp_train_kernel(TrainArgs A) {
+  __shared__ float s_g[4][kParams + 1];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, q = lane >> 4;
+  const uint16_t* pk = A.P.packed;
+  const floatx4 z = {0.f, 0.f, 0.f, 0.f};
+  floatx4 g1[4][3], g2[4][4], g3[4];  // dW1 (48 inputs), dW2, dW3 tiles
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    g3[i] = z;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) g2[i][j] = z;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) g1[i][j] = z;
+  }
+  float db1[4] = {0.f, 0.f, 0.f, 0.f}, db2[4] = {0.f, 0.f, 0.f, 0.f}, db3 = 0.f, loss = 0.f;
+  // identity operands: column c of the transposed features is input 16 nt + c
+  bf16x8 eye[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) eye[h][j] = (__bf16)(8 * q + j == 16 * h + col ? 1.0f : 0.0f);
+
+  for (uint32_t base = (blockIdx.x * 4u + (uint32_t)wave) * 32u; base < A.n; base += gridDim.x * kTrainRows) {
+    uint32_t row[2];
+    bf16x8 x[2][2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const uint32_t k = base + 16u * t + (uint32_t)col;
+      row[t] = k;
+      if (A.perm && k < A.n) {
+        const uint64_t r = (uint64_t)A.first + k;
+        row[t] = A.perm[r >= A.nset ? r - A.nset : r];
+      }
+      row_frags(A.X, row[t], k < A.n, x[t][0], x[t][1]);
+    }
+    // albedo and target of the samples x outputs tile: output col, samples 4 q + i
+    float al[2][4], tg[2][4];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t r = (uint32_t)__shfl((int)row[t], 4 * q + i, 64);
+        const bool in = col < kOut && base + 16u * t + 4u * q + i < A.n;
+        al[t][i] = in ? A.Alb[(size_t)r * 3 + col] : 0.f;
+        tg[t][i] = in ? A.Y[(size_t)r * 3 + col] : 0.f;
+      }
+    // forward; masks of the positive activations, bit 4 mt + i
+    uint2 xT[2][3], h1T[2][4], h2T[2][4];
+    bf16x8 hf[2][2];
+    uint32_t m1T[2] = {0u, 0u}, m2[2] = {0u, 0u}, m2T[2] = {0u, 0u};
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+      for (int nt = 0; nt < 3; ++nt) xT[t][nt] = pack4(mfma32(x[t][nt >> 1], eye[nt & 1], z));
+      uint2 p[4];
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt) {
+        const bf16x8 w0 = ld_frag(pk + kPW1 + mt * 16 * 64, 64), w1 = ld_frag(pk + kPW1 + mt * 16 * 64 + 32, 64);
+        p[mt] = relu_pack(mfma32(w1, x[t][1], mfma32(w0, x[t][0], z)),
+                          *reinterpret_cast<const floatx4*>(A.P.b1 + mt * 16 + q * 4));
+        floatx4 h = mfma32(x[t][1], w1, mfma32(x[t][0], w0, z));
+        const float b = A.P.b1[mt * 16 + col];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          h[i] = fmaxf(h[i] + b, 0.f);
+          m1T[t] |= (h[i] > 0.f ? 1u : 0u) << (4 * mt + i);
+        }
+        h1T[t][mt] = pack4(h);
+      }
+      hf[t][0] = next_frag(p[0], p[1]);
+      hf[t][1] = next_frag(p[2], p[3]);
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      uint2 p[4];
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt) {
+        const bf16x8 w0 = ld_frag(pk + kPW2 + mt * 16 * 64, 64), w1 = ld_frag(pk + kPW2 + mt * 16 * 64 + 32, 64);
+        floatx4 h = mfma32(w1, hf[t][1], mfma32(w0, hf[t][0], z));
+        const floatx4 b4 = *reinterpret_cast<const floatx4*>(A.P.b2 + mt * 16 + q * 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          h[i] = fmaxf(h[i] + b4[i], 0.f);
+          m2[t] |= (h[i] > 0.f ? 1u : 0u) << (4 * mt + i);
+        }
+        p[mt] = pack4(h);
+        h = mfma32(hf[t][1], w1, mfma32(hf[t][0], w0, z));
+        const float b = A.P.b2[mt * 16 + col];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          h[i] = fmaxf(h[i] + b, 0.f);
+          m2T[t] |= (h[i] > 0.f ? 1u : 0u) << (4 * mt + i);
+        }
+        h2T[t][mt] = pack4(h);
+      }
+      hf[t][0] = next_frag(p[0], p[1]);
+      hf[t][1] = next_frag(p[2], p[3]);
+    }
+    // outputs (samples x outputs) and their gradient; lanes past the outputs hold zeros
+    uint2 dyT[2];
+    bf16x8 dy[2];
+    {
+      const bf16x8 w0 = ld_frag(pk + kPW3, 64), w1 = ld_frag(pk + kPW3 + 32, 64);
+      const float b = A.P.b3[col];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const floatx4 y = mfma32(hf[t][1], w1, mfma32(hf[t][0], w0, z));
+        floatx4 d;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float e = al[t][i] * ((y[i] + b) - tg[t][i]);
+          loss += e * e;
+          d[i] = A.scale * al[t][i] * e;  // d(loss)/dy
+          db3 += d[i];
+        }
+        dyT[t] = pack4(d);
+        // the same values as a B operand (outputs in k, sample col): sample
+        // col = 4 q' + i is element i of lane (output, q')
+        uint32_t o[kOut];
+#pragma unroll
+        for (int k = 0; k < kOut; ++k) {
+          const int src = (col >> 2) * 16 + k;
+          const uint32_t lo = (uint32_t)__shfl((int)dyT[t].x, src, 64), hi = (uint32_t)__shfl((int)dyT[t].y, src, 64);
+          const uint32_t w = (col & 2) ? hi : lo;
+          o[k] = (col & 1) ? w >> 16 : w & 0xffffu;
+        }
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (q == 0) v = make_uint4(o[0] | (o[1] << 16), o[2], 0, 0);
+        dy[t] = __builtin_bit_cast(bf16x8, v);
+      }
+    }
+    // dZ2 = (W3^T dY) [h2 > 0], in both orientations
+    uint2 z2T[2][4], z1T[2][4];
+    bf16x8 zf[2][2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      uint2 p[4];
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt) {
+        const bf16x8 w = ld_frag(pk + kPW3T + mt * 16 * 32, 32);
+        floatx4 d = mfma32(w, dy[t], z), dT = mfma32(dy[t], w, z);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          d[i] = (m2[t] >> (4 * mt + i)) & 1u ? d[i] : 0.f;
+          dT[i] = (m2T[t] >> (4 * mt + i)) & 1u ? dT[i] : 0.f;
+        }
+        p[mt] = pack4(d);
+        z2T[t][mt] = pack4(dT);
+        db2[mt] += (dT[0] + dT[1]) + (dT[2] + dT[3]);
+      }
+      zf[t][0] = next_frag(p[0], p[1]);
+      zf[t][1] = next_frag(p[2], p[3]);
+    }
+    // dZ1 = (W2^T dZ2) [h1 > 0], samples x units
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt) {
+        const bf16x8 w0 = ld_frag(pk + kPW2T + mt * 16 * 64, 64), w1 = ld_frag(pk + kPW2T + mt * 16 * 64 + 32, 64);
+        floatx4 d = mfma32(zf[t][1], w1, mfma32(zf[t][0], w0, z));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d[i] = (m1T[t] >> (4 * mt + i)) & 1u ? d[i] : 0.f;
+        z1T[t][mt] = pack4(d);
+        db1[mt] += (d[0] + d[1]) + (d[2] + d[3]);
+      }
+    // weight gradients over the wave's 32 samples
+    const bf16x8 fy = join(dyT[0], dyT[1]);
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+      g3[mt] = mfma32(fy, join(h2T[0][mt], h2T[1][mt]), g3[mt]);
+      const bf16x8 a2 = join(z2T[0][mt], z2T[1][mt]), a1 = join(z1T[0][mt], z1T[1][mt]);
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt) g2[mt][nt] = mfma32(a2, join(h1T[0][nt], h1T[1][nt]), g2[mt][nt]);
+#pragma unroll
+      for (int nt = 0; nt < 3; ++nt) g1[mt][nt] = mfma32(a1, join(xT[0][nt], xT[1][nt]), g1[mt][nt]);
+    }
+  }
+  // ---- the workgroup's gradients: each wave's, added in wave order ------------------
+  float* o = s_g[wave];
+#pragma unroll
+  for (int mt = 0; mt < 4; ++mt) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = 4 * q + i;
+      if (m < kOut) o[kOffW3 + m * 64 + mt * 16 + col] = g3[mt][i];
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt) o[kOffW2 + (mt * 16 + m) * 64 + nt * 16 + col] = g2[mt][nt][i];
+#pragma unroll
+      for (int nt = 0; nt < 3; ++nt)
+        if (nt * 16 + col < kIn) o[kOffW1 + (mt * 16 + m) * kIn + nt * 16 + col] = g1[mt][nt][i];
+    }
+    // bias gradients: the four sample groups of a unit's lanes
+    float b1 = db1[mt], b2 = db2[mt];
+    b1 += __shfl_xor(b1, 16, 64);
+    b2 += __shfl_xor(b2, 16, 64);
+    b1 += __shfl_xor(b1, 32, 64);
+    b2 += __shfl_xor(b2, 32, 64);
+    if (q == 0) {
+      o[kOffB1 + mt * 16 + col] = b1;
+      o[kOffB2 + mt * 16 + col] = b2;
+    }
+  }
+  db3 += __shfl_xor(db3, 16, 64);
+  db3 += __shfl_xor(db3, 32, 64);
+  if (lane < kOut) o[kOffB3 + lane] = db3;
+#pragma unroll
+  for (int k = 1; k < 64; k <<= 1) loss += __shfl_xor(loss, k, 64);
+  if (lane == 0) o[kParams] = loss;
+  __syncthreads();
+  float* out = A.partial + (size_t)blockIdx.x * (kParams + 1);
+  for (int k = threadIdx.x; k <= kParams; k += 256) out[k] = ((s_g[0][k] + s_g[1][k]) + s_g[2][k]) + s_g[3][k];
+}
+
+// Writes one master parameter's BF16 operand copies (or its FP32 bias).
+__device__ __forceinline__ void pack_param(int p, float v, uint16_t* __restrict__ pk, float* __restrict__ bias) {
+  const uint16_t b = bf16_bits(v);
+  if (p < kOffB1) {
+    pk[kPW1 + (p / kIn) * 64 + p % kIn] = b;
+  } else if (p < kOffW2) {
+    bias[p - kOffB1] = v;
+  } else if (p < kOffB2) {
+    const int i = p - kOffW2;
+    pk[kPW2 + i] = b;
+    pk[kPW2T + (i & 63) * 64 + (i >> 6)] = b;
+  } else if (p < kOffW3) {
+    bias[64 + p - kOffB2] = v;
+  } else if (p < kOffB3) {
+    const int i = p - kOffW3;
+    pk[kPW3 + i] = b;
+    pk[kPW3T + (i & 63) * 32 + (i >> 6)] = b;
+  } else {
+    bias[128 + p - kOffB3] = v;
+  }
+}
+
+// Fixed-order reduction of the partials + Adam (FP32 master weights) + the
+// operand copies of the updated weights (their zero padding was written by
+// mlp_pack_kernel).  With lr == 0 it only reduces (gradient and loss
+// read-back).  A workgroup takes 64 parameters, each wave a quarter of the
+// partials with 16 loads in flight: 4.3 us for 64 partials, where one lane per
+// parameter reading 128 one after another took 31, and the operand copies as
+// a kernel of their own 5 more.
 __global__ __launch_bounds__(256) void mlp_adam_kernel(float* __restrict__ params, float* __restrict__ m1,
                                                        float* __restrict__ m2, const float* __restrict__ partial,
                                                        int nblk, float lr, float beta1, float beta2, float eps,
                                                        float bc1, float bc2, float* __restrict__ grad_out,
-                                                       float* __restrict__ loss_out) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p > kParams) return;
+                                                       float* __restrict__ loss_out, uint16_t* __restrict__ pk,
+                                                       float* __restrict__ bias) {
+  __shared__ float s_sum[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int p = blockIdx.x * 64 + lane;
+  const int per = (nblk + 3) / 4, lo = min(wave * per, nblk), hi = min(lo + per, nblk);
   float g = 0.f;
-  for (int b = 0; b < nblk; ++b) g += partial[(size_t)b * (kParams + 1) + p];
+  if (p <= kParams) {
+    const float* src = partial + p;
+    int b = lo;
+    for (; b + 16 <= hi; b += 16) {
+      float v[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) v[k] = src[(size_t)(b + k) * (kParams + 1)];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) g += v[k];
+    }
+    for (; b < hi; ++b) g += src[(size_t)b * (kParams + 1)];
+  }
+  s_sum[wave][lane] = g;
+  __syncthreads();
+  if (wave != 0 || p > kParams) return;
+  g = ((s_sum[0][lane] + s_sum[1][lane]) + s_sum[2][lane]) + s_sum[3][lane];
   if (p == kParams) {
     if (loss_out) *loss_out = g;
     return;
@@ -712,7 +773,9 @@ __global__ __launch_bounds__(256) void mlp_adam_kernel(float* __restrict__ param
     const float b = beta2 * m2[p] + (1.f - beta2) * g * g;
     m1[p] = a;
     m2[p] = b;
-    params[p] -= lr * (a / bc1) / (sqrtf(b / bc2) + eps);
+    const float v = params[p] - lr * (a / bc1) / (sqrtf(b / bc2) + eps);
+    params[p] = v;
+    pack_param(p, v, pk, bias);
   }
 }
 
@@ -1121,18 +1184,24 @@ int launch_forward(vct_context* ctx, const T* X, uint32_t n, float* Y, hipStream
   return VCT_OK;
 }
 
-// Training step over X/A/Y rows [off, off + n) already on the device.
+// Training step over n rows already on the device: rows 0 .. n - 1, or the
+// minibatch of ctx->train_perm (an order of nset rows) that starts at `first`.
 int mlp_train_on(vct_context* ctx, const uint16_t* X, const float* Alb, const float* Y, uint32_t n, float lr,
-                 float* loss_host, float* grad_host) {
-  const uint32_t nchunks = (n + kP - 1) / kP;
-  const int G = (int)std::min<uint32_t>(nchunks, 1024u);
+                 float* loss_host, float* grad_host, const uint32_t* perm = nullptr, uint32_t first = 0,
+                 uint32_t nset = 0) {
+  const int G = (int)std::min<uint32_t>((uint32_t)(((uint64_t)n + kTrainRows - 1) / kTrainRows), kTrainBlocks);
   int rc;
   if ((rc = vct_ensure(ctx->mlp_partial, (size_t)G * (kParams + 1) * 4, ctx))) return rc;
+  // the kernel's sample counter passes n by less than one step of the grid
+  if (n > 0xffffffffu - kTrainBlocks * kTrainRows) return vct_set_error(VCT_ERR_LIMIT, "too many samples");
   TrainArgs A;
   A.P = mlp_dev(ctx);
   A.X = X;
   A.Alb = Alb;
   A.Y = Y;
+  A.perm = perm;
+  A.first = first;
+  A.nset = nset;
   A.n = n;
   A.scale = 2.0f / (3.0f * (float)n);
   A.partial = (float*)ctx->mlp_partial.p;
@@ -1145,13 +1214,11 @@ int mlp_train_on(vct_context* ctx, const uint16_t* X, const float* Alb, const fl
     bc2 = 1.0f - powf(0.999f, (float)ctx->mlp_step);
   }
   float* gout = (float*)ctx->mlp_grad.p;
-  hipLaunchKernelGGL(mlp_adam_kernel, dim3((kParams + 1 + 255) / 256), dim3(256), 0, ctx->stream,
+  hipLaunchKernelGGL(mlp_adam_kernel, dim3((kParams + 1 + 63) / 64), dim3(256), 0, ctx->stream,
                      (float*)ctx->mlp_params.p, (float*)ctx->mlp_m1.p, (float*)ctx->mlp_m2.p,
-                     (const float*)ctx->mlp_partial.p, G, lr, 0.9f, 0.999f, 1e-8f, bc1, bc2, gout, gout + kParams);
+                     (const float*)ctx->mlp_partial.p, G, lr, 0.9f, 0.999f, 1e-8f, bc1, bc2, gout, gout + kParams,
+                     (uint16_t*)ctx->mlp_packed.p, (float*)ctx->mlp_bias.p);
   VCT_HIP(hipGetLastError());
-  if (lr > 0.f) {
-    if ((rc = mlp_pack(ctx))) return rc;
-  }
   if (loss_host || grad_host) {
     std::vector<float> g(kParams + 1);
     VCT_HIP(hipMemcpyAsync(g.data(), gout, (kParams + 1) * 4, hipMemcpyDeviceToHost, ctx->stream));
@@ -1442,29 +1509,6 @@ int refine(vct_context* ctx, bool selected) {
   return VCT_OK;
 }
 
-// Minibatch k of a training run: rows perm[(k*batch + i) mod n] of the
-// sample set, gathered into contiguous batch buffers.  Eight threads per row
-// move its 128-byte BF16 feature row as 16-byte pieces; the first of them
-// also moves albedo and target.
-__global__ __launch_bounds__(256) void mlp_batch_gather_kernel(const uint32_t* __restrict__ perm, uint32_t n,
-                                                               uint64_t first, uint32_t batch,
-                                                               const uint16_t* __restrict__ X,
-                                                               const float* __restrict__ A,
-                                                               const float* __restrict__ Y, uint16_t* __restrict__ bx,
-                                                               float* __restrict__ ba, float* __restrict__ by) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t i = t >> 3, c = t & 7;
-  if (i >= batch) return;
-  const uint32_t r = perm[(first + i) % n];
-  reinterpret_cast<uint4*>(bx + (size_t)i * 64)[c] = reinterpret_cast<const uint4*>(X + (size_t)r * 64)[c];
-  if (c == 0) {
-    for (int q = 0; q < 3; ++q) {
-      ba[(size_t)i * 3 + q] = A[(size_t)r * 3 + q];
-      by[(size_t)i * 3 + q] = Y[(size_t)r * 3 + q];
-    }
-  }
-}
-
 // A uniformly random order of the n training rows (Fisher-Yates, the
 // library's splitmix64 stream of `seed`), on the device in ctx->train_perm.
 int shuffle_rows(vct_context* ctx, uint32_t n, uint64_t seed) {
@@ -1676,18 +1720,11 @@ int vct_upsample_train(vct_ctx ctx, uint32_t steps, uint32_t batch, float lr, ui
   // Minibatches walk one random order of the whole sample set (samples are
   // stored frame by frame, so a contiguous window would hold one camera pose).
   if ((rc = shuffle_rows(ctx, n, seed))) return rc;
-  if ((rc = vct_ensure(ctx->batch_X, (size_t)batch * 128, ctx))) return rc;
-  if ((rc = vct_ensure(ctx->batch_A, (size_t)batch * 12, ctx))) return rc;
-  if ((rc = vct_ensure(ctx->batch_Y, (size_t)batch * 12, ctx))) return rc;
   for (uint32_t s = 0; s < steps; ++s) {
-    hipLaunchKernelGGL(mlp_batch_gather_kernel, dim3((batch * 8 + 255) / 256), dim3(256), 0, ctx->stream,
-                       (const uint32_t*)ctx->train_perm.p, n, (uint64_t)s * batch, batch,
-                       (const uint16_t*)ctx->train_X.p, (const float*)ctx->train_A.p, (const float*)ctx->train_Y.p,
-                       (uint16_t*)ctx->batch_X.p, (float*)ctx->batch_A.p, (float*)ctx->batch_Y.p);
-    VCT_HIP(hipGetLastError());
     const bool last = s + 1 == steps;
-    if ((rc = mlp_train_on(ctx, (const uint16_t*)ctx->batch_X.p, (const float*)ctx->batch_A.p,
-                           (const float*)ctx->batch_Y.p, batch, lr, last ? last_loss : nullptr, nullptr)))
+    if ((rc = mlp_train_on(ctx, (const uint16_t*)ctx->train_X.p, (const float*)ctx->train_A.p,
+                           (const float*)ctx->train_Y.p, batch, lr, last ? last_loss : nullptr, nullptr,
+                           (const uint32_t*)ctx->train_perm.p, (uint32_t)(((uint64_t)s * batch) % n), n)))
       return rc;
   }
   return VCT_OK;
