@@ -364,6 +364,36 @@ def test_large_triangles_bit_exact(gpu_available, orc, n, res, W, H):
     assert np.array_equal(bits(gn), bits(n32))
 
 
+@pytest.mark.parametrize("res,n,size", [(4, 3, 1.0), (8, 1, 2.0), (8, 64, 1.0), (8, 129, 0.02), (8, 1024, 0.3),
+                                        (8, 1025, 0.3), (16, 9000, 0.1), (64, 3000, 1.0)])
+def test_reference_average_rounds_bit_exact(gpu_available, orc, res, n, size):
+    """The reference average takes a brick's triangles sorted by original
+    index (in LDS up to 1024 of them, by radix passes past that) in rounds of
+    up to 128 whose fragments fit in LDS, halving a round that does not.
+    Grids of one brick or few (8^3 voxels) with 1 to 9000 triangles each,
+    from tiny ones (whole rounds) to ones that fill the brick's footprint
+    (three a round), the triangles' order shuffled by the upload's own sort."""
+    say(f"reference average rounds res={res} n={n} size={size}")
+    rng = np.random.default_rng(n + res)
+    p = rng.uniform(-1.0, 1.0, (n, 1, 3)) + size * rng.standard_normal((n, 3, 3))
+    nrm = np.cross(p[:, 1] - p[:, 0], p[:, 2] - p[:, 0])
+    nrm /= np.linalg.norm(nrm, axis=1, keepdims=True)
+    sc = SceneSpec("soup", ntri=n, res=res, W=16, H=16)
+    sc.pos = np.ascontiguousarray(p.reshape(n, 9).astype(np.float32))
+    sc.nrm = np.ascontiguousarray(np.repeat(nrm[:, None], 3, 1).reshape(n, 9).astype(np.float32))
+    want = orc.voxelize(res, sc.cube_size, sc.M, sc.pos, sc.nrm, sc.tri_mat, sc.mat_records, sc.lights,
+                        want=("ref", "count"))
+    with Context(16, 16) as ctx:
+        sc.build(ctx, L.RGBA8, L.AVG_REFERENCE)
+        for _ in range(2):
+            ctx.voxelize()
+            got = ctx.download_level(0)
+            assert np.array_equal(got, want["ref"])
+        nfrag, _ = ctx.voxelize_stats()
+    say(f"  {nfrag} fragments, up to {int(want['count'].max())} in a voxel")
+    assert nfrag == int(want["count"].sum())
+
+
 # ---- trace (kernel c) ----------------------------------------------------------------
 @pytest.mark.parametrize("kind,dtype,res,ntri", [("cornell", L.RGBA8, 64, 34), ("cornell", L.FP16, 64, 34),
                                                  ("soup", L.FP16, 64, 4000), ("soup", L.BF16, 64, 4000),
@@ -563,6 +593,30 @@ def test_voxel_view_matches_oracle(gpu_available, orc, view_dir, lod, extra, dty
     err = np.abs(img - want).max()
     say(f"  max-abs vs FP32 oracle = {err:.3e}")
     assert err == 0.0  # the same float operations in the same order (measured bit-exact)
+
+
+@pytest.mark.parametrize("n,W,H,extra", [(64, 70, 45, {}), (65, 33, 64, {}), (400, 96, 64, {}),
+                                         (150, 61, 47, dict(eye=(0.05, 0.02, 0.1), target=(0.4, -0.1, -1.0),
+                                                            fovy_deg=90.0))])
+def test_voxel_view_chunks_match_oracle(gpu_available, orc, n, W, H, extra):
+    """Tiles with more entries than the composite stages at a time (64), at
+    viewports that cut its 8x8 blocks, with overlapping triangles of all sizes
+    in draw order, the last case clipped around the eye."""
+    say(f"voxel view chunks n={n} {W}x{H} {extra}")
+    res = 32
+    sc = SceneSpec("soup", ntri=n, res=res, W=W, H=H, **extra)
+    sc.pos, sc.nrm = large_triangles(n, n + 1)
+    with Context(W, H) as ctx:
+        sc.build(ctx, L.FP16)
+        ctx.set_voxel_view(3, 0.6)
+        ctx.render()
+        img = ctx.download_image()
+        l0 = decode_level(ctx.download_level(0), L.FP16)
+        mips = {(l, d): decode_level(ctx.download_level(l, d), L.FP16) for l in range(1, 6) for d in range(6)}
+    want = orc.voxel_view(W, H, sc.view, sc.proj, [(sc.M, sc.pos)], res, 6, l0, mips, sc.cube_size, 3, 0.6)
+    err = np.abs(img - want).max()
+    say(f"  max-abs vs FP32 oracle = {err:.3e}")
+    assert err == 0.0
 
 
 def test_voxel_view_over_many_models(gpu_available, orc):

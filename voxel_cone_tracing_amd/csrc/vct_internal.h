@@ -245,7 +245,7 @@ struct vct_context {
   // voxelize scratch
   VctBuf tri_count, tri_off, tri_base;  // per-brick triangle counts + cursors, triangle lists, per-brick offsets
   VctBuf vox_box;                      // voxelize: packed brick box per triangle
-  VctBuf frags_sorted, vox_count, vox_off, scan_tmp, g_scan_tmp, counters;
+  VctBuf vox_count, vox_off, scan_tmp, g_scan_tmp, counters;
   VctBuf setup;  // per-frame triangle list (model index, transform)
   // voxelize: the material terms of the queued models' triangles, in frame
   // order; rebuilt only when shade_epoch (bumped by every material change and
@@ -269,6 +269,7 @@ struct vct_context {
   bool vox_total_pending = false;
   bool vox_sized = false;            // this frame's list was launched against vox_cap
   bool vox_pairs_on_device = false;  // last_candidates still to be read from counters[2]
+  uint32_t vox_frag_bricks = 0;      // per-brick fragment counts of the reference average, still on the device (0: none)
 
   // G-buffer + image
   VctBuf g_list, g_pos, g_nrm, image;

@@ -425,7 +425,7 @@ int vct_destroy(vct_ctx ctx) {
   for (auto& t : ctx->textures)
     if (t.dptr) (void)hipFree(t.dptr);
   VctBuf* bufs[] = {&ctx->d_materials, &ctx->volume, &ctx->tri_count, &ctx->tri_off,
-                    &ctx->tri_base, &ctx->frags_sorted, &ctx->vox_count, &ctx->vox_off,
+                    &ctx->tri_base, &ctx->vox_count, &ctx->vox_off,
                     &ctx->scan_tmp, &ctx->g_scan_tmp, &ctx->counters, &ctx->setup, &ctx->g_list, &ctx->g_pos,
                     &ctx->g_nrm, &ctx->image, &ctx->g_count, &ctx->g_off, &ctx->g_recs,
                     &ctx->mlp_params, &ctx->mlp_m1, &ctx->mlp_m2, &ctx->mlp_packed, &ctx->mlp_bias,
@@ -882,6 +882,15 @@ int vct_get_voxelize_stats(vct_ctx ctx, uint64_t* fragments, uint64_t* candidate
     VCT_HIP(hipStreamSynchronize(ctx->stream));
     ctx->last_candidates = total;
     ctx->vox_pairs_on_device = false;
+  }
+  if (ctx->vox_frag_bricks) {  // the reference average's counts per brick
+    std::vector<uint32_t> per(ctx->vox_frag_bricks);
+    VCT_HIP(hipMemcpyAsync(per.data(), (const uint32_t*)ctx->tri_count.p + per.size(), per.size() * 4,
+                           hipMemcpyDeviceToHost, ctx->stream));
+    VCT_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->last_fragments = 0;
+    for (uint32_t c : per) ctx->last_fragments += c;
+    ctx->vox_frag_bricks = 0;
   }
   if (fragments) *fragments = ctx->last_fragments;
   if (candidates) *candidates = ctx->last_candidates;

@@ -20,13 +20,11 @@
 //     fragment is found exactly once.
 //  4a. exact mean (any storage): 16.16 fixed-point sums in LDS (exact, so
 //     order-independent); the workgroup writes its brick's texels once.
-//  4b. reference running average (RGBA8): a count pass sizes every voxel's
-//     slots (scan over the voxels), a place pass stores (canonical candidate
-//     key, colour) in them and then sorts each voxel's slots and replays the
-//     packed RGBA8 + count-nibble recurrence of imageAtomicRGBA8Avg
-//     (voxelize.frag:95-120) - the result no longer depends on scheduling.
-//     No counter is shared between workgroups (a single append counter for
-//     all fragments serialises at one L2 channel).
+//  4b. reference running average (RGBA8): the workgroup takes its brick's
+//     triangles in their original order, a round's fragments at a time in
+//     LDS, and replays the packed RGBA8 + count-nibble recurrence of
+//     imageAtomicRGBA8Avg (voxelize.frag:95-120) on each voxel's in canonical
+//     order - the result does not depend on scheduling.
 // Bit-exact parts (coverage, voxel coordinates, fragment colours) use no
 // fused multiply-add and correctly rounded division / square root.
 #include <cmath>
@@ -273,10 +271,10 @@ __device__ __forceinline__ bool vox_covers(const VEdges& e) {
 // edge values (wa, wb, wc): coverage, voxel (Morton index) and colour.
 // Returns false if the pixel is not covered or the voxel falls outside the
 // grid (with kBrick: also when the voxel's Morton index >> bshift is not
-// bwant, before any shading).  kKeyOnly stops once the voxel is known.
+// bwant, before any shading).
 // `c` holds the coverage fields (X, Y, area, flags), `sp` the whole record
 // and `sh` the triangle's material terms (both read only for covered pixels).
-template <bool kBrick = false, bool kKeyOnly = false, typename Rec>
+template <bool kBrick = false, typename Rec>
 __device__ __forceinline__ bool shade_w(const Rec& c, const TriRec* sp, const VoxShade* sh, const VEdges& e, int i,
                                         int j, int64_t wa, int64_t wb, int64_t wc, const VoxParams& vp,
                                         uint32_t& key, float4& color, uint32_t bshift = 0, uint32_t bwant = 0) {
@@ -305,7 +303,6 @@ __device__ __forceinline__ bool shade_w(const Rec& c, const TriRec* sp, const Vo
   }
   key = brick_index((uint32_t)v[0], (uint32_t)v[1], (uint32_t)v[2]);
   if (kBrick && (key >> bshift) != bwant) return false;
-  if (kKeyOnly) return true;
   // normal: per-vertex normals (record), interpolated, normalised in the
   // fragment shader (voxelize.frag:134)
   float n[3];
@@ -347,16 +344,6 @@ __device__ __forceinline__ bool shade_w(const Rec& c, const TriRec* sp, const Vo
   color = make_float4(out[0], out[1], out[2], out[3]);
   return true;
 }
-
-// Buffers of the reference running average's two brick passes.
-struct RefPass {
-  uint32_t* vcount;              // count pass: fragments per voxel; place pass: fragments placed so far
-  const uint32_t* vox_off;       // first slot of each voxel's fragments (exclusive scan of the counts)
-  unsigned long long* s_cand;    // canonical key per slot: original triangle << 32 | candidate
-  float4* s_color;               // colour per slot
-  uint32_t nfrag;                // slots
-  uint32_t nvox;                 // voxels of level 0
-};
 
 // ---- exact mean: bricks of the grid accumulated in LDS ----------------------
 // The grid is cut into cubes of kBrick^3 voxels (the whole grid when smaller);
@@ -723,65 +710,34 @@ __device__ __forceinline__ uint32_t dec_nibble(uint32_t m) {
   return (m & 1u) | ((m & 0x100u) >> 7) | ((m & 0x10000u) >> 14) | ((m & 0x1000000u) >> 21);
 }
 
-// Level-0 texel of one voxel from its fragments in slots [beg, end): sorted
-// into canonical order (insertion sort by candidate key), then the packed
-// RGBA8 + count-nibble recurrence of imageAtomicRGBA8Avg, one fragment after
-// another (voxelize.frag:95-120).
-__device__ __forceinline__ uint32_t replay_voxel(unsigned long long* __restrict__ s_cand,
-                                                 float4* __restrict__ s_color, uint32_t beg, uint32_t end) {
+// One fragment (vx .. vw: its colour times 255) into a voxel's packed RGBA8 +
+// count nibble, as imageAtomicRGBA8Avg does (voxelize.frag:95-120).
+__device__ __forceinline__ uint32_t replay_step(uint32_t stored, float vx, float vy, float vz, float vw) {
 #pragma clang fp contract(off)
-  // canonical order: insertion sort of the bucket by candidate index
-  for (uint32_t i = beg + 1; i < end; ++i) {
-    const unsigned long long kc = s_cand[i];
-    const float4 kv = s_color[i];
-    uint32_t j = i;
-    while (j > beg && s_cand[j - 1] > kc) {
-      s_cand[j] = s_cand[j - 1];
-      s_color[j] = s_color[j - 1];
-      --j;
-    }
-    s_cand[j] = kc;
-    s_color[j] = kv;
-  }
-  uint32_t stored = 0u;
-  for (uint32_t i = beg; i < end; ++i) {
-    const float4 c = s_color[i];
-    const float vx = c.x * 255.0f, vy = c.y * 255.0f, vz = c.z * 255.0f, vw = c.w * 255.0f;
-    if (stored == 0u) {  // imageAtomicCompSwap(0 -> new) succeeds
-      stored = enc_nibble(conv_vec4_to_rgba8(vx, vy, vz, vw), 1u);
-      continue;
-    }
-    const uint32_t cur = stored & 0xFEFEFEFEu;
-    float rx = (float)(cur & 0xffu), ry = (float)((cur >> 8) & 0xffu), rz = (float)((cur >> 16) & 0xffu),
-          rw = (float)(cur >> 24);
-    uint32_t n = dec_nibble(stored);
-    const float fn = (float)n;
-    rx = rx * fn + vx;
-    ry = ry * fn + vy;
-    rz = rz * fn + vz;
-    rw = rw * fn + vw;
-    ++n;
-    const float fn1 = (float)n;
-    rx = rx / fn1;
-    ry = ry / fn1;
-    rz = rz / fn1;
-    rw = rw / fn1;
-    rx = __builtin_rintf(rx / 2.0f) * 2.0f;
-    ry = __builtin_rintf(ry / 2.0f) * 2.0f;
-    rz = __builtin_rintf(rz / 2.0f) * 2.0f;
-    rw = __builtin_rintf(rw / 2.0f) * 2.0f;
-    stored = enc_nibble(conv_vec4_to_rgba8(rx, ry, rz, rw), n);
-  }
-  return stored;
+  if (stored == 0u)  // imageAtomicCompSwap(0 -> new) succeeds
+    return enc_nibble(conv_vec4_to_rgba8(vx, vy, vz, vw), 1u);
+  const uint32_t cur = stored & 0xFEFEFEFEu;
+  float rx = (float)(cur & 0xffu), ry = (float)((cur >> 8) & 0xffu), rz = (float)((cur >> 16) & 0xffu),
+        rw = (float)(cur >> 24);
+  uint32_t n = dec_nibble(stored);
+  const float fn = (float)n;
+  rx = rx * fn + vx;
+  ry = ry * fn + vy;
+  rz = rz * fn + vz;
+  rw = rw * fn + vw;
+  ++n;
+  const float fn1 = (float)n;
+  rx = rx / fn1;
+  ry = ry / fn1;
+  rz = rz / fn1;
+  rw = rw / fn1;
+  rx = __builtin_rintf(rx / 2.0f) * 2.0f;
+  ry = __builtin_rintf(ry / 2.0f) * 2.0f;
+  rz = __builtin_rintf(rz / 2.0f) * 2.0f;
+  rw = __builtin_rintf(rw / 2.0f) * 2.0f;
+  return enc_nibble(conv_vec4_to_rgba8(rx, ry, rz, rw), n);
 }
 
-// kMode: kExactMean sums the brick's fragments and writes its texels.  The
-// reference running average takes two passes over the same candidates:
-// kRefCount counts the fragments per voxel (into r.vcount), and after the
-// counts are scanned into r.vox_off, kRefPlace shades them and stores
-// (canonical key, colour) in the voxel's slots, in no particular order, and
-// then replays its brick's voxels and writes their texels.  No global counter
-// is shared between workgroups.
 // The brick lists' capacity: a brick whose range [off, off + count) runs past
 // `cap` entries walks the packed brick boxes of all `ntri` triangles and keeps
 // those that contain it (the same triangles its list would hold).
@@ -791,51 +747,184 @@ struct ListCap {
   uint32_t cap;
 };
 
-enum { kExactMean = 0, kRefCount = 1, kRefPlace = 2 };
-// Its phases wait on LDS and L2 more than they compute (fewer VALU
-// instructions per fragment or candidate measured no faster; more waves
-// did), so it runs at 8 waves per SIMD: 64 registers, no spills, and LDS for
-// 8 workgroups per CU.
-template <int DT, int kMode>
-__global__ __launch_bounds__(kBrickThreads) __attribute__((amdgpu_waves_per_eu(8))) void vox_brick_kernel(VoxParams vp, const TriRec* __restrict__ recs,
-                                                                  const VoxShade* __restrict__ shade,
-                                                                  const uint32_t* __restrict__ brick_count,
-                                                                  const uint32_t* __restrict__ brick_off,
-                                                                  const uint32_t* __restrict__ list,
-                                                                  ListCap lc, void* level0, RefPass r) {
-  constexpr int kVox = kBrick * kBrick * kBrick;
-  __shared__ uint32_t s_sum[4][kMode == kExactMean ? kVox : 1];
-  __shared__ uint32_t s_cnt[kVox];
-  __shared__ uint32_t s_base[kMode == kRefPlace ? kVox : 1];
-  __shared__ CovRec s_cov[kBrickItems];
-  __shared__ uint32_t s_end[kBrickItems];  // inclusive prefix of candidate counts
-  __shared__ uint32_t s_org[kBrickItems];  // clipped box origin: i | j << 16
-  __shared__ uint32_t s_div[kBrickItems];  // ceil(65536 / width) | width << 20
-  __shared__ uint32_t s_wsum[kBrickItems / 64];
-  __shared__ uint32_t s_q[kBrickThreads / 64][128];  // per-wave queue of covered candidates
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const BrickGeom g = brick_geom(vp.res);
-  // Workgroups are dealt to the 8 XCDs round-robin in dispatch order; XCD k
-  // takes the k-th eighth of the bricks in Morton order (one region of the
-  // grid), so the records of triangles shared by neighbouring bricks stay
-  // in one L2 (voxelize 1.04 -> 1.01 ms)
-  uint32_t brick = blockIdx.x;
-  {
-    const uint32_t full = gridDim.x & ~7u;
-    if (brick < full) brick = (brick & 7u) * (full >> 3) + (brick >> 3);
+// A round of up to kBrickItems triangles of a brick, in LDS.
+struct BrickRound {
+  CovRec cov[kBrickItems];
+  uint32_t end[kBrickItems];  // inclusive prefix of candidate counts
+  uint32_t org[kBrickItems];  // clipped box origin: i | j << 16
+  uint32_t div[kBrickItems];  // ceil(65536 / width) | width << 20
+  uint32_t wsum[kBrickItems / 64];
+  uint32_t q[kBrickThreads / 64][128];  // per-wave queue of covered candidates
+};
+
+// Stages triangle t as entry `slot` of the round for the brick at bc (bricks);
+// returns its candidate pixels: its box clipped to the brick's footprint.  A
+// covered pixel (i, j) lands in voxel (i >> 1, j >> 1) on the projection
+// plane: its centre sits a quarter voxel inside that voxel, and the
+// interpolated position is a convex combination of the vertices that differs
+// from the centre by the 1/512-pixel vertex snap plus rounding, far below a
+// quarter voxel.  So pixels outside the footprint never land in the brick.
+__device__ __forceinline__ uint32_t brick_stage(BrickRound& B, int slot, uint32_t t, const TriRec* __restrict__ recs,
+                                                const uint32_t (&bc)[3], int span, int lim) {
+  const TriRec* rp = recs + t;
+  const uint32_t fl = rp->flags;
+  const int axis = (int)((fl >> 1) & 3u);
+  const int ia = axis == 0 ? 1 : 0, ib = axis == 2 ? 1 : 2;
+  const int qh = (int)(fl >> 8);
+  const int qx0 = rp->qx0, qy0 = rp->qy0, qw = rp->qw;
+  const int fx = (int)bc[ia] * span, fy = (int)bc[ib] * span;
+  const int i0 = max(qx0, fx), i1 = min(min(qx0 + 2 * qw - 1, fx + span - 1), lim);
+  const int j0 = max(qy0, fy), j1 = min(min(qy0 + 2 * qh - 1, fy + span - 1), lim);
+  if (i1 < i0 || j1 < j0) return 0u;
+  const uint32_t cw = (uint32_t)(i1 - i0 + 1);
+  B.org[slot] = (uint32_t)i0 | ((uint32_t)j0 << 16);
+  B.div[slot] = ((65536u + cw - 1u) / cw) | (cw << 20);
+  CovRec cr;
+  cr.area = rp->area;
+  for (int v = 0; v < 3; ++v) {
+    cr.X[v] = rp->X[v];
+    cr.Y[v] = rp->Y[v];
   }
+  cr.flags = fl;
+  cr.tri = t;
+  B.cov[slot] = cr;
+  return cw * (uint32_t)(j1 - j0 + 1);
+}
+
+// Prefix of the entries' candidate counts (cnt of thread tid < kBrickItems);
+// every thread of the workgroup calls it; returns the total.
+__device__ __forceinline__ uint32_t brick_prefix(BrickRound& B, uint32_t cnt) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  uint32_t x = cnt;
+  if (tid < kBrickItems) {
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) B.wsum[wave] = x;
+  }
+  __syncthreads();
+  if (tid < kBrickItems) {
+    for (int w = 0; w < wave; ++w) x += B.wsum[w];
+    B.end[tid] = x;
+  }
+  __syncthreads();
+  return B.end[kBrickItems - 1];
+}
+
+// The round's candidates in two phases.  1: the wave's 64 candidates are
+// tested for coverage only (exact edge functions, top-left rule); the covered
+// ones are appended to the wave's queue in LDS.  2: whenever the queue holds
+// 64, every lane takes one (entry | i << 8 | j << 19) and runs the exact
+// fragment path (voxel address, brick test, shading, accumulation), so the
+// expensive part runs with all lanes busy instead of on the covered ~40 % of
+// them.  The set of fragments, and every value computed for one, is the same
+// as testing each candidate in full.  `fragment` is called by whole waves:
+// fragment(d, on).
+template <class Frag>
+__device__ __forceinline__ void brick_scan(BrickRound& B, uint32_t total, Frag&& fragment) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t* s_end = B.end;
+  uint32_t* q = B.q[wave];
+  uint32_t qn = 0;    // entries in the queue (the same in every lane)
+  uint32_t own0 = 0;  // the entry of the wave's first candidate (the same in every lane; never decreases)
+  for (uint32_t cb = (uint32_t)wave * 64u; cb < total; cb += kBrickThreads) {
+    const uint32_t c = cb + (uint32_t)lane;
+    // The entry (triangle) of each lane's candidate, for the window
+    // [cb, cb + 64) of consecutive candidates.  own0 moves to the first
+    // entry ending after cb: lane k tests entry own0 + k and the ballot
+    // counts those ending at or before cb (a prefix, the ends being
+    // sorted).  Lane k then holds the end of entry own0 + k, and each lane
+    // finds how many of these end at or before its candidate by a binary
+    // search over the lanes (register shuffles): that count from own0 is
+    // its entry.  A window that spans more than 64 entries (entries with
+    // one candidate or none) finishes with a per-lane walk.
+    for (;;) {
+      const uint32_t ek = own0 + (uint32_t)lane < kBrickItems ? s_end[own0 + lane] : 0xffffffffu;
+      const uint32_t k = (uint32_t)__popcll(__ballot(ek <= cb));
+      own0 += k;
+      if (k < 64u) break;
+    }
+    const uint32_t ek = own0 + (uint32_t)lane < kBrickItems ? s_end[own0 + lane] : 0xffffffffu;
+    // Only entries ending inside the window can end at or before a
+    // candidate: nend of them, the first nend lanes (the ends are sorted).  A
+    // window usually spans a few entries, and a scan of their ends read
+    // into scalar registers has no LDS round trip in its chain, where the
+    // binary search takes seven dependent shuffles; the count is the same.
+    const uint32_t nend = (uint32_t)__popcll(__ballot(ek < cb + 64u));
+    uint32_t past = 0;
+    if (nend <= 8u) {
+      for (uint32_t k = 0; k < nend; ++k) past += (uint32_t)__builtin_amdgcn_readlane((int)ek, (int)k) <= c ? 1u : 0u;
+    } else {
+      for (uint32_t st = 32; st; st >>= 1)
+        if ((uint32_t)__shfl(ek, (int)(past + st - 1u), 64) <= c) past += st;
+      if ((uint32_t)__shfl(ek, (int)past, 64) <= c) ++past;
+    }
+    bool hit = false;
+    uint32_t desc = 0;
+    if (c < total) {
+      uint32_t lo = own0 + past;
+      if (past == 64u)
+        while (s_end[lo] <= c) ++lo;
+      const uint32_t local = c - (lo ? s_end[lo - 1] : 0u);
+      const uint32_t dv = B.div[lo], cw = dv >> 20;
+      const uint32_t row = (local * (dv & 0xfffffu)) >> 16;  // exact: local < 35 * 35, cw <= 35
+      const uint32_t col = local - row * cw;
+      const uint32_t org = B.org[lo];
+      const int i = (int)(org & 0xffffu) + (int)col, j = (int)(org >> 16) + (int)row;
+      const CovRec cr = B.cov[lo];
+      VEdges e;
+      vox_edges(cr, i, j, e);
+      hit = vox_covers(e);
+      desc = lo | ((uint32_t)i << 8) | ((uint32_t)j << 19);
+    }
+    const unsigned long long m = __ballot(hit);
+    if (hit) q[qn + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = desc;
+    qn += (uint32_t)__popcll(m);
+    if (qn >= 64u) {
+      qn -= 64u;
+      fragment(q[qn + (uint32_t)lane], true);
+    }
+  }
+  if (qn) {
+    const bool on = (uint32_t)lane < qn;
+    fragment(on ? q[lane] : 0u, on);
+  }
+}
+
+// The brick of a workgroup: workgroups are dealt to the 8 XCDs round-robin in
+// dispatch order; XCD k takes the k-th eighth of the bricks in Morton order
+// (one region of the grid), so the records of triangles shared by neighbouring
+// bricks stay in one L2 (voxelize 1.04 -> 1.01 ms).
+__device__ __forceinline__ uint32_t brick_of_block() {
+  const uint32_t full = gridDim.x & ~7u, b = blockIdx.x;
+  return b < full ? (b & 7u) * (full >> 3) + (b >> 3) : b;
+}
+
+// Exact mean: sums the brick's fragments and writes its texels.  Its phases
+// wait on LDS and L2 more than they compute (fewer VALU instructions per
+// fragment or candidate measured no faster; more waves did), so it runs at 8
+// waves per SIMD: 64 registers, no spills, and LDS for 8 workgroups per CU.
+template <int DT>
+__global__ __launch_bounds__(kBrickThreads) __attribute__((amdgpu_waves_per_eu(8))) void vox_brick_kernel(
+    VoxParams vp, const TriRec* __restrict__ recs, const VoxShade* __restrict__ shade,
+    const uint32_t* __restrict__ brick_count, const uint32_t* __restrict__ brick_off,
+    const uint32_t* __restrict__ list, ListCap lc, void* level0) {
+  constexpr int kVox = kBrick * kBrick * kBrick;
+  __shared__ uint32_t s_sum[4][kVox];
+  __shared__ uint32_t s_cnt[kVox];
+  __shared__ BrickRound s_round;
+  const int tid = threadIdx.x;
+  const BrickGeom g = brick_geom(vp.res);
+  const uint32_t brick = brick_of_block();
   const uint32_t nvox = 1u << (3 * g.bits);
   const uint32_t bshift = 3 * g.bits;
   const uint32_t bc[3] = {compact3(brick), compact3(brick >> 1), compact3(brick >> 2)};
   for (uint32_t v = tid; v < nvox; v += kBrickThreads) {
-    if constexpr (kMode == kExactMean) {
-      s_sum[0][v] = 0u;
-      s_sum[1][v] = 0u;
-      s_sum[2][v] = 0u;
-      s_sum[3][v] = 0u;
-    }
-    if constexpr (kMode == kRefPlace)
-      s_base[v] = r.vox_off[brick * nvox + v];
+    s_sum[0][v] = 0u;
+    s_sum[1][v] = 0u;
+    s_sum[2][v] = 0u;
+    s_sum[3][v] = 0u;
     s_cnt[v] = 0u;
   }
   const uint32_t n = brick_count[brick], base = brick_off[brick];
@@ -847,7 +936,6 @@ __global__ __launch_bounds__(kBrickThreads) __attribute__((amdgpu_waves_per_eu(8
   const int span = 2 << g.bits;  // footprint of the brick on the raster, pixels per axis
   __syncthreads();
   for (uint32_t b0 = 0; b0 < nitems; b0 += kBrickItems) {
-    uint32_t cnt = 0;
     uint32_t t = b0 + (uint32_t)tid;
     bool in = tid < kBrickItems && t < nitems;
     if (in && walk) {  // the box as pack_box stores it: first brick, bricks per axis
@@ -857,171 +945,283 @@ __global__ __launch_bounds__(kBrickThreads) __attribute__((amdgpu_waves_per_eu(8
     } else if (in) {
       t = list[base + t];
     }
-    if (in) {
-      const TriRec* rp = recs + t;
-      const uint32_t fl = rp->flags;
-      const int axis = (int)((fl >> 1) & 3u);
-      const int ia = axis == 0 ? 1 : 0, ib = axis == 2 ? 1 : 2;
-      const int qh = (int)(fl >> 8);
-      const int qx0 = rp->qx0, qy0 = rp->qy0, qw = rp->qw;
-      // the brick's footprint clipped to the triangle's box.  A covered
-      // pixel (i, j) lands in voxel (i >> 1, j >> 1) on the projection plane:
-      // its centre sits a quarter voxel inside that voxel, and the
-      // interpolated position is a convex combination of the vertices that
-      // differs from the centre by the 1/512-pixel vertex snap plus rounding,
-      // far below a quarter voxel.  So pixels outside the footprint never
-      // land in the brick.
-      const int fx = (int)bc[ia] * span, fy = (int)bc[ib] * span;
-      const int i0 = max(qx0, fx), i1 = min(min(qx0 + 2 * qw - 1, fx + span - 1), lim);
-      const int j0 = max(qy0, fy), j1 = min(min(qy0 + 2 * qh - 1, fy + span - 1), lim);
-      if (i1 >= i0 && j1 >= j0) {
-        const uint32_t cw = (uint32_t)(i1 - i0 + 1);
-        cnt = cw * (uint32_t)(j1 - j0 + 1);
-        s_org[tid] = (uint32_t)i0 | ((uint32_t)j0 << 16);
-        s_div[tid] = ((65536u + cw - 1u) / cw) | (cw << 20);
-        CovRec cr;
-        cr.area = rp->area;
-        for (int v = 0; v < 3; ++v) {
-          cr.X[v] = rp->X[v];
-          cr.Y[v] = rp->Y[v];
-        }
-        cr.flags = fl;
-        cr.tri = t;
-        s_cov[tid] = cr;
-      }
-    }
-    uint32_t x = cnt;
-    if (tid < kBrickItems) {
-      for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-      }
-      if (lane == 63) s_wsum[wave] = x;
-    }
-    __syncthreads();
-    if (tid < kBrickItems) {
-      for (int w = 0; w < wave; ++w) x += s_wsum[w];
-      s_end[tid] = x;
-    }
-    __syncthreads();
-    const uint32_t total = s_end[kBrickItems - 1];
-    // Candidates in two phases.  1: the wave's 64 candidates are tested for
-    // coverage only (exact edge functions, top-left rule); the covered ones
-    // are appended to the wave's queue in LDS.  2: whenever the queue holds
-    // 64, every lane takes one and runs the exact fragment path (voxel
-    // address, brick test, shading, accumulation), so the expensive part
-    // runs with all lanes busy instead of on the covered ~40 % of them.  The
-    // set of fragments, and every value computed for one, is the same as
-    // testing each candidate in full.
-    uint32_t* q = s_q[wave];
-    uint32_t qn = 0;  // entries in the queue (the same in every lane)
-    uint32_t own0 = 0;  // the entry of the wave's first candidate (the same in every lane; never decreases)
-    auto fragment = [&](uint32_t d) {
-      const uint32_t lo = d & 255u;
+    const uint32_t total = brick_prefix(s_round, in ? brick_stage(s_round, tid, t, recs, bc, span, lim) : 0u);
+    brick_scan(s_round, total, [&](uint32_t d, bool on) {
+      if (!on) return;
+      const CovRec cr = s_round.cov[d & 255u];
       const int i = (int)((d >> 8) & 0x7ffu), j = (int)(d >> 19);
-      const CovRec cr = s_cov[lo];
       VEdges e;
       vox_edges(cr, i, j, e);
       uint32_t key;
       float4 color;
-      if (!shade_w<true, kMode == kRefCount>(cr, recs + cr.tri, shade + cr.tri, e, i, j, e.w[0], e.w[1], e.w[2], vp, key,
-                                             color, bshift, brick))
-        return;
-      const uint32_t lv = key & (nvox - 1u);
-      if constexpr (kMode == kExactMean) {
-        brick_add(s_sum, s_cnt, lv, color);
-      } else if constexpr (kMode == kRefCount) {
-        atomicAdd(&s_cnt[lv], 1u);
-      } else {
-        // canonical key: the candidate's place in the triangle's quad-ordered
-        // box (2x2 quads row by row, each quad x then y)
-        const TriRec* rp = recs + cr.tri;
-        const uint32_t dx = (uint32_t)(i - rp->qx0), dy = (uint32_t)(j - rp->qy0);
-        const uint32_t lc = (((dy >> 1) * (uint32_t)rp->qw + (dx >> 1)) << 2) | ((dy & 1u) << 1) | (dx & 1u);
-        const uint32_t slot = s_base[lv] + atomicAdd(&s_cnt[lv], 1u);
-        if (slot < r.nfrag) {  // always: the count pass found the same fragments
-          r.s_cand[slot] = ((unsigned long long)rp->otri << 32) | (unsigned long long)lc;
-          r.s_color[slot] = color;
-        }
-      }
-    };
-    for (uint32_t cb = (uint32_t)wave * 64u; cb < total; cb += kBrickThreads) {
-      const uint32_t c = cb + (uint32_t)lane;
-      // The entry (triangle) of each lane's candidate, for the window
-      // [cb, cb + 64) of consecutive candidates.  own0 moves to the first
-      // entry ending after cb: lane k tests entry own0 + k and the ballot
-      // counts those ending at or before cb (a prefix, the ends being
-      // sorted).  Lane k then holds the end of entry own0 + k, and each lane
-      // finds how many of these end at or before its candidate by a binary
-      // search over the lanes (register shuffles): that count from own0 is
-      // its entry.  A window that spans more than 64 entries (entries with
-      // one candidate or none) finishes with a per-lane walk.
-      for (;;) {
-        const uint32_t ek = own0 + (uint32_t)lane < kBrickItems ? s_end[own0 + lane] : 0xffffffffu;
-        const uint32_t k = (uint32_t)__popcll(__ballot(ek <= cb));
-        own0 += k;
-        if (k < 64u) break;
-      }
-      const uint32_t ek = own0 + (uint32_t)lane < kBrickItems ? s_end[own0 + lane] : 0xffffffffu;
-      // Only entries ending inside the window can end at or before a
-      // candidate: nend of them, the first nend lanes (the ends are sorted).  A
-      // window usually spans a few entries, and a scan of their ends read
-      // into scalar registers has no LDS round trip in its chain, where the
-      // binary search takes seven dependent shuffles; the count is the same.
-      const uint32_t nend = (uint32_t)__popcll(__ballot(ek < cb + 64u));
-      uint32_t past = 0;
-      if (nend <= 8u) {
-        for (uint32_t k = 0; k < nend; ++k) past += (uint32_t)__builtin_amdgcn_readlane((int)ek, (int)k) <= c ? 1u : 0u;
-      } else {
-        for (uint32_t st = 32; st; st >>= 1)
-          if ((uint32_t)__shfl(ek, (int)(past + st - 1u), 64) <= c) past += st;
-        if ((uint32_t)__shfl(ek, (int)past, 64) <= c) ++past;
-      }
-      bool hit = false;
-      uint32_t desc = 0;
-      if (c < total) {
-        uint32_t lo = own0 + past;
-        if (past == 64u)
-          while (s_end[lo] <= c) ++lo;
-        const uint32_t local = c - (lo ? s_end[lo - 1] : 0u);
-        const uint32_t dv = s_div[lo], cw = dv >> 20;
-        const uint32_t row = (local * (dv & 0xfffffu)) >> 16;  // exact: local < 35 * 35, cw <= 35
-        const uint32_t col = local - row * cw;
-        const uint32_t org = s_org[lo];
-        const int i = (int)(org & 0xffffu) + (int)col, j = (int)(org >> 16) + (int)row;
-        const CovRec cr = s_cov[lo];
-        VEdges e;
-        vox_edges(cr, i, j, e);
-        hit = vox_covers(e);
-        desc = lo | ((uint32_t)i << 8) | ((uint32_t)j << 19);
-      }
-      const unsigned long long m = __ballot(hit);
-      if (hit) q[qn + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = desc;
-      qn += (uint32_t)__popcll(m);
-      if (qn >= 64u) {
-        qn -= 64u;
-        fragment(q[qn + (uint32_t)lane]);
-      }
-    }
-    if ((uint32_t)lane < qn) fragment(q[lane]);
+      if (shade_w<true>(cr, recs + cr.tri, shade + cr.tri, e, i, j, e.w[0], e.w[1], e.w[2], vp, key, color, bshift,
+                        brick))
+        brick_add(s_sum, s_cnt, key & (nvox - 1u), color);
+    });
     __syncthreads();
   }
-  if constexpr (kMode == kExactMean) {
-    for (uint32_t v = tid; v < nvox; v += kBrickThreads)
-      store_mean<DT>(level0, brick * nvox + v, s_cnt[v], s_sum[0][v], s_sum[1][v], s_sum[2][v], s_sum[3][v]);
-  } else if (kMode == kRefCount) {
-    // one workgroup per brick: it writes the count of every voxel it owns
-    for (uint32_t v = tid; v < nvox; v += kBrickThreads) r.vcount[brick * nvox + v] = s_cnt[v];
-  } else {
-    // the barrier makes the workgroup's slot stores visible to all its lanes
-    // (the loop above ended with one)
-    for (uint32_t v = tid; v < nvox; v += kBrickThreads) {
-      const uint32_t gv = brick * nvox + v;
-      const uint32_t beg = r.vox_off[gv];
-      const uint32_t end = gv + 1u < r.nvox ? r.vox_off[gv + 1u] : r.nfrag;
-      reinterpret_cast<uint32_t*>(level0)[gv] = replay_voxel(r.s_cand, r.s_color, beg, end);
+  for (uint32_t v = tid; v < nvox; v += kBrickThreads)
+    store_mean<DT>(level0, brick * nvox + v, s_cnt[v], s_sum[0][v], s_sum[1][v], s_sum[2][v], s_sum[3][v]);
+}
+
+// ---- reference running average: one pass over the brick's triangles in order --------
+// The average depends on the order of a voxel's fragments: triangle, then
+// pixel quad, then pixel.  The workgroup sorts the brick's list by original
+// triangle index (in LDS up to kRefSort triangles, by a radix sort in global
+// memory past that), takes the triangles in rounds in that order, keeps a
+// round's fragments in LDS (colour and a 15-bit key: place of the triangle in
+// the round, pixel in the brick's footprint), groups them by voxel, and each
+// voxel's lane sorts its few by key and replays the packed RGBA8 + count
+// nibble recurrence on them.  A round whose fragments do not fit is taken
+// again with half its triangles: three triangles always fit (a footprint has
+// 256 pixels).  A pass that counted the fragments of every voxel, a scan over
+// the voxels, a host wait for the number of fragments and a pass that stored
+// them in global memory, sorted and replayed them took the voxelize pass of
+// the 1M-triangle soup at 256^3 1.15 ms; this one pass 0.81 (voxels replayed
+// in their own order rather than the fullest first: 0.99).
+constexpr int kRefFrags = 768;   // fragments of a round (512 at 6 waves per SIMD: no faster)
+constexpr int kRefSort = 1024;   // triangles sorted in LDS
+
+struct RefLds {
+  union {
+    struct {
+      float col[3][kRefFrags];
+      uint16_t key[kRefFrags], vox[kRefFrags], idx[kRefFrags];
+    };
+    unsigned long long sort[kRefSort];  // original triangle << 32 | triangle
+    uint32_t hist[4][256];
+  };
+};
+static_assert(sizeof(RefLds) >= kRefSort * 8, "the sort uses the fragments' space");
+
+// Sorts the brick's list segment by original triangle index in global memory
+// (4 stable passes of 8 bits between the segment and its place in `other`; an
+// even number of passes ends where it began).
+__device__ void ref_radix_sort(RefLds& R, uint32_t* seg, uint32_t* other, uint32_t n, const TriRec* __restrict__ recs) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int pass = 0; pass < 4; ++pass) {
+    uint32_t* src = pass & 1 ? other : seg;
+    uint32_t* dst = pass & 1 ? seg : other;
+    const int sh = 8 * pass;
+    __syncthreads();
+    R.hist[0][tid] = 0u;
+    __syncthreads();
+    for (uint32_t k = tid; k < n; k += kBrickThreads) atomicAdd(&R.hist[0][(recs[src[k]].otri >> sh) & 255u], 1u);
+    __syncthreads();
+    // exclusive prefix of the 256 counts: where the digit's next element goes
+    const uint32_t c = R.hist[0][tid];
+    uint32_t x = c;
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) R.hist[1][wave] = x;
+    __syncthreads();
+    uint32_t at = x - c;
+    for (int w = 0; w < wave; ++w) at += R.hist[1][w];
+    __syncthreads();
+    R.hist[0][tid] = at;
+    __syncthreads();
+    for (uint32_t b = 0; b < n; b += kBrickThreads) {  // 256 elements at a time, waves one after another
+      const uint32_t k = b + (uint32_t)tid;
+      const bool in = k < n;
+      const uint32_t t = in ? src[k] : 0u;
+      const uint32_t dg = in ? (recs[t].otri >> sh) & 255u : 0u;
+      unsigned long long same = __ballot(in);
+      for (int bit = 0; bit < 8; ++bit) {
+        const unsigned long long m = __ballot((dg >> bit) & 1u);
+        same &= (dg >> bit) & 1u ? m : ~m;
+      }
+      const uint32_t rank = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+      for (int w = 0; w < kBrickThreads / 64; ++w) {
+        if (w == wave && in) {
+          const uint32_t p = R.hist[0][dg] + rank;
+          dst[p] = t;
+        }
+        __syncthreads();
+        if (w == wave && in && rank == 0u) R.hist[0][dg] += (uint32_t)__popcll(same);
+        __syncthreads();
+      }
     }
   }
+  __syncthreads();
+}
+
+__global__ __launch_bounds__(kBrickThreads) __attribute__((amdgpu_waves_per_eu(5))) void vox_ref_kernel(
+    VoxParams vp, const TriRec* __restrict__ recs, const VoxShade* __restrict__ shade, const uint32_t* brick_count,
+    const uint32_t* __restrict__ brick_off, uint32_t* list, uint32_t* list2, uint32_t* __restrict__ level0,
+    uint32_t* __restrict__ brick_frags) {
+#pragma clang fp contract(off)
+  constexpr int kVox = kBrick * kBrick * kBrick;
+  __shared__ uint32_t s_state[kVox];  // the voxels' texels so far
+  __shared__ uint32_t s_cnt[kVox];    // fragments of the round per voxel
+  __shared__ uint16_t s_off[kVox];    // first place of the voxel's fragments in idx
+  __shared__ float s_alpha[kBrickItems];
+  __shared__ uint16_t s_ord[kVox];    // the round's voxels, most fragments first
+  __shared__ uint32_t s_place[64];    // voxels by fragment count (63: or more), then where they go in s_ord
+  __shared__ BrickRound s_round;
+  __shared__ RefLds R;
+  __shared__ uint32_t s_nfrag, s_wsum[kBrickThreads / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const BrickGeom g = brick_geom(vp.res);
+  const uint32_t brick = brick_of_block();
+  const uint32_t nvox = 1u << (3 * g.bits);
+  const uint32_t bshift = 3 * g.bits;
+  const uint32_t bc[3] = {compact3(brick), compact3(brick >> 1), compact3(brick >> 2)};
+  const int lim = 2 * (int)vp.res - 1;
+  const int span = 2 << g.bits;  // footprint of the brick on the raster, pixels per axis
+  const uint32_t n = brick_count[brick], base = brick_off[brick];
+  for (uint32_t v = tid; v < nvox; v += kBrickThreads) s_state[v] = 0u;
+  uint32_t* seg = list + base;
+  // ---- the list in order ---------------------------------------------------------
+  if (n > (uint32_t)kRefSort) {
+    ref_radix_sort(R, seg, list2 + base, n, recs);
+  } else if (n > 1u) {
+    uint32_t m = 64;  // a bitonic sort of the next power of two
+    while (m < n) m <<= 1;
+    for (uint32_t k = tid; k < m; k += kBrickThreads) {
+      unsigned long long e = ~0ull;
+      if (k < n) {
+        const uint32_t t = seg[k];
+        e = ((unsigned long long)recs[t].otri << 32) | t;
+      }
+      R.sort[k] = e;
+    }
+    for (uint32_t w = 2; w <= m; w <<= 1)
+      for (uint32_t d = w >> 1; d; d >>= 1) {
+        __syncthreads();
+        for (uint32_t k = tid; k < m / 2; k += kBrickThreads) {
+          const uint32_t lo = ((k & ~(d - 1u)) << 1) | (k & (d - 1u)), hi = lo | d;
+          const unsigned long long a = R.sort[lo], b = R.sort[hi];
+          if ((a > b) == ((lo & w) == 0u)) {
+            R.sort[lo] = b;
+            R.sort[hi] = a;
+          }
+        }
+      }
+    __syncthreads();
+    for (uint32_t k = tid; k < n; k += kBrickThreads) seg[k] = (uint32_t)R.sort[k];
+  }
+  uint32_t nall = 0;                 // fragments of the brick
+  uint32_t take = kBrickItems;       // triangles to try in a round
+  for (uint32_t pos = 0; pos < n;) {
+    const uint32_t m = min(take, n - pos);
+    for (uint32_t v = tid; v < nvox; v += kBrickThreads) s_cnt[v] = 0u;
+    if (tid < 64) s_place[tid] = 0u;
+    if (tid == 0) s_nfrag = 0u;
+    __syncthreads();  // also: the sorted segment is in memory, the round before is done
+    uint32_t cnt = 0;
+    if ((uint32_t)tid < m) {
+      const uint32_t t = seg[pos + tid];
+      cnt = brick_stage(s_round, tid, t, recs, bc, span, lim);
+      s_alpha[tid] = shade[t].alpha;
+    }
+    const uint32_t total = brick_prefix(s_round, cnt);
+    brick_scan(s_round, total, [&](uint32_t d, bool on) {
+      const uint32_t lo = d & 255u;
+      const int i = (int)((d >> 8) & 0x7ffu), j = (int)(d >> 19);
+      uint32_t key = 0;
+      float4 color = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (on) {
+        const CovRec cr = s_round.cov[lo];
+        VEdges e;
+        vox_edges(cr, i, j, e);
+        on = shade_w<true>(cr, recs + cr.tri, shade + cr.tri, e, i, j, e.w[0], e.w[1], e.w[2], vp, key, color, bshift,
+                           brick);
+      }
+      const unsigned long long mk = __ballot(on);
+      if (!mk) return;
+      uint32_t slot = 0;
+      if (lane == 0) slot = atomicAdd(&s_nfrag, (uint32_t)__popcll(mk));
+      slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)slot) + (uint32_t)__popcll(mk & ((1ull << lane) - 1ull));
+      if (on && slot < (uint32_t)kRefFrags) {
+        const uint32_t lv = key & (nvox - 1u);
+        R.col[0][slot] = color.x;
+        R.col[1][slot] = color.y;
+        R.col[2][slot] = color.z;
+        // the order within a triangle: 2x2 quads row by row, each quad x then y
+        R.key[slot] = (uint16_t)((lo << 8) | (((uint32_t)j >> 1 & 7u) << 5) | (((uint32_t)i >> 1 & 7u) << 2) |
+                                 (((uint32_t)j & 1u) << 1) | ((uint32_t)i & 1u));
+        R.vox[slot] = (uint16_t)lv;
+        atomicAdd(&s_cnt[lv], 1u);
+      }
+    });
+    __syncthreads();
+    const uint32_t nf = s_nfrag;
+    if (nf > (uint32_t)kRefFrags) {  // too many: the same triangles in halves
+      take = max(m / 2u, 3u);
+      __syncthreads();
+      continue;
+    }
+    // ---- group by voxel: two voxels per lane --------------------------------------
+    const uint32_t v0 = 2u * (uint32_t)tid, v1 = v0 + 1u;
+    const uint32_t c0 = v0 < nvox ? s_cnt[v0] : 0u, c1 = v1 < nvox ? s_cnt[v1] : 0u;
+    uint32_t x = c0 + c1;
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) s_wsum[wave] = x;
+    __syncthreads();
+    uint32_t off = x - c0 - c1;
+    for (int w = 0; w < wave; ++w) off += s_wsum[w];
+    if (v0 < nvox) s_off[v0] = (uint16_t)off;
+    if (v1 < nvox) s_off[v1] = (uint16_t)(off + c0);
+    if (c0) atomicAdd(&s_place[min(c0, 63u)], 1u);
+    if (c1) atomicAdd(&s_place[min(c1, 63u)], 1u);
+    __syncthreads();
+    for (uint32_t f = tid; f < nf; f += kBrickThreads) {
+      const uint32_t lv = R.vox[f];
+      R.idx[s_off[lv] + atomicSub(&s_cnt[lv], 1u) - 1u] = (uint16_t)f;
+    }
+    // voxels with fragments, most first: a wave's lanes then replay voxels of
+    // like length, and voxels without fragments take no lanes
+    if (wave == 0) {
+      const uint32_t c = s_place[63 - lane];
+      uint32_t y = c;
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t z = __shfl_up(y, o, 64);
+        if (lane >= o) y += z;
+      }
+      s_place[63 - lane] = y - c;
+      if (lane == 63) s_nfrag = y;  // voxels with fragments (count 0 was not counted)
+    }
+    __syncthreads();
+    if (c0) s_ord[atomicAdd(&s_place[min(c0, 63u)], 1u)] = (uint16_t)v0;
+    if (c1) s_ord[atomicAdd(&s_place[min(c1, 63u)], 1u)] = (uint16_t)v1;
+    __syncthreads();
+    // ---- each voxel's fragments in order, through the recurrence -------------------
+    const uint32_t nused = s_nfrag;
+    for (uint32_t k = tid; k < nused; k += kBrickThreads) {
+      const uint32_t v = s_ord[k], beg = s_off[v], end = v + 1u < nvox ? s_off[v + 1u] : nf;
+      for (uint32_t a = beg + 1u; a < end; ++a) {  // insertion sort by key
+        const uint16_t f = R.idx[a];
+        const uint32_t kf = R.key[f];
+        uint32_t b = a;
+        while (b > beg) {
+          const uint16_t p = R.idx[b - 1u];
+          if (R.key[p] <= kf) break;
+          R.idx[b] = p;
+          --b;
+        }
+        R.idx[b] = f;
+      }
+      uint32_t st = s_state[v];
+      for (uint32_t a = beg; a < end; ++a) {
+        const uint32_t f = R.idx[a];
+        const float al = fminf(fmaxf(s_alpha[R.key[f] >> 8], 0.0f), 1.0f);
+        st = replay_step(st, R.col[0][f] * 255.0f, R.col[1][f] * 255.0f, R.col[2][f] * 255.0f, al * 255.0f);
+      }
+      s_state[v] = st;
+    }
+    nall += nf;
+    pos += m;
+    take = kBrickItems;
+    __syncthreads();
+  }
+  __syncthreads();
+  for (uint32_t v = tid; v < nvox; v += kBrickThreads) level0[brick * nvox + v] = s_state[v];
+  if (tid == 0) brick_frags[brick] = nall;
 }
 
 __global__ void zero_u32_kernel(uint32_t* p, uint64_t n) {
@@ -1139,13 +1339,11 @@ static int launch_list(vct_context* ctx, uint32_t ntri, const uint32_t* off, uin
   return VCT_OK;
 }
 
-template <int DT, int kMode = kExactMean>
-static void launch_brick(vct_context* ctx, uint32_t nbricks, uint32_t ntri, const VoxParams& vp,
-                         const uint32_t* count, const uint32_t* off, const uint32_t* list, void* level0,
-                         const RefPass& r = RefPass{}, ListCap lc = ListCap{nullptr, 0u, 0xffffffffu}) {
-  hipLaunchKernelGGL((vox_brick_kernel<DT, kMode>), dim3(nbricks), dim3(kBrickThreads), 0, ctx->stream, vp,
-                     (const TriRec*)ctx->setup.p, (const VoxShade*)ctx->vox_shade.p, count, off, list, lc, level0,
-                     r);
+template <int DT>
+static void launch_brick(vct_context* ctx, uint32_t nbricks, const VoxParams& vp, const uint32_t* count,
+                         const uint32_t* off, const uint32_t* list, void* level0, ListCap lc) {
+  hipLaunchKernelGGL(vox_brick_kernel<DT>, dim3(nbricks), dim3(kBrickThreads), 0, ctx->stream, vp,
+                     (const TriRec*)ctx->setup.p, (const VoxShade*)ctx->vox_shade.p, count, off, list, lc, level0);
 }
 
 // Exact mean: all queued draws in one batch (brick lists span every draw).
@@ -1175,10 +1373,10 @@ static int voxelize_exact(vct_context* ctx, const std::vector<uint32_t>& q, cons
   const uint32_t ntri = b.ntri;
   auto bricks = [&](const uint32_t* list, ListCap lc) {
     switch (ctx->dtype) {
-      case VCT_RGBA8: launch_brick<VCT_RGBA8>(ctx, nbricks, ntri, vp, bcount, boff, list, level0, RefPass{}, lc); break;
-      case VCT_FP16: launch_brick<VCT_FP16>(ctx, nbricks, ntri, vp, bcount, boff, list, level0, RefPass{}, lc); break;
-      case VCT_BF16: launch_brick<VCT_BF16>(ctx, nbricks, ntri, vp, bcount, boff, list, level0, RefPass{}, lc); break;
-      default: launch_brick<VCT_FP32>(ctx, nbricks, ntri, vp, bcount, boff, list, level0, RefPass{}, lc); break;
+      case VCT_RGBA8: launch_brick<VCT_RGBA8>(ctx, nbricks, vp, bcount, boff, list, level0, lc); break;
+      case VCT_FP16: launch_brick<VCT_FP16>(ctx, nbricks, vp, bcount, boff, list, level0, lc); break;
+      case VCT_BF16: launch_brick<VCT_BF16>(ctx, nbricks, vp, bcount, boff, list, level0, lc); break;
+      default: launch_brick<VCT_FP32>(ctx, nbricks, vp, bcount, boff, list, level0, lc); break;
     }
   };
   if (phase & 1) {
@@ -1246,88 +1444,65 @@ static int voxelize_exact(vct_context* ctx, const std::vector<uint32_t>& q, cons
   return VCT_OK;
 }
 
-// Brick lists of the queued draws for the reference running average:
-// records, per-brick triangle counts (bcount), offsets (boff) and lists
-// (tri_off).  Returns the number of (triangle, brick) pairs in `pairs`.
-static int ref_lists(vct_context* ctx, const std::vector<uint32_t>& q, const DrawTable& b, const VoxParams& vp,
-                     uint32_t nbricks, uint32_t& pairs) {
-  uint32_t* counters = (uint32_t*)ctx->counters.p;
-  uint32_t* bcount = (uint32_t*)ctx->tri_count.p;
-  uint32_t* cursor = bcount + nbricks;
-  uint32_t* boff = (uint32_t*)ctx->tri_base.p;
-  const uint32_t ntri = b.ntri;
-  int rc;
-  pairs = 0;
-  if ((rc = vct_ensure(ctx->setup, setup_bytes(ntri), ctx))) return rc;
-  if ((rc = vct_ensure(ctx->tri_off, 16, ctx))) return rc;
-  hipLaunchKernelGGL(zero_u32_kernel, dim3((2 * nbricks + 255) / 256), dim3(256), 0, ctx->stream, bcount,
-                     (uint64_t)2 * nbricks);
-  VCT_HIP(hipGetLastError());
-  if (!ntri) return VCT_OK;
-  if ((rc = vct_ensure(ctx->vox_box, (size_t)ntri * 8, ctx))) return rc;
-  if ((rc = launch_setup(ctx, q, b, vp, bcount))) return rc;
-  if ((rc = vct_launch_scan_u32(ctx, bcount, boff, nbricks, counters + 2))) return rc;
-  VCT_HIP(hipMemcpyAsync(ctx->h_readback + 2, counters + 2, 4, hipMemcpyDeviceToHost, ctx->stream));
-  VCT_HIP(hipStreamSynchronize(ctx->stream));
-  pairs = ctx->h_readback[2];
-  if (!pairs) return VCT_OK;
-  if ((rc = vct_ensure(ctx->tri_off, (size_t)pairs * 4 + (size_t)pairs / 4 * 4, ctx))) return rc;
-  return launch_list(ctx, ntri, boff, cursor, pairs);
-}
-
-// Reference running average: the brick pipeline of the exact mean finds the
-// same fragments (each covered pixel of a triangle once, in the brick of its
-// voxel).  A count pass writes the fragments of every voxel, a scan gives
-// every voxel its slots, a place pass stores (canonical key, colour) in them,
-// and the replay sorts each voxel's slots and runs the RGBA8 recurrence.
-static int voxelize_reference(vct_context* ctx, const std::vector<uint32_t>& q, const VoxParams& vp, void* level0) {
+// Reference running average: the exact mean's records and brick lists, then
+// one pass that takes every brick's triangles in order (vox_ref_kernel).
+// Phase 1 launches up to the copy of the (triangle, brick) pair count to
+// pinned host memory, phase 2 waits for that copy, sizes the lists (and the
+// sort's second buffer) and launches the rest.
+static int voxelize_reference(vct_context* ctx, const std::vector<uint32_t>& q, const VoxParams& vp, void* level0,
+                              int phase) {
   const uint32_t res = ctx->res;
-  const uint64_t nvox = (uint64_t)res * res * res;
   const uint32_t edge = res < (uint32_t)kBrick ? res : (uint32_t)kBrick;
   const uint32_t per = res / edge;
   const uint32_t nbricks = per * per * per;
-  uint32_t* counters = (uint32_t*)ctx->counters.p;  // [1] fragments, [2] scan totals
+  uint32_t* counters = (uint32_t*)ctx->counters.p;  // [2] pairs
   int rc;
-  if ((rc = vct_ensure(ctx->vox_count, nvox * 4, ctx))) return rc;
-  if ((rc = vct_ensure(ctx->vox_off, nvox * 4, ctx))) return rc;
-  // per-brick counts + cursors, per-brick offsets
+  // per-brick counts + cursors (the cursors hold the fragment counts at the end), offsets
   if ((rc = vct_ensure(ctx->tri_count, (size_t)nbricks * 8 + 16, ctx))) return rc;
   if ((rc = vct_ensure(ctx->tri_base, (size_t)nbricks * 4 + 16, ctx))) return rc;
-  uint32_t* vcount = (uint32_t*)ctx->vox_count.p;
-  const uint32_t* bcount = (const uint32_t*)ctx->tri_count.p;
-  const uint32_t* boff = (const uint32_t*)ctx->tri_base.p;
+  uint32_t* bcount = (uint32_t*)ctx->tri_count.p;
+  uint32_t* cursor = bcount + nbricks;
+  uint32_t* boff = (uint32_t*)ctx->tri_base.p;
   DrawTable b;
-  if ((rc = fill_draws(ctx, q, b))) return rc;
-  uint32_t pairs = 0;
-  if ((rc = ref_lists(ctx, q, b, vp, nbricks, pairs))) return rc;
-  ctx->last_candidates += pairs;
-  RefPass r;
-  memset(&r, 0, sizeof(r));
-  r.vcount = vcount;
-  // every brick's workgroup writes its voxels' counts, zeros included
-  launch_brick<VCT_RGBA8, kRefCount>(ctx, nbricks, b.ntri, vp, bcount, boff, (const uint32_t*)ctx->tri_off.p, nullptr,
-                                     r);
-  VCT_HIP(hipGetLastError());
-  if ((rc = vct_launch_scan_u32(ctx, vcount, (uint32_t*)ctx->vox_off.p, (uint32_t)nvox, counters + 1))) return rc;
-  VCT_HIP(hipMemcpyAsync(ctx->h_readback + 2, counters + 1, 4, hipMemcpyDeviceToHost, ctx->stream));
-  VCT_HIP(hipStreamSynchronize(ctx->stream));
-  const uint32_t nfrag = ctx->h_readback[2];
-  ctx->last_fragments = nfrag;
-  if (!nfrag) {
+  if ((rc = fill_draws(ctx, q, b, (phase & 1) != 0))) return rc;
+  const uint32_t ntri = b.ntri;
+  if (phase & 1) {
+    hipLaunchKernelGGL(zero_u32_kernel, dim3((2 * nbricks + 255) / 256), dim3(256), 0, ctx->stream, bcount,
+                       (uint64_t)2 * nbricks);
+    VCT_HIP(hipGetLastError());
+    ctx->h_readback[2] = 0u;
+    if (ntri) {
+      if ((rc = vct_ensure(ctx->setup, setup_bytes(ntri), ctx))) return rc;
+      if ((rc = vct_ensure(ctx->vox_box, (size_t)ntri * 8, ctx))) return rc;
+      if ((rc = launch_setup(ctx, q, b, vp, bcount))) return rc;
+      if ((rc = vct_launch_scan_u32(ctx, bcount, boff, nbricks, counters + 2))) return rc;
+      VCT_HIP(hipMemcpyAsync(ctx->h_readback + 2, counters + 2, 4, hipMemcpyDeviceToHost, ctx->stream));
+    }
+    // also when nothing was counted: a copy an interrupted earlier frame left
+    // in flight must not land after the word is read
+    VCT_HIP(hipEventRecord(ctx->vox_total_ev, ctx->stream));
+    ctx->vox_total_pending = false;  // the event no longer stands for an exact-mean frame's count
+    ctx->vox_known_total = 0;
+  }
+  if (!(phase & 2)) return VCT_OK;
+  VCT_HIP(hipEventSynchronize(ctx->vox_total_ev));
+  const uint32_t pairs = ctx->h_readback[2];
+  ctx->last_candidates = pairs;
+  if (!pairs) {
+    const uint64_t nvox = (uint64_t)res * res * res;
     hipLaunchKernelGGL(zero_u32_kernel, dim3(2048), dim3(256), 0, ctx->stream, (uint32_t*)level0, nvox);
     VCT_HIP(hipGetLastError());
     return VCT_OK;
   }
-  const size_t ns = ((size_t)nfrag + 4) & ~(size_t)3;
-  if ((rc = vct_ensure(ctx->frags_sorted, ns * 24, ctx))) return rc;
-  r.vox_off = (const uint32_t*)ctx->vox_off.p;
-  r.s_cand = (unsigned long long*)ctx->frags_sorted.p;
-  r.s_color = (float4*)((char*)ctx->frags_sorted.p + ns * 8);
-  r.nfrag = nfrag;
-  r.nvox = (uint32_t)nvox;
-  launch_brick<VCT_RGBA8, kRefPlace>(ctx, nbricks, b.ntri, vp, bcount, boff, (const uint32_t*)ctx->tri_off.p, level0,
-                                     r);
+  const size_t seg = ((size_t)pairs + pairs / 4 + 3) & ~(size_t)3;
+  if ((rc = vct_ensure(ctx->tri_off, seg * 8, ctx))) return rc;
+  if ((rc = launch_list(ctx, ntri, boff, cursor, pairs))) return rc;
+  hipLaunchKernelGGL(vox_ref_kernel, dim3(nbricks), dim3(kBrickThreads), 0, ctx->stream, vp,
+                     (const TriRec*)ctx->setup.p, (const VoxShade*)ctx->vox_shade.p, (const uint32_t*)bcount,
+                     (const uint32_t*)boff, (uint32_t*)ctx->tri_off.p, (uint32_t*)ctx->tri_off.p + seg,
+                     (uint32_t*)level0, cursor);
   VCT_HIP(hipGetLastError());
+  ctx->vox_frag_bricks = nbricks;
   return VCT_OK;
 }
 
@@ -1363,7 +1538,8 @@ int vct_launch_voxelize_phase(vct_context* ctx, int phase) {
     ctx->last_candidates = 0;
     ctx->last_fragments = 0;
     ctx->vox_pairs_on_device = false;
+    ctx->vox_frag_bricks = 0;
   }
   if (ctx->average == VCT_AVG_EXACT) return voxelize_exact(ctx, q, vp, level0, phase);
-  return (phase & 2) ? voxelize_reference(ctx, q, vp, level0) : VCT_OK;
+  return voxelize_reference(ctx, q, vp, level0, phase);
 }
