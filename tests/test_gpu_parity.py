@@ -289,6 +289,22 @@ def test_gbuffer_bit_exact(gpu_available, orc, kind, ntri, W, H, extra):
     assert np.array_equal(bits(gn), bits(n32))
 
 
+@pytest.mark.parametrize("W,H", [(4096, 4096), (4128, 4096)])
+def test_gbuffer_tile_count_past_one_scan_workgroup(gpu_available, orc, W, H):
+    """16,384 tiles, the most whose counts one workgroup scans, and 16,512,
+    which take the three-launch scan."""
+    say(f"gbuffer parity at {W}x{H}")
+    sc = SceneSpec("soup", ntri=1500, W=W, H=H)
+    with Context(W, H) as ctx:
+        sc.build(ctx, L.RGBA8)
+        ctx.gbuffer()
+        gp, gn = ctx.download_gbuffer()
+    p32, n32, _, _, _ = orc.gbuffer(W, H, sc.view, sc.proj, [(sc.M, sc.pos, sc.nrm, sc.tri_mat)])
+    assert (p32[..., 3] != 0).any()
+    assert np.array_equal(bits(gp), bits(p32))
+    assert np.array_equal(bits(gn), bits(n32))
+
+
 def test_gbuffer_many_models(gpu_available, orc):
     """Any number of queued models (renderer.cpp:242-256): 37 draws, two of
     them with a model matrix, camera inside the soup (clipped triangles)."""

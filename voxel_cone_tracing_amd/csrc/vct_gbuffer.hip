@@ -1253,8 +1253,6 @@ int vct_launch_gbuffer_phase(vct_context* ctx, int phase) {
   int rc;
   if ((rc = vct_ensure(ctx->g_pos, npix * 16, ctx))) return rc;
   if ((rc = vct_ensure(ctx->g_nrm, npix * 16, ctx))) return rc;
-  if ((rc = vct_ensure(ctx->counters, 256, ctx))) return rc;
-  uint32_t* counters = (uint32_t*)ctx->counters.p;
 
   GParams p;
   memset(&p, 0, sizeof(p));
@@ -1292,42 +1290,43 @@ int vct_launch_gbuffer_phase(vct_context* ctx, int phase) {
   p.H = H;
   const int tiles_x = (W + kTile - 1) / kTile, tiles_y = (H + kTile - 1) / kTile;
   const uint32_t ntiles = (uint32_t)(tiles_x * tiles_y);
-  // [0, ntiles): counts, [ntiles, 2 ntiles): write cursors
+  // [0, ntiles): counts, [ntiles, 2 ntiles): write cursors, then the fan
+  // triangles and the clipped triangles (cleared with them)
   if ((rc = vct_ensure(ctx->g_count, (size_t)ntiles * 8 + 16, ctx))) return rc;
   if ((rc = vct_ensure(ctx->g_off, (size_t)ntiles * 4 + 16, ctx))) return rc;
   uint32_t* tile_count = (uint32_t*)ctx->g_count.p;
   uint32_t* cursor = tile_count + ntiles;
+  uint32_t* fan_total = cursor + ntiles;
+  uint32_t* clip_count = fan_total + 1;
   uint32_t* tile_off = (uint32_t*)ctx->g_off.p;
   const int lsh = vct_lanes_log2(p.ntri);
   if (phase & 1) {
-    hipLaunchKernelGGL(fill_u32_kernel, dim3((2 * ntiles + 255) / 256), dim3(256), 0, ctx->stream, tile_count,
-                       2 * ntiles, 0u);
+    hipLaunchKernelGGL(fill_u32_kernel, dim3((2 * ntiles + 2 + 255) / 256), dim3(256), 0, ctx->stream, tile_count,
+                       2 * ntiles + 2, 0u);
     VCT_HIP(hipGetLastError());
     ctx->h_readback[0] = 0u;
     ctx->h_readback[1] = 0u;
     if (ntri) {
       if ((rc = vct_ensure(ctx->g_recs, (size_t)ntri * sizeof(GRec), ctx))) return rc;
       if ((rc = vct_ensure(ctx->g_clip, (size_t)ntri * 4, ctx))) return rc;
-      hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, ctx->stream, counters + 5, 2u, 0u);
       hipLaunchKernelGGL(g_bin_count_kernel, dim3(vct_lane_blocks(p.ntri, lsh)), dim3(256), 0, ctx->stream, p,
-                         (GRec*)ctx->g_recs.p, tile_count, tiles_x, (uint32_t*)ctx->g_clip.p, counters + 6, lsh);
+                         (GRec*)ctx->g_recs.p, tile_count, tiles_x, (uint32_t*)ctx->g_clip.p, clip_count, lsh);
       hipLaunchKernelGGL(g_fan_count_kernel, dim3(kFanGrid), dim3(256), 0, ctx->stream, p, (GRec*)ctx->g_recs.p,
-                         (const uint32_t*)ctx->g_clip.p, (const uint32_t*)(counters + 6), tile_count, tiles_x,
-                         counters + 5);
+                         (const uint32_t*)ctx->g_clip.p, (const uint32_t*)clip_count, tile_count, tiles_x,
+                         fan_total);
       VCT_HIP(hipGetLastError());
-      if ((rc = vct_launch_scan_u32(ctx, tile_count, tile_off, ntiles, counters + 4, &ctx->g_scan_tmp))) return rc;
       // the list size and the number of fan triangles of clipped triangles
       // are known on the device only
-      VCT_HIP(hipMemcpyAsync(ctx->h_readback, counters + 4, 8, hipMemcpyDeviceToHost, ctx->stream));
+      if ((rc = vct_launch_scan_u32(ctx, tile_count, tile_off, ntiles, nullptr, &ctx->g_scan_tmp, ctx->h_readback,
+                                    fan_total)))
+        return rc;
     }
-    // also when nothing was counted: a copy an interrupted earlier frame left
-    // in flight must not land after the words are read
     VCT_HIP(hipEventRecord(ctx->g_count_ev, ctx->stream));
   }
   if (!(phase & 2)) return VCT_OK;
   VCT_HIP(hipEventSynchronize(ctx->g_count_ev));
-  const uint32_t total = ctx->h_readback[0];
-  const uint32_t nfans = ctx->h_readback[1];
+  const uint32_t total = ntri ? ctx->h_readback[0] : 0u;
+  const uint32_t nfans = ntri ? ctx->h_readback[1] : 0u;
   if ((rc = vct_ensure(ctx->g_fans, (size_t)nfans * (sizeof(GRec) + sizeof(GFan)) + 64, ctx))) return rc;
   GRec* fan_recs = (GRec*)ctx->g_fans.p;
   GFan* fans = (GFan*)((char*)ctx->g_fans.p + (size_t)nfans * sizeof(GRec));
@@ -1338,7 +1337,7 @@ int vct_launch_gbuffer_phase(vct_context* ctx, int phase) {
                        (uint32_t*)ctx->g_list.p, lsh);
     if (nfans)
       hipLaunchKernelGGL(g_fan_write_kernel, dim3(kFanGrid), dim3(256), 0, ctx->stream, p, (const GRec*)ctx->g_recs.p,
-                         (const uint32_t*)ctx->g_clip.p, (const uint32_t*)(counters + 6), (const uint32_t*)tile_off,
+                         (const uint32_t*)ctx->g_clip.p, (const uint32_t*)clip_count, (const uint32_t*)tile_off,
                          cursor, tiles_x, (uint32_t*)ctx->g_list.p, fan_recs, fans);
     VCT_HIP(hipGetLastError());
   } else {

@@ -194,10 +194,12 @@ struct VctBuf {
 
 // A per-frame table (the draws of a pass) copied to the device on a stream:
 // pinned host staging and the device copy.  The staging area is rewritten
-// only once the copy that last read it has completed (its event).
+// only once the copy that last read it has completed (its event), and a table
+// equal to the last one is not copied again.
 struct VctUpload {
   void* host = nullptr;
   size_t cap = 0;
+  size_t bytes = 0;  // of the table last copied (0: none)
   hipEvent_t ev = nullptr;
   VctBuf dev;
 };
@@ -207,9 +209,9 @@ struct vct_context {
   hipStream_t stream = nullptr;
   hipStream_t side = nullptr;          // second stream (default priority): the G-buffer beside voxelize + mip
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  // pinned host words the list sizes are copied into: [0] G-buffer
+  // pinned host words the scans write the list sizes to: [0] G-buffer
   // (triangle, tile) pairs, [1] G-buffer fan triangles of clipped triangles,
-  // [2] voxelize (triangle, brick) pairs
+  // [2] voxelize (triangle, brick) pairs, [3] the same, of a sized list
   uint32_t* h_readback = nullptr;
   int width = 0, height = 0;
   unsigned res = 128;
@@ -317,7 +319,7 @@ struct vct_context {
   float pass_ms[6] = {0, 0, 0, 0, 0, 0};
   bool ev_recorded[6] = {false, false, false, false, false, false};
   uint32_t time_mask = 0x3fu;  // passes timed with events (bit k: pass k; vct_set_pass_timing)
-  hipEvent_t g_count_ev = nullptr;    // the G-buffer's list sizes copied to h_readback[0..1]
+  hipEvent_t g_count_ev = nullptr;    // the G-buffer's list sizes are in h_readback[0..1]
 };
 
 // ---- internal helpers (vct_runtime.hip) ---------------------------------
@@ -368,8 +370,8 @@ int vct_frame_front(vct_context* ctx);   // voxelize + mip beside the G-buffer, 
 int vct_launch_voxelize(vct_context* ctx);
 int vct_launch_gbuffer(vct_context* ctx);
 // The two passes that size a triangle list on the device, in two phases:
-// phase 1 launches the work up to the list size and its copy to pinned host
-// memory, phase 2 waits for that copy and launches the rest (3 = both).  The
+// phase 1 launches the work up to the list size (written to pinned host
+// memory), phase 2 waits for it and launches the rest (3 = both).  The
 // frame front runs phase 1 of both passes before either waits.
 int vct_launch_voxelize_phase(vct_context* ctx, int phase);
 int vct_launch_gbuffer_phase(vct_context* ctx, int phase);
@@ -399,6 +401,7 @@ int vct_trace_select(vct_context* ctx, const float4* gpos, const float4* gnrm, f
 int vct_trace_into(vct_context* ctx, const float4* gpos, const float4* gnrm, float4* out, int W, int H,
                    int demodulate, unsigned long long* step_counter);
 int vct_launch_scan_u32(vct_context* ctx, const uint32_t* in, uint32_t* out, uint32_t n,
-                        uint32_t* total_dev, VctBuf* tmp = nullptr);
+                        uint32_t* total_dev, VctBuf* tmp = nullptr, uint32_t* host = nullptr,
+                        const uint32_t* extra = nullptr);
 int vct_tex3d_mip_launch(vct_context* ctx, VctTex3D& t);
 int vct_tex3d_clear_launch(vct_context* ctx, VctTex3D& t, const float rgba[4]);

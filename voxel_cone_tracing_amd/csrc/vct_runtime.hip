@@ -55,6 +55,9 @@ static void free_buf(VctBuf& b) {
 }
 
 int vct_upload(vct_context* ctx, VctUpload& u, const void* data, size_t bytes) {
+  // the same table as the last one (staging still holds it): the device copy stands
+  if (u.ev && bytes == u.bytes && u.dev.p && memcmp(u.host, data, bytes) == 0) return VCT_OK;
+  u.bytes = 0;
   if (!u.ev) VCT_HIP(hipEventCreateWithFlags(&u.ev, hipEventDisableTiming));
   else VCT_HIP(hipEventSynchronize(u.ev));  // the last copy out of the staging area has completed
   if (bytes > u.cap) {
@@ -70,6 +73,7 @@ int vct_upload(vct_context* ctx, VctUpload& u, const void* data, size_t bytes) {
   memcpy(u.host, data, bytes);
   VCT_HIP(hipMemcpyAsync(u.dev.p, u.host, bytes, hipMemcpyHostToDevice, ctx->stream));
   VCT_HIP(hipEventRecord(u.ev, ctx->stream));
+  u.bytes = bytes;
   return VCT_OK;
 }
 
@@ -83,6 +87,7 @@ void vct_upload_free(VctUpload& u) {
   u.ev = nullptr;
   u.host = nullptr;
   u.cap = 0;
+  u.bytes = 0;
 }
 
 // ---- scan (exclusive, u32) --------------------------------------------------
@@ -122,8 +127,25 @@ __global__ __launch_bounds__(256) void scan_reduce_kernel(const uint32_t* in, ui
   if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
+// Where a scan's sum goes: a device word, and a pinned host word (the host
+// reads it after an event behind the scan; no copy command of its own) with
+// another device word beside it.
+struct ScanTotal {
+  uint32_t* dev;
+  uint32_t* host;         // null: not wanted
+  const uint32_t* extra;  // null, or copied to host[1]
+  __device__ __forceinline__ void put(uint32_t total) const {
+    if (dev) *dev = total;
+    if (host) {
+      host[0] = total;
+      if (extra) host[1] = *extra;
+      __threadfence_system();
+    }
+  }
+};
+
 __global__ __launch_bounds__(256) void scan_apply_kernel(const uint32_t* in, uint32_t n, const uint32_t* block_off,
-                                                        uint32_t* out, uint32_t* total_out) {
+                                                        uint32_t* out, ScanTotal total_out) {
   __shared__ uint32_t sh[4];
   const uint32_t base = blockIdx.x * kScanBlock;
   uint32_t v[4];
@@ -141,19 +163,69 @@ __global__ __launch_bounds__(256) void scan_apply_kernel(const uint32_t* in, uin
     if (i < n) out[i] = run;
     run += v[k];
   }
-  if (total_out && blockIdx.x == gridDim.x - 1 && threadIdx.x == 255) *total_out = run;
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 255) total_out.put(run);
+}
+
+// The whole scan in one workgroup, each lane over its own run of up to 16
+// elements: one launch instead of three, whose gaps cost a small frame more
+// than the idle rest of the chip (Cornell box at 512x512, both scans: 10 us of
+// the frame; at 32,768 elements one workgroup is 7 us slower than three
+// launches).
+constexpr uint32_t kScanOne = 16384;
+
+__global__ __launch_bounds__(1024) void scan_one_kernel(const uint32_t* __restrict__ in, uint32_t n,
+                                                        uint32_t* __restrict__ out, ScanTotal total_out) {
+  __shared__ uint32_t sh[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t per = (n + 4095u) / 4096u * 4u;  // a multiple of 4: 16-byte loads and stores
+  const uint32_t beg = min(n, threadIdx.x * per), end = min(n, beg + per);
+  uint32_t s = 0;
+  uint32_t i = beg;
+  for (; i + 4 <= end; i += 4) {
+    const uint4 v = *reinterpret_cast<const uint4*>(in + i);
+    s += v.x + v.y + v.z + v.w;
+  }
+  for (; i < end; ++i) s += in[i];
+  uint32_t x = s;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(x, o, 64);
+    if (lane >= o) x += y;
+  }
+  if (lane == 63) sh[wave] = x;
+  __syncthreads();
+  uint32_t run = x - s;
+  for (int w = 0; w < wave; ++w) run += sh[w];
+  for (i = beg; i + 4 <= end; i += 4) {
+    const uint4 v = *reinterpret_cast<const uint4*>(in + i);
+    uint4 o;
+    o.x = run;
+    o.y = o.x + v.x;
+    o.z = o.y + v.y;
+    o.w = o.z + v.z;
+    run = o.w + v.w;
+    *reinterpret_cast<uint4*>(out + i) = o;
+  }
+  for (; i < end; ++i) {
+    out[i] = run;
+    run += in[i];
+  }
+  if (threadIdx.x == 1023) total_out.put(run);
 }
 }  // namespace
 
-// Exclusive scan of n u32 values; *total_dev (device) receives the sum.
-// Scratch comes from *tmp, by default ctx->scan_tmp (scans that may run at
-// the same time on two streams need scratch of their own).  Sums must fit in
-// 32 bits.
+// Exclusive scan of n > 0 u32 values (in and out 16-byte aligned); *total_dev
+// (device) receives the sum, and *host (pinned, optional) as well, with *extra
+// (device, optional) in host[1].  Scratch comes from *tmp, by default
+// ctx->scan_tmp (scans that may run at the same time on two streams need
+// scratch of their own).  Sums must fit in 32 bits.
 int vct_launch_scan_u32(vct_context* ctx, const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* total_dev,
-                        VctBuf* tmp_buf) {
+                        VctBuf* tmp_buf, uint32_t* host, const uint32_t* extra) {
   VctBuf& scratch = tmp_buf ? *tmp_buf : ctx->scan_tmp;
-  if (n == 0) {
-    if (total_dev) VCT_HIP(hipMemsetAsync(total_dev, 0, 4, ctx->stream));
+  const ScanTotal total{total_dev, host, extra};
+  if (n <= kScanOne) {
+    hipLaunchKernelGGL(scan_one_kernel, dim3(1), dim3(1024), 0, ctx->stream, in, n, out, total);
+    VCT_HIP(hipGetLastError());
     return VCT_OK;
   }
   // level sizes
@@ -192,7 +264,7 @@ int vct_launch_scan_u32(vct_context* ctx, const uint32_t* in, uint32_t* out, uin
     const uint32_t* boff = (i + 1 < sizes.size()) ? offs[i + 1] : nullptr;
     uint32_t nb = (sizes[i] + kScanBlock - 1) / kScanBlock;
     hipLaunchKernelGGL(scan_apply_kernel, dim3(nb), dim3(256), 0, ctx->stream, src, sizes[i], boff, dst,
-                       i == 0 ? total_dev : nullptr);
+                       i == 0 ? total : ScanTotal{nullptr, nullptr, nullptr});
   }
   VCT_HIP(hipGetLastError());
   return VCT_OK;
@@ -292,12 +364,14 @@ static void identity(float* m) {
 // beside voxelize and mip on the context stream (they read the same geometry
 // and write disjoint buffers; each pass is timed on its own stream, so the
 // pass times overlap); the context stream then waits for the G-buffer.
-// Voxelize sizes its triangle list from earlier frames' counts and is
-// launched whole without a host wait (after the first frame, which reads its
-// count back); the G-buffer reads its list size and fan count back, the host
-// waiting on the copy's event.  Starting the G-buffer's raster only after
+// Voxelize's exact mean sizes its triangle list from earlier frames' counts
+// and is launched whole without a host wait (after the first frame, which
+// reads its count back); the reference average and the G-buffer read their
+// list sizes back, the host waiting on the event behind each scan.  Starting the G-buffer's raster only after
 // voxelize's brick kernel, beside the HBM-bound mip, measured slower: its
 // long workgroups take the slots the mip's 512-lane ones need.
+constexpr uint64_t kVoxelizeFirst = 1u << 19;  // triangles up to which voxelize is launched first
+
 int vct_frame_front(vct_context* ctx) {
   int rc;
   if ((rc = sync_materials(ctx))) return rc;
@@ -310,15 +384,32 @@ int vct_frame_front(vct_context* ctx) {
   };
   VCT_HIP(hipEventRecord(ctx->ev_fork, ctx->stream));
   VCT_HIP(hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0));
-  if ((rc = vct_pass_event(ctx, 2, false, ctx->side))) return rc;
-  if ((rc = on_side([ctx] { return vct_launch_gbuffer_phase(ctx, 1); }))) return rc;
   ++ctx->volume_version;
-  if ((rc = vct_pass_event(ctx, 0, false, ctx->stream))) return rc;
-  if ((rc = vct_launch_voxelize_phase(ctx, 1))) return rc;
-  if ((rc = on_side([ctx] { return vct_launch_gbuffer_phase(ctx, 2); }))) return rc;
-  if (ctx->front_lowres && (rc = on_side([ctx] { return vct_launch_lowres_gather(ctx); }))) return rc;
-  if ((rc = vct_pass_event(ctx, 2, true, ctx->side))) return rc;
-  if ((rc = vct_launch_voxelize_phase(ctx, 2))) return rc;
+  auto vox = [&](int phase) -> int {
+    if (phase == 1 && (rc = vct_pass_event(ctx, 0, false, ctx->stream))) return rc;
+    return vct_launch_voxelize_phase(ctx, phase);
+  };
+  auto gbuf = [&](int phase) -> int {
+    if (phase == 1 && (rc = vct_pass_event(ctx, 2, false, ctx->side))) return rc;
+    if ((rc = on_side([ctx, phase] { return vct_launch_gbuffer_phase(ctx, phase); }))) return rc;
+    if (phase == 1) return VCT_OK;
+    if (ctx->front_lowres && (rc = on_side([ctx] { return vct_launch_lowres_gather(ctx); }))) return rc;
+    return vct_pass_event(ctx, 2, true, ctx->side);
+  };
+  // The front of a frame of few triangles waits for its launches, and voxelize
+  // -> mip is its longer chain, so voxelize goes first; with many triangles
+  // the brick pass would then take the chip ahead of the raster, which ends
+  // beside the mip instead (frame with voxelize first: 34 triangles 434 ->
+  // 420 us, 300,000 1.93 -> 1.92 ms, 1,000,000 2.77 -> 2.79 ms and learned
+  // 2.77 -> 2.82).
+  uint64_t ntri = 0;
+  for (uint32_t id : ctx->queue)
+    if (id < ctx->models.size()) ntri += ctx->models[id].ntri;
+  if (ntri <= kVoxelizeFirst) {
+    if ((rc = vox(1)) || (rc = gbuf(1)) || (rc = vox(2)) || (rc = gbuf(2))) return rc;
+  } else {
+    if ((rc = gbuf(1)) || (rc = vox(1)) || (rc = gbuf(2)) || (rc = vox(2))) return rc;
+  }
   if ((rc = vct_pass_event(ctx, 0, true, ctx->stream))) return rc;
   VCT_HIP(hipEventRecord(ctx->ev_join, ctx->side));
   if ((rc = vct_mip_aniso(ctx))) return rc;

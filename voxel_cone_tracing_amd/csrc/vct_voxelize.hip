@@ -1352,8 +1352,8 @@ static void launch_brick(vct_context* ctx, uint32_t nbricks, const VoxParams& vp
 // (a brick whose range runs past it walks the triangles' boxes, so a frame
 // whose geometry grew is still exact), and this frame's count comes back
 // asynchronously for the next.  Otherwise (the first frame, or another
-// triangle count) phase 1 launches up to the copy of the count to pinned
-// host memory and phase 2 waits for it and launches the rest.
+// triangle count) phase 1 launches up to the scan that writes the count to
+// pinned host memory and phase 2 waits for it and launches the rest.
 static int voxelize_exact(vct_context* ctx, const std::vector<uint32_t>& q, const VoxParams& vp, void* level0,
                           int phase) {
   const uint32_t res = ctx->res;
@@ -1401,10 +1401,11 @@ static int voxelize_exact(vct_context* ctx, const std::vector<uint32_t>& q, cons
       if ((rc = vct_ensure(ctx->setup, setup_bytes(ntri), ctx))) return rc;
       if ((rc = vct_ensure(ctx->vox_box, (size_t)ntri * 8, ctx))) return rc;
       if ((rc = launch_setup(ctx, q, b, vp, bcount))) return rc;
-      if ((rc = vct_launch_scan_u32(ctx, bcount, boff, nbricks, counters + 2))) return rc;
-      if (!ctx->vox_sized) {
-        VCT_HIP(hipMemcpyAsync(ctx->h_readback + 2, counters + 2, 4, hipMemcpyDeviceToHost, ctx->stream));
-      } else {
+      if ((rc = vct_launch_scan_u32(ctx, bcount, boff, nbricks, counters + 2, nullptr,
+                                    ctx->h_readback + (ctx->vox_sized ? 3 : 2))))
+        return rc;
+      if (ctx->vox_sized) {
+        VCT_HIP(hipEventRecord(ctx->vox_total_ev, ctx->stream));
         // a quarter more than the last count, at least two pairs per triangle
         const uint64_t want = std::max<uint64_t>((uint64_t)ctx->vox_known_total + ctx->vox_known_total / 4,
                                                  2ull * ntri + 1024u);
@@ -1412,8 +1413,6 @@ static int voxelize_exact(vct_context* ctx, const std::vector<uint32_t>& q, cons
         if ((rc = vct_ensure(ctx->tri_off, (size_t)cap * 4, ctx))) return rc;
         ctx->vox_cap = cap;
         if ((rc = launch_list(ctx, ntri, boff, cursor, cap))) return rc;
-        VCT_HIP(hipMemcpyAsync(ctx->h_readback + 3, counters + 2, 4, hipMemcpyDeviceToHost, ctx->stream));
-        VCT_HIP(hipEventRecord(ctx->vox_total_ev, ctx->stream));
         ctx->vox_total_pending = true;
         ctx->vox_pairs_on_device = true;
         bricks((const uint32_t*)ctx->tri_off.p, ListCap{(const uint2*)ctx->vox_box.p, ntri, cap});
@@ -1422,10 +1421,8 @@ static int voxelize_exact(vct_context* ctx, const std::vector<uint32_t>& q, cons
     }
   }
   if (!(phase & 2) || ctx->vox_sized) return VCT_OK;
-  // also when nothing was counted: a copy an interrupted earlier frame left
-  // in flight must not land after the word is read
   VCT_HIP(hipStreamSynchronize(ctx->stream));
-  const uint32_t total = ctx->h_readback[2];
+  const uint32_t total = ntri ? ctx->h_readback[2] : 0u;
   if (total) {
     if ((rc = vct_ensure(ctx->tri_off, (size_t)total * 4 + (size_t)total / 4 * 4, ctx))) return rc;
     if ((rc = launch_list(ctx, ntri, boff, cursor, total))) return rc;
@@ -1446,9 +1443,9 @@ static int voxelize_exact(vct_context* ctx, const std::vector<uint32_t>& q, cons
 
 // Reference running average: the exact mean's records and brick lists, then
 // one pass that takes every brick's triangles in order (vox_ref_kernel).
-// Phase 1 launches up to the copy of the (triangle, brick) pair count to
-// pinned host memory, phase 2 waits for that copy, sizes the lists (and the
-// sort's second buffer) and launches the rest.
+// Phase 1 launches up to the scan that writes the (triangle, brick) pair count
+// to pinned host memory, phase 2 waits for it, sizes the lists (and the sort's
+// second buffer) and launches the rest.
 static int voxelize_reference(vct_context* ctx, const std::vector<uint32_t>& q, const VoxParams& vp, void* level0,
                               int phase) {
   const uint32_t res = ctx->res;
@@ -1475,18 +1472,16 @@ static int voxelize_reference(vct_context* ctx, const std::vector<uint32_t>& q, 
       if ((rc = vct_ensure(ctx->setup, setup_bytes(ntri), ctx))) return rc;
       if ((rc = vct_ensure(ctx->vox_box, (size_t)ntri * 8, ctx))) return rc;
       if ((rc = launch_setup(ctx, q, b, vp, bcount))) return rc;
-      if ((rc = vct_launch_scan_u32(ctx, bcount, boff, nbricks, counters + 2))) return rc;
-      VCT_HIP(hipMemcpyAsync(ctx->h_readback + 2, counters + 2, 4, hipMemcpyDeviceToHost, ctx->stream));
+      if ((rc = vct_launch_scan_u32(ctx, bcount, boff, nbricks, counters + 2, nullptr, ctx->h_readback + 2)))
+        return rc;
     }
-    // also when nothing was counted: a copy an interrupted earlier frame left
-    // in flight must not land after the word is read
     VCT_HIP(hipEventRecord(ctx->vox_total_ev, ctx->stream));
     ctx->vox_total_pending = false;  // the event no longer stands for an exact-mean frame's count
     ctx->vox_known_total = 0;
   }
   if (!(phase & 2)) return VCT_OK;
   VCT_HIP(hipEventSynchronize(ctx->vox_total_ev));
-  const uint32_t pairs = ctx->h_readback[2];
+  const uint32_t pairs = ntri ? ctx->h_readback[2] : 0u;
   ctx->last_candidates = pairs;
   if (!pairs) {
     const uint64_t nvox = (uint64_t)res * res * res;
