@@ -13,11 +13,11 @@
 //     1/256 pixel, pixel bounding box in 2x2 quads, a 128-byte record; each
 //     triangle is counted into the 8^3-voxel bricks its voxel box overlaps.
 //  2. exclusive scan of the brick counts, then per-brick triangle lists.
-//  3. one workgroup per brick: the pixels of its triangles' boxes inside the
-//     brick's footprint are spread over the lanes, coverage is tested with
-//     exact 64-bit edge functions (top-left rule) from records in LDS, and
-//     only fragments whose voxel lies in the brick are shaded, so every
-//     fragment is found exactly once.
+//  3. one workgroup per brick: the pixel rows of its triangles' boxes inside
+//     the brick's footprint are spread over the lanes, which queue the pixels
+//     of each row's span; those are tested with exact 64-bit edge functions
+//     (top-left rule) from records in LDS, and only fragments whose voxel lies
+//     in the brick are shaded, so every fragment is found exactly once.
 //  4a. exact mean (any storage): 16.16 fixed-point sums in LDS (exact, so
 //     order-independent); the workgroup writes its brick's texels once.
 //  4b. reference running average (RGBA8): the workgroup takes its brick's
@@ -675,12 +675,12 @@ __device__ __forceinline__ void store_mean(void* level0, uint32_t v, uint32_t cn
 }
 
 // 4. one workgroup per brick (each workgroup maps its index to one brick's
-//    Morton index, one to one).  The
-//    brick's triangles are taken 256 at a time; the pixels of their boxes
-//    inside the brick's footprint on the projection plane are spread over the
-//    lanes (a lane finds its triangle by a binary search over the prefix of
-//    the box sizes), coverage is tested from a compact copy of the records in
-//    LDS, and only covered pixels read the rest of the record.
+//    Morton index, one to one).  The brick's triangles are taken kBrickItems
+//    at a time; the pixel rows of their boxes inside the brick's footprint on
+//    the projection plane are spread over the lanes (a lane finds its triangle
+//    from the prefix of the row counts), the pixels of the rows' spans are
+//    tested from a compact copy of the records in LDS, and only covered pixels
+//    read the rest of the record.
 struct CovRec {  // the coverage fields of a TriRec
   int64_t area;
   int32_t X[3], Y[3];
@@ -750,15 +750,14 @@ struct ListCap {
 // A round of up to kBrickItems triangles of a brick, in LDS.
 struct BrickRound {
   CovRec cov[kBrickItems];
-  uint32_t end[kBrickItems];  // inclusive prefix of candidate counts
-  uint32_t org[kBrickItems];  // clipped box origin: i | j << 16
-  uint32_t div[kBrickItems];  // ceil(65536 / width) | width << 20
+  uint32_t end[kBrickItems];  // inclusive prefix of the row counts
+  uint32_t org[kBrickItems];  // clipped box: i | j << 11 | width << 22 (width at most 16)
   uint32_t wsum[kBrickItems / 64];
-  uint32_t q[kBrickThreads / 64][128];  // per-wave queue of covered candidates
+  uint32_t q[kBrickThreads / 64][128];  // per-wave queue of pixels inside the spans
 };
 
 // Stages triangle t as entry `slot` of the round for the brick at bc (bricks);
-// returns its candidate pixels: its box clipped to the brick's footprint.  A
+// returns its rows: those of its box clipped to the brick's footprint.  A
 // covered pixel (i, j) lands in voxel (i >> 1, j >> 1) on the projection
 // plane: its centre sits a quarter voxel inside that voxel, and the
 // interpolated position is a convex combination of the vertices that differs
@@ -776,9 +775,7 @@ __device__ __forceinline__ uint32_t brick_stage(BrickRound& B, int slot, uint32_
   const int i0 = max(qx0, fx), i1 = min(min(qx0 + 2 * qw - 1, fx + span - 1), lim);
   const int j0 = max(qy0, fy), j1 = min(min(qy0 + 2 * qh - 1, fy + span - 1), lim);
   if (i1 < i0 || j1 < j0) return 0u;
-  const uint32_t cw = (uint32_t)(i1 - i0 + 1);
-  B.org[slot] = (uint32_t)i0 | ((uint32_t)j0 << 16);
-  B.div[slot] = ((65536u + cw - 1u) / cw) | (cw << 20);
+  B.org[slot] = (uint32_t)i0 | ((uint32_t)j0 << 11) | ((uint32_t)(i1 - i0 + 1) << 22);
   CovRec cr;
   cr.area = rp->area;
   for (int v = 0; v < 3; ++v) {
@@ -788,10 +785,10 @@ __device__ __forceinline__ uint32_t brick_stage(BrickRound& B, int slot, uint32_
   cr.flags = fl;
   cr.tri = t;
   B.cov[slot] = cr;
-  return cw * (uint32_t)(j1 - j0 + 1);
+  return (uint32_t)(j1 - j0 + 1);
 }
 
-// Prefix of the entries' candidate counts (cnt of thread tid < kBrickItems);
+// Prefix of the entries' row counts (cnt of thread tid < kBrickItems);
 // every thread of the workgroup calls it; returns the total.
 __device__ __forceinline__ uint32_t brick_prefix(BrickRound& B, uint32_t cnt) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -812,33 +809,54 @@ __device__ __forceinline__ uint32_t brick_prefix(BrickRound& B, uint32_t cnt) {
   return B.end[kBrickItems - 1];
 }
 
-// The round's candidates in two phases.  1: the wave's 64 candidates are
-// tested for coverage only (exact edge functions, top-left rule); the covered
-// ones are appended to the wave's queue in LDS.  2: whenever the queue holds
-// 64, every lane takes one (entry | i << 8 | j << 19) and runs the exact
-// fragment path (voxel address, brick test, shading, accumulation), so the
-// expensive part runs with all lanes busy instead of on the covered ~40 % of
-// them.  The set of fragments, and every value computed for one, is the same
-// as testing each candidate in full.  `fragment` is called by whole waves:
-// fragment(d, on).
+// Narrows [lo, hi] to the columns k where w - 256 ey k >= 0 may hold.  The
+// crossing t = w / (256 ey) is bounded in float with a margin of 1e-3 pixel
+// plus 2^-19 |t| (far above the rounding of the conversions, the reciprocal
+// and the product), so it never drops a pixel the exact test would keep.
+__device__ __forceinline__ void vox_span(int64_t w, int32_t ey, int& lo, int& hi) {
+  if (ey == 0) {
+    if (w < 0) hi = lo - 1;  // the whole row is outside this edge
+    return;
+  }
+  float t = (float)w * __builtin_amdgcn_rcpf(256.0f * (float)ey);
+  t = fminf(fmaxf(t, -4096.0f), 4096.0f);
+  const float m = 1e-3f + fabsf(t) * 1.9073486e-6f;
+  if (ey < 0) lo = max(lo, (int)ceilf(t - m));
+  else hi = min(hi, (int)floorf(t + m));
+}
+
+// The round's pixels in two phases.  1: the rows of the triangles' boxes are
+// dealt over the lanes; each lane bounds the span of its row inside the three
+// edges, and the pixels of the spans are appended to the wave's queue in LDS.  2: whenever the queue
+// holds 64, every lane takes one (entry | i << 8 | j << 19) and runs the exact
+// fragment path (coverage, voxel address, brick test, shading, accumulation),
+// so the expensive part runs with all lanes busy.  The set of fragments, and
+// every value computed for one, is the same as testing each pixel of the boxes
+// in full.  `fragment` is called by whole waves: fragment(d, on).
+//
+// Testing every pixel of the boxes, one per lane with its own three 64-bit
+// edge functions, cost a pixel inside or outside the triangle the same; a row
+// pays for its edges once and its pixels one queue entry each.  The voxelize
+// pass of the 10M-triangle soup at 512^3 4.85 -> 4.08 ms, of the 1M-triangle
+// one at 256^3 0.40 -> 0.37; a walk that also tests each pixel of the span
+// exactly needs spills: 4.34 and 0.40.
 template <class Frag>
 __device__ __forceinline__ void brick_scan(BrickRound& B, uint32_t total, Frag&& fragment) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t* s_end = B.end;
   uint32_t* q = B.q[wave];
   uint32_t qn = 0;    // entries in the queue (the same in every lane)
-  uint32_t own0 = 0;  // the entry of the wave's first candidate (the same in every lane; never decreases)
+  uint32_t own0 = 0;  // the entry of the wave's first row (the same in every lane; never decreases)
   for (uint32_t cb = (uint32_t)wave * 64u; cb < total; cb += kBrickThreads) {
     const uint32_t c = cb + (uint32_t)lane;
-    // The entry (triangle) of each lane's candidate, for the window
-    // [cb, cb + 64) of consecutive candidates.  own0 moves to the first
-    // entry ending after cb: lane k tests entry own0 + k and the ballot
-    // counts those ending at or before cb (a prefix, the ends being
-    // sorted).  Lane k then holds the end of entry own0 + k, and each lane
-    // finds how many of these end at or before its candidate by a binary
-    // search over the lanes (register shuffles): that count from own0 is
-    // its entry.  A window that spans more than 64 entries (entries with
-    // one candidate or none) finishes with a per-lane walk.
+    // The entry (triangle) of each lane's row, for the window [cb, cb + 64) of
+    // consecutive rows.  own0 moves to the first entry ending after cb: lane k
+    // tests entry own0 + k and the ballot counts those ending at or before cb
+    // (a prefix, the ends being sorted).  Lane k then holds the end of entry
+    // own0 + k, and each lane finds how many of these end at or before its row
+    // by a binary search over the lanes (register shuffles): that count from
+    // own0 is its entry.  A window that spans more than 64 entries (entries
+    // with one row or none) finishes with a per-lane walk.
     for (;;) {
       const uint32_t ek = own0 + (uint32_t)lane < kBrickItems ? s_end[own0 + lane] : 0xffffffffu;
       const uint32_t k = (uint32_t)__popcll(__ballot(ek <= cb));
@@ -846,10 +864,9 @@ __device__ __forceinline__ void brick_scan(BrickRound& B, uint32_t total, Frag&&
       if (k < 64u) break;
     }
     const uint32_t ek = own0 + (uint32_t)lane < kBrickItems ? s_end[own0 + lane] : 0xffffffffu;
-    // Only entries ending inside the window can end at or before a
-    // candidate: nend of them, the first nend lanes (the ends are sorted).  A
-    // window usually spans a few entries, and a scan of their ends read
-    // into scalar registers has no LDS round trip in its chain, where the
+    // Only entries ending inside the window can end at or before a row: nend
+    // of them, the first nend lanes (the ends are sorted).  A scan of few ends
+    // read into scalar registers has no LDS round trip in its chain, where the
     // binary search takes seven dependent shuffles; the count is the same.
     const uint32_t nend = (uint32_t)__popcll(__ballot(ek < cb + 64u));
     uint32_t past = 0;
@@ -860,30 +877,36 @@ __device__ __forceinline__ void brick_scan(BrickRound& B, uint32_t total, Frag&&
         if ((uint32_t)__shfl(ek, (int)(past + st - 1u), 64) <= c) past += st;
       if ((uint32_t)__shfl(ek, (int)past, 64) <= c) ++past;
     }
-    bool hit = false;
+    int len = 0;
     uint32_t desc = 0;
     if (c < total) {
       uint32_t lo = own0 + past;
       if (past == 64u)
         while (s_end[lo] <= c) ++lo;
-      const uint32_t local = c - (lo ? s_end[lo - 1] : 0u);
-      const uint32_t dv = B.div[lo], cw = dv >> 20;
-      const uint32_t row = (local * (dv & 0xfffffu)) >> 16;  // exact: local < 35 * 35, cw <= 35
-      const uint32_t col = local - row * cw;
+      const uint32_t row = c - (lo ? s_end[lo - 1] : 0u);
       const uint32_t org = B.org[lo];
-      const int i = (int)(org & 0xffffu) + (int)col, j = (int)(org >> 16) + (int)row;
+      const int i = (int)(org & 0x7ffu), j = (int)((org >> 11) & 0x7ffu) + (int)row;
       const CovRec cr = B.cov[lo];
       VEdges e;
       vox_edges(cr, i, j, e);
-      hit = vox_covers(e);
-      desc = lo | ((uint32_t)i << 8) | ((uint32_t)j << 19);
+      int k0 = 0, k1 = (int)(org >> 22) - 1;
+      vox_span(e.w[0], (int32_t)e.ey[0], k0, k1);
+      vox_span(e.w[1], (int32_t)e.ey[1], k0, k1);
+      vox_span(e.w[2], (int32_t)e.ey[2], k0, k1);
+      len = k1 - k0 + 1;
+      desc = lo | ((uint32_t)(i + k0) << 8) | ((uint32_t)j << 19);
     }
-    const unsigned long long m = __ballot(hit);
-    if (hit) q[qn + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = desc;
-    qn += (uint32_t)__popcll(m);
-    if (qn >= 64u) {
-      qn -= 64u;
-      fragment(q[qn + (uint32_t)lane], true);
+    // the wave walks its longest span; each lane stops at the end of its own span
+    for (int k = 0;; ++k) {
+      const bool hit = k < len;
+      const unsigned long long m = __ballot(hit);
+      if (m == 0ull) break;
+      if (hit) q[qn + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = desc + ((uint32_t)k << 8);
+      qn += (uint32_t)__popcll(m);
+      if (qn >= 64u) {
+        qn -= 64u;
+        fragment(q[qn + (uint32_t)lane], true);
+      }
     }
   }
   if (qn) {
@@ -901,9 +924,10 @@ __device__ __forceinline__ uint32_t brick_of_block() {
   return b < full ? (b & 7u) * (full >> 3) + (b >> 3) : b;
 }
 
-// Exact mean: sums the brick's fragments and writes its texels.  Its phases
-// wait on LDS and L2 more than they compute (fewer VALU instructions per
-// fragment or candidate measured no faster; more waves did), so it runs at 8
+// Exact mean: sums the brick's fragments and writes its texels.  On grids of
+// many small bricks' worth of fragments the vector ALUs bound it (10M triangles
+// at 512^3: 2.3 G wave instructions in 3.55 ms, about all the issue slots), on
+// smaller ones the waits on LDS and L2 between its phases do, so it runs at 8
 // waves per SIMD: 64 registers, no spills, and LDS for 8 workgroups per CU.
 template <int DT>
 __global__ __launch_bounds__(kBrickThreads) __attribute__((amdgpu_waves_per_eu(8))) void vox_brick_kernel(
