@@ -712,3 +712,75 @@ def test_sampler_at_the_volume_faces(gpu_available, orc, dtype, view_dir, lod):
     say(f"  max-abs vs FP32 oracle = {err:.3e}")
     # 16-bit pairs blend with weights rounded to the storage type (2^-11 / 2^-8)
     assert err <= {L.RGBA8: 1e-5, L.FP16: 2e-3, L.BF16: 1.6e-2, L.FP32: 1e-5}[dtype]
+
+
+@pytest.mark.parametrize("dtype", [L.RGBA8, L.FP16, L.BF16, L.FP32])
+@pytest.mark.parametrize("res,levels,lod", [(8, 4, 3.0), (8, 4, 2.5), (4, 3, 1.3), (4, 1, 0.0), (4, 2, 7.0)])
+def test_sampler_far_past_the_faces(gpu_available, orc, dtype, res, levels, lod):
+    """One sample per pixel at points from 1.5 texels of the coarsest level
+    before the cube to as far behind it, in levels down to a single texel: the
+    two texels an axis reads are clamped into the level, so the weights alone
+    have to make the border zero, on both sides and in the level of one texel
+    (where the second texel has no place at all)."""
+    say(f"sampler past faces dtype={dtype} res={res} levels={levels} lod={lod}")
+    W, H = 64, 48
+    sc = SceneSpec("cornell", res=res, W=W, H=H)
+    rng = np.random.default_rng(7 + dtype)
+    far = 1.5 * 2.0 ** (levels - 1) / res
+    with Context(W, H) as ctx:
+        sc.build(ctx, dtype, levels=levels)
+        maps = {}
+        for lvl in range(levels):
+            s = res >> lvl
+            for d in range(1 if lvl == 0 else 6):
+                enc = encode_level(rng.random((s, s, s, 4)).astype(np.float32), dtype)
+                ctx.upload_level(lvl, d, enc)
+                maps[(lvl, d)] = decode_level(enc, dtype)
+        b = rng.uniform(-far, 1.0 + far, (H, W, 3)).astype(np.float32)
+        b[: H // 2] = np.clip(b[: H // 2], 0.01, 0.99)  # half of them inside
+        b[0, :, 1] = 1.0 + 0.25 * far
+        b[1, :, 2] = -0.25 * far
+        world = (b - 0.5) * 2.0 * sc.cube_size
+        gp = np.concatenate([world, np.ones((H, W, 1), np.float32)], -1).astype(np.float32)
+        gn = np.zeros((H, W, 4), np.float32)
+        gn[..., 1] = 1.0
+        gn[..., 3] = np.uint32(1).view(np.float32)
+        ctx.upload_gbuffer(gp, gn)
+        ctx.set_voxel_view(3, lod)
+        ctx.trace()
+        img = ctx.download_image()
+    mips = {k: v for k, v in maps.items() if k[0] > 0}
+    want, _ = orc.trace(np.float32, res, levels, maps[(0, 0)], mips, gp, gn, sc.mat_records, sc.lights, sc.cam,
+                        sc.cube_size, cone_set=sc.cone_set, phases=sc.phases, view_dir=3, view_lod=lod)
+    err = np.abs(img.reshape(-1, 4) - want).max()
+    say(f"  max-abs vs FP32 oracle = {err:.3e}")
+    # 16-bit pairs blend with weights rounded to the storage type (2^-11 / 2^-8)
+    assert err <= {L.RGBA8: 1e-5, L.FP16: 2e-3, L.BF16: 1.6e-2, L.FP32: 1e-5}[dtype]
+
+
+@pytest.mark.parametrize("dtype,res,levels", [(L.RGBA8, 32, 1), (L.FP32, 32, 2), (L.FP16, 64, 4), (L.RGBA8, 16, 5)])
+def test_cones_end_past_the_volume(gpu_available, orc, dtype, res, levels):
+    """Cones that leave the volume through every face, with mip chains cut
+    short (the coarsest texel sets how far out a cone still reads): the exit
+    distance changes no pixel, and the steps taken are those of the oracle's
+    loop that tests the position at every step."""
+    say(f"cone exits dtype={dtype} res={res} levels={levels}")
+    W, H = 96, 64
+    sc = SceneSpec("soup", res=res, ntri=20000, W=W, H=H)
+    with Context(W, H) as ctx:
+        sc.build(ctx, dtype, levels=levels)
+        ctx.render()
+        img = ctx.download_image()
+        steps = ctx.trace_steps()
+        gp, gn = ctx.download_gbuffer()
+        l0 = decode_level(ctx.download_level(0), dtype)
+        mips = {(l, d): decode_level(ctx.download_level(l, d), dtype) for l in range(1, levels) for d in range(6)}
+    want, (_, live) = orc.trace(np.float32, res, levels, l0, mips, gp, gn, sc.mat_records, sc.lights, sc.cam,
+                                sc.cube_size, cone_set=sc.cone_set, early_exit_steps=True)
+    cov = (gp[..., 3] != 0).reshape(-1)
+    assert cov.sum() > 500
+    err = np.abs(img.reshape(-1, 4)[cov, :3] - want[cov, :3]).max()
+    rel = abs(int(steps) - int(live)) / live
+    say(f"  {int(cov.sum())} pixels, max-abs vs FP32 oracle = {err:.3e}; steps GPU {steps}, oracle {live}")
+    assert err <= 2e-3
+    assert rel <= 1e-3
