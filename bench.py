@@ -141,7 +141,12 @@ def algorithmic(name, wl, bpe, steps, fb_tiles):
         wr = sum(6 * (wl.res >> l) ** 3 * bpe for l in range(1, wl.levels))
         if bpe == 16:
             return rd + wr, "B", "hbm", "each source level read once, every mip texel written once"
-        vol = wl.res ** 3 * bpe + wr  # the x-paired copy: the whole volume written twice over
+        vol = wl.res ** 3 * bpe + wr
+        if bpe == 4:  # the tiled copy: every element 8 bytes, every third column twice; a pass over the volume
+            return rd + wr + vol + vol * 8 // 3, "B", "hbm", (
+                "each source level read once, every mip texel written once; the volume read once more and its "
+                "tiled copy (8/3 of the volume) written")
+        # the x-paired copy: the whole volume written twice over
         return rd + wr + 2 * vol, "B", "hbm", ("each source level read once, every mip texel written once, and the "
                                                 "x-paired copy (2x the volume) written")
     if name == "gbuffer":

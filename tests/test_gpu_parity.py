@@ -715,7 +715,8 @@ def test_sampler_at_the_volume_faces(gpu_available, orc, dtype, view_dir, lod):
 
 
 @pytest.mark.parametrize("dtype", [L.RGBA8, L.FP16, L.BF16, L.FP32])
-@pytest.mark.parametrize("res,levels,lod", [(8, 4, 3.0), (8, 4, 2.5), (4, 3, 1.3), (4, 1, 0.0), (4, 2, 7.0)])
+@pytest.mark.parametrize("res,levels,lod", [(8, 4, 3.0), (8, 4, 2.5), (4, 3, 1.3), (4, 1, 0.0), (4, 2, 7.0),
+                                            (32, 6, 0.5), (128, 2, 0.4)])
 def test_sampler_far_past_the_faces(gpu_available, orc, dtype, res, levels, lod):
     """One sample per pixel at points from 1.5 texels of the coarsest level
     before the cube to as far behind it, in levels down to a single texel: the

@@ -90,13 +90,15 @@ VCT_HD uint32_t dtype_bytes(int dt) {
 
 // One entry of the marcher's x-paired copy: texel a and its +x neighbour b.
 // 16-bit storage pairs channel by channel (four words of (c(a), c(b))), so a
-// two-term dot product weights both x-corners of a channel at once; RGBA8
-// texels pair as two words.
+// two-term dot product weights both x-corners of a channel at once.
 VCT_HD uint4 pair_pack(uint2 a, uint2 b) {
   return make_uint4((a.x & 0xffffu) | (b.x << 16), (a.x >> 16) | (b.x & 0xffff0000u), (a.y & 0xffffu) | (b.y << 16),
                     (a.y >> 16) | (b.y & 0xffff0000u));
 }
-VCT_HD uint2 pair_pack(uint32_t a, uint32_t b) { return make_uint2(a, b); }
+
+// The span of the marcher's copy of a map (0: it reads the volume itself), in
+// sizes of the map: x-paired 16-bit texels 2, tiled RGBA8 texels 4.
+VCT_HD uint64_t vct_copy_factor(int dt) { return dt == VCT_FP32 ? 0u : (dt == VCT_RGBA8 ? 4u : 2u); }
 
 // Round-to-nearest-even float -> bf16 bits (NaN kept quiet).
 VCT_HD uint16_t f32_to_bf16(float f) {
@@ -239,7 +241,7 @@ struct vct_context {
   uint64_t lvl_off[16][6];  // byte offsets
   uint32_t lvl_size[16];
   uint64_t volume_version = 1;  // advanced by every write of the volume
-  // x-paired copy of the volume for the cone marcher (16-bit and RGBA8 storage)
+  // the cone marcher's copy of the volume (x-paired 16-bit, tiled RGBA8 storage)
   VctBuf pairs;
   uint64_t pair_off[16][6];
   uint64_t pairs_version = 0;  // volume_version the copy was built from
@@ -360,10 +362,11 @@ inline uint32_t vct_lane_blocks(uint32_t ntri, int lsh) { return (uint32_t)((((u
 
 // kernels launchers
 int vct_launch_mip(vct_context* ctx);
-int vct_ensure_pairs(vct_context* ctx);  // x-paired copy of the volume for the marcher
-// Offsets of the paired copy's maps (ctx->pair_off) and its buffer.
+int vct_ensure_pairs(vct_context* ctx);  // the marcher's copy of the volume
+// Offsets of the copy's maps (ctx->pair_off) and its buffer.
 int vct_pair_layout(vct_context* ctx);
-// The paired copy of levels first.. (the mip kernel writes levels 0 and 1).
+// The copy of levels first.. (the mip kernel writes 16-bit pairs of levels 0
+// and 1; RGBA8 has all of them copied).
 int vct_pairs_from(vct_context* ctx, int first);
 int vct_launch_voxel_view(vct_context* ctx);  // the voxel view blended in draw order (last G-buffer's lists)
 int vct_frame_front(vct_context* ctx);   // voxelize + mip beside the G-buffer, joined

@@ -121,7 +121,7 @@ struct MipArgs {
   uint32_t n_src;      // texels in the source level
   int nout;            // output levels produced by this launch (1..4)
   int shared_src;      // 1: one source for all six maps (level 0)
-  // level 0 -> 1 launch, paired storage: the marcher's x-paired copy of the
+  // level 0 -> 1 launch, 16-bit storage: the marcher's x-paired copy of the
   // source level and of the first output level per map (null: not written)
   void* pair0;
   void* pair1[6];
@@ -166,7 +166,7 @@ __global__ __launch_bounds__(kThreads) void mip_kernel(MipArgs a) {
   __shared__ T s2[6][64];
   __shared__ T s3[6][8];
   // x = 0 face of each source block (the paired copy, level 0 -> 1 launch)
-  __shared__ T s0[sizeof(T) < 16 ? 512 : 1][4];
+  __shared__ T s0[sizeof(T) == 8 ? 512 : 1][4];
 
   const int dir_lo = a.shared_src ? 0 : (int)blockIdx.y;
   const int ndir = a.shared_src ? 6 : 1;
@@ -187,7 +187,7 @@ __global__ __launch_bounds__(kThreads) void mip_kernel(MipArgs a) {
         reinterpret_cast<T*>(a.dst[0][d])[m] = e;
         s1[d][t] = e;
       }
-      if constexpr (sizeof(T) < 16) {
+      if constexpr (sizeof(T) == 8) {
         if (a.pair0) {  // the x = 0 face of this 2x2x2 block, for the -x neighbour's pairs
 #pragma unroll
           for (int k = 0; k < 4; ++k) s0[t][k] = raw[2 * k];
@@ -208,11 +208,11 @@ __global__ __launch_bounds__(kThreads) void mip_kernel(MipArgs a) {
   // the +x neighbours inside the cube come from the neighbouring lane through
   // LDS, those of the cube's last block column from the first block of the
   // next cube in x, loaded again (its output texels recomputed from it).
-  if constexpr (sizeof(T) < 16) {
+  if constexpr (sizeof(T) == 8) {
     if (a.pair0) {
       using PR = decltype(pair_pack(raw[0], raw[0]));
-      // 16-byte entries of whole waves go out through LDS (below)
-      const bool staged = sizeof(PR) == 16 && n1 >= 64u;
+      // entries of whole waves go out through LDS (below)
+      const bool staged = n1 >= 64u;
       PR e0[8];  // (y, z) = (k & 1, k >> 1): entries 2k (x = 0) and 2k + 1 (x = 1)
       __syncthreads();
       if (t < n1) {
@@ -312,8 +312,8 @@ __global__ __launch_bounds__(kThreads) void mip_kernel(MipArgs a) {
   }
 }
 
-// paired: the level 0 -> 1 launch also writes the x-paired copy of levels 0
-// and 1 (ctx->pair_off laid out beforehand).
+// paired (16-bit storage): the level 0 -> 1 launch also writes the x-paired
+// copy of levels 0 and 1 (ctx->pair_off laid out beforehand).
 template <int DT>
 int launch_chain(vct_context* ctx, bool paired) {
   const int L = ctx->levels;
@@ -353,15 +353,17 @@ int launch_chain(vct_context* ctx, bool paired) {
 }  // namespace
 }  // namespace vct
 
-// The mip chain, then the cone marcher's x-paired copy of the finished volume:
-// the first launch of the chain writes the copy of levels 0 and 1 from the
-// blocks it holds, a copy pass the rest (1/17 of the texels).
+// The mip chain, then the cone marcher's copy of the finished volume.  The
+// x-paired copy of 16-bit storage: the first launch of the chain writes levels
+// 0 and 1 from the blocks it holds, a copy pass the rest (1/17 of the texels).
+// The tiled copy of RGBA8 is a pass of its own over the volume: a line of it
+// draws on more blocks than a workgroup holds.
 int vct_launch_mip(vct_context* ctx) {
   int rc;
-  const bool paired = ctx->dtype != VCT_FP32 && ctx->levels >= 2;
+  const bool paired = (ctx->dtype == VCT_FP16 || ctx->dtype == VCT_BF16) && ctx->levels >= 2;
   if (paired && (rc = vct_pair_layout(ctx))) return rc;
   switch (ctx->dtype) {
-    case VCT_RGBA8: rc = vct::launch_chain<VCT_RGBA8>(ctx, paired); break;
+    case VCT_RGBA8: rc = vct::launch_chain<VCT_RGBA8>(ctx, false); break;
     case VCT_FP16: rc = vct::launch_chain<VCT_FP16>(ctx, paired); break;
     case VCT_BF16: rc = vct::launch_chain<VCT_BF16>(ctx, paired); break;
     case VCT_FP32: rc = vct::launch_chain<VCT_FP32>(ctx, false); break;

@@ -311,11 +311,11 @@ static int validate_grid(unsigned res, int levels, int dtype, int average) {
     return vct_set_error(VCT_ERR_INVALID_ARG, "bad averaging mode");
   if (average == VCT_AVG_REFERENCE && dtype != VCT_RGBA8)
     return vct_set_error(VCT_ERR_INVALID_ARG, "the reference running average needs RGBA8 storage");
-  // the cone marcher addresses texels by 32-bit byte offsets (512^3 with FP32
-  // or with 16-bit storage, whose x-paired copy is twice the volume, is the
-  // largest grid that fits)
-  const uint64_t paired = dtype == VCT_FP32 ? 1 : 2;  // the cone marcher's x-paired copy
-  if (paired * volume_layout(res, levels, dtype, nullptr) > 0xffffffffull)
+  // the cone marcher addresses texels by 32-bit byte offsets (512^3 is the
+  // largest grid that fits, in every storage type: 3.99 GB of FP32 texels,
+  // 16-bit pairs or RGBA8 tiles)
+  const uint64_t span = dtype == VCT_FP32 ? 1 : vct::vct_copy_factor(dtype);
+  if (span * volume_layout(res, levels, dtype, nullptr) > 0xffffffffull)
     return vct_set_error(VCT_ERR_INVALID_ARG, "radiance volume above 4 GiB (use a smaller grid or 16-bit storage)");
   return VCT_OK;
 }
