@@ -289,6 +289,43 @@ def test_gbuffer_bit_exact(gpu_available, orc, kind, ntri, W, H, extra):
     assert np.array_equal(bits(gn), bits(n32))
 
 
+@pytest.mark.parametrize("ntri,W,H,extra", [
+    (20000, 16, 16, {}), (129, 33, 31, {}), (128, 64, 64, {}), (60000, 83, 61, {}), (5000, 2048, 1024, {}),
+    (20000, 70, 45, {"eye": (0.0, 0.1, 0.6), "target": (0.3, 0.0, -1.0)})])
+def test_gbuffer_shared_tiles_bit_exact(gpu_available, orc, ntri, W, H, extra):
+    """Viewports whose tiles several workgroups share: one tile, lists of one
+    chunk and of one chunk and a triangle, more chunks than sharers, the last
+    tile count with two sharers, clipped triangles from an eye inside; every
+    frame twice, the second on the keys the first left."""
+    say(f"gbuffer shared tiles {ntri} triangles {W}x{H}")
+    sc = SceneSpec("soup", ntri=ntri, W=W, H=H, mu=-2.0, **extra)
+    with Context(W, H) as ctx:
+        sc.build(ctx, L.FP16)
+        for _ in range(2):
+            ctx.gbuffer()
+            gp, gn = ctx.download_gbuffer()
+            p32, n32, _, _, _ = orc.gbuffer(W, H, sc.view, sc.proj, [(sc.M, sc.pos, sc.nrm, sc.tri_mat)])
+            assert (p32[..., 3] != 0).any()
+            assert np.array_equal(bits(gp), bits(p32))
+            assert np.array_equal(bits(gn), bits(n32))
+
+
+@pytest.mark.parametrize("dtype,average", [(L.RGBA8, L.AVG_REFERENCE), (L.FP16, L.AVG_EXACT)])
+@pytest.mark.parametrize("res,ntri", [(4, 300), (8, 2000), (16, 5000), (32, 40000), (64, 3000)])
+def test_voxelize_small_grids_bit_exact(gpu_available, orc, res, ntri, dtype, average):
+    """Grids on both sides of the brick edge's rule (4^3 bricks up to 32^3),
+    down to the one that is a single brick."""
+    say(f"voxelize small grid {res}^3 {ntri} triangles dtype={dtype}")
+    sc = SceneSpec("soup", ntri=ntri, res=res, mu=-2.5)
+    with Context(sc.W, sc.H) as ctx:
+        sc.build(ctx, dtype, average)
+        ctx.voxelize()
+        lvl = ctx.download_level(0)
+    key = "ref" if average == L.AVG_REFERENCE else "q32"
+    want = orc.voxelize(res, sc.cube_size, sc.M, sc.pos, sc.nrm, sc.tri_mat, sc.mat_records, sc.lights, want=(key,))[key]
+    assert np.array_equal(bits(lvl), bits(want if key == "ref" else encode_level(want, dtype)))
+
+
 @pytest.mark.parametrize("W,H", [(4096, 4096), (4128, 4096)])
 def test_gbuffer_tile_count_past_one_scan_workgroup(gpu_available, orc, W, H):
     """16,384 tiles, the most whose counts one workgroup scans, and 16,512,

@@ -10,7 +10,7 @@
 //     32x32 tiles the box overlaps (one atomic per distinct tile per wave).
 //  2. exclusive scan of the tile counts.
 //  3. bin write: (triangle, fan triangle) entries into per-tile lists.
-//  4. tile pass (workgroup per tile): exact 64-bit edge functions with the
+//  4. tile pass (a workgroup per tile, several where tiles are few): exact 64-bit edge functions with the
 //     top-left rule, screen-linear depth, LDS atomicMin of
 //     (depth bits << 32 | triangle << 3 | fan triangle); then
 //     perspective-correct world position and normal of each pixel's winner,
@@ -26,6 +26,7 @@
 // rare (they pass near the eye), so their polygon is recomputed where it is
 // needed instead of stored.
 #include <cmath>
+#include <algorithm>
 #include <cstring>
 
 #include <hipcub/hipcub.hpp>
@@ -671,7 +672,7 @@ __device__ __forceinline__ void g_resolve_pixel(const GParams& p, const GRec* __
   gnrm[idx] = make_float4(n[0], n[1], n[2], __builtin_bit_cast(float, dr.mat[lt]));
 }
 
-// 4. one workgroup per 32x32 tile: the depth test runs on a tile depth buffer
+// 4. one workgroup per 32x32 tile (or several, g_tile_share): the depth test runs on a tile depth buffer
 //    in LDS ((depth bits << 32 | original triangle id), 64-bit LDS atomicMin;
 //    equal depths resolve to the lower triangle id, the draw-order winner of
 //    GL_LESS).  The tile's triangles are taken kChunk at a time: their
@@ -755,12 +756,26 @@ __device__ __forceinline__ void g_depth_test(unsigned long long* s_depth, int li
 
 // 6 waves per SIMD: the LDS of 6 workgroups fits a CU, and 80 registers
 // hold the kernel without spills.
+// Workgroups that share a tile's list.  A viewport of few tiles leaves most of
+// the chip idle if each tile has one workgroup, and the longest list decides;
+// so up to kShareMax workgroups take a tile's chunks in turn, each with its own
+// depth buffer, and merge their keys in memory (64-bit minimum, the order does
+// not matter); the last to finish resolves the tile.  G-buffer of 155,000
+// triangles at 211x162 (42 tiles): 0.99 -> 0.20 ms; 46,000 at 83x61 (6 tiles):
+// 0.62 -> 0.15; 300,000 at 1363x767 (1032 tiles), where the tiles' lists differ:
+// 0.28 -> 0.21.  Past kShareTiles / 2 tiles one workgroup
+// each is enough (2560x1440, 3600 tiles: two of them gain the G-buffer 6 % and
+// cost the passes beside it more).
+constexpr uint32_t kShareTiles = 4096, kShareMax = 64;
+static uint32_t g_tile_share(uint32_t ntiles) { return std::min(std::max(kShareTiles / ntiles, 1u), kShareMax); }
+
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void g_tile_kernel(GParams p, const GRec* __restrict__ recs,
                                                      const GRec* __restrict__ fan_recs,
                                                      const GFan* __restrict__ fans,
                                                      const uint32_t* __restrict__ tile_count,
                                                      const uint32_t* __restrict__ tile_off,
-                                                     const uint32_t* __restrict__ list, int tiles_x,
+                                                     const uint32_t* __restrict__ list, int tiles_x, uint32_t ntiles,
+                                                     unsigned long long* merge, uint32_t* done,
                                                      float4* __restrict__ gpos, float4* __restrict__ gnrm) {
 #pragma clang fp contract(off)
   __shared__ unsigned long long s_depth[kTile * kTile];
@@ -770,12 +785,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void g
   __shared__ uint32_t s_wsum[kChunk / 64];
   __shared__ uint32_t s_q[4][128];  // per-wave queue of pixels that passed the edge signs and early depth test
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int tile = blockIdx.x;
+  const uint32_t part = blockIdx.x / ntiles;
+  const int tile = (int)(blockIdx.x - part * ntiles);
   const int x0 = (tile % tiles_x) * kTile, y0 = (tile / tiles_x) * kTile;
-  for (int q = tid; q < kTile * kTile; q += 256) s_depth[q] = ~0ull;
   const uint32_t n = tile_count[tile], base = tile_off[tile];
+  // the workgroups that have a chunk of the list (an empty tile is resolved too)
+  const uint32_t parts = min(gridDim.x / ntiles, max((n + kChunk - 1) / kChunk, 1u));
+  if (part >= parts) return;
+  for (int q = tid; q < kTile * kTile; q += 256) s_depth[q] = ~0ull;
   __syncthreads();
-  for (uint32_t b0 = 0; b0 < n; b0 += kChunk) {
+  for (uint32_t b0 = part * kChunk; b0 < n; b0 += parts * kChunk) {
     if (tid < kChunk) {
       uint32_t rows = 0;
       if (b0 + tid < n) {
@@ -933,6 +952,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void g
     }
     if ((uint32_t)lane < qn) pixel(q[lane]);
     __syncthreads();
+  }
+  if (parts > 1u) {  // merge; the last part to arrive has everyone's keys (the counter's release and acquire)
+    unsigned long long* m = merge + (size_t)tile * (kTile * kTile);
+    for (int q = tid; q < kTile * kTile; q += 256)
+      if (s_depth[q] != ~0ull)
+        __hip_atomic_fetch_min(m + q, s_depth[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (tid == 0)
+      s_wsum[0] = __hip_atomic_fetch_add(done + tile, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (s_wsum[0] != parts - 1u) return;
+    for (int q = tid; q < kTile * kTile; q += 256)  // read back by the lane that resolves it
+      s_depth[q] = __hip_atomic_load(m + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   for (int q = tid; q < kTile * kTile; q += 256) {
     const int i = x0 + (q % kTile), j = y0 + (q / kTile);
@@ -1212,6 +1244,14 @@ __global__ void fill_u32_kernel(uint32_t* p, uint32_t n, uint32_t v) {
 
 using namespace vct;
 
+// Clears a frame's counters and, where workgroups share tiles, the tiles' keys.
+__global__ __launch_bounds__(256) void g_clear_kernel(uint32_t* counters, uint32_t ncounters, unsigned long long* keys,
+                                                      uint32_t nkeys) {
+  const uint32_t n = gridDim.x * 256u;
+  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < ncounters; i += n) counters[i] = 0u;
+  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < nkeys; i += n) keys[i] = ~0ull;
+}
+
 static void mat4_mul(const float* A, const float* B, float* C) {
   // C = A * B, column-major, each element summed k = 0..3 in float
   for (int c = 0; c < 4; ++c)
@@ -1291,18 +1331,23 @@ int vct_launch_gbuffer_phase(vct_context* ctx, int phase) {
   const int tiles_x = (W + kTile - 1) / kTile, tiles_y = (H + kTile - 1) / kTile;
   const uint32_t ntiles = (uint32_t)(tiles_x * tiles_y);
   // [0, ntiles): counts, [ntiles, 2 ntiles): write cursors, then the fan
-  // triangles and the clipped triangles (cleared with them)
-  if ((rc = vct_ensure(ctx->g_count, (size_t)ntiles * 8 + 16, ctx))) return rc;
+  // triangles and the clipped triangles, and the tiles' finished parts
+  // (cleared with them)
+  const uint32_t share = g_tile_share(ntiles), nkeys = share > 1 ? ntiles * (kTile * kTile) : 0u;
+  if ((rc = vct_ensure(ctx->g_count, (size_t)ntiles * 12 + 16, ctx))) return rc;
+  if ((rc = vct_ensure(ctx->g_merge, (size_t)nkeys * 8 + 16, ctx))) return rc;
   if ((rc = vct_ensure(ctx->g_off, (size_t)ntiles * 4 + 16, ctx))) return rc;
   uint32_t* tile_count = (uint32_t*)ctx->g_count.p;
   uint32_t* cursor = tile_count + ntiles;
   uint32_t* fan_total = cursor + ntiles;
   uint32_t* clip_count = fan_total + 1;
+  uint32_t* done = clip_count + 1;
   uint32_t* tile_off = (uint32_t*)ctx->g_off.p;
-  const int lsh = vct_lanes_log2(p.ntri);
+  const int lsh = vct_lanes_log2(p.ntri, ntiles);
   if (phase & 1) {
-    hipLaunchKernelGGL(fill_u32_kernel, dim3((2 * ntiles + 2 + 255) / 256), dim3(256), 0, ctx->stream, tile_count,
-                       2 * ntiles + 2, 0u);
+    const uint32_t ncounters = 3 * ntiles + 2;
+    hipLaunchKernelGGL(g_clear_kernel, dim3((std::max(ncounters, nkeys / 8) + 255) / 256), dim3(256), 0, ctx->stream,
+                       tile_count, ncounters, (unsigned long long*)ctx->g_merge.p, nkeys);
     VCT_HIP(hipGetLastError());
     ctx->h_readback[0] = 0u;
     ctx->h_readback[1] = 0u;
@@ -1347,9 +1392,10 @@ int vct_launch_gbuffer_phase(vct_context* ctx, int phase) {
     if ((rc = vct_ensure(ctx->g_list, 16, ctx))) return rc;
   }
   if ((rc = vct_ensure(ctx->g_recs, 64, ctx))) return rc;
-  hipLaunchKernelGGL(g_tile_kernel, dim3(ntiles), dim3(256), 0, ctx->stream, p, (const GRec*)ctx->g_recs.p,
+  hipLaunchKernelGGL(g_tile_kernel, dim3(ntiles * share), dim3(256), 0, ctx->stream, p, (const GRec*)ctx->g_recs.p,
                      (const GRec*)fan_recs, (const GFan*)fans, (const uint32_t*)tile_count, (const uint32_t*)tile_off, (const uint32_t*)ctx->g_list.p,
-                     tiles_x, (float4*)ctx->g_pos.p, (float4*)ctx->g_nrm.p);
+                     tiles_x, ntiles, (unsigned long long*)ctx->g_merge.p, done, (float4*)ctx->g_pos.p,
+                     (float4*)ctx->g_nrm.p);
   VCT_HIP(hipGetLastError());
   ctx->last_gbuffer_refs = total;
   ctx->g_frame.valid = true;

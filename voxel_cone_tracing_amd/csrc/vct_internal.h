@@ -278,6 +278,7 @@ struct vct_context {
   // G-buffer + image
   VctBuf g_list, g_pos, g_nrm, image;
   VctBuf g_count, g_off, g_recs;  // per-tile counts + cursors, per-tile offsets, per-triangle records
+  VctBuf g_merge;  // depth keys of tiles that several workgroups share
   VctUpload g_draws;               // the G-buffer's draw table
   VctUpload v_draws;               // voxelize's draw table
   VctBuf g_fans;                   // records and resolve data of clipped triangles' fan triangles
@@ -353,7 +354,14 @@ inline int vct_pass_event(vct_context* ctx, int slot, bool end, hipStream_t s) {
 // Lanes per triangle (log2) of the set-up and list kernels: few triangles are
 // spread until 2^18 lanes (4096 waves) run, so that each wave has few large
 // triangles to take one after another; from 2^18 triangles on, one lane each.
-inline int vct_lanes_log2(uint32_t ntri) {
+// A wave adds its triangles to the counters of their tiles or bricks
+// (`targets`) with one atomic per distinct target, so spread triangles add one
+// by one: where that is many per target, the counters' atomics bound the
+// kernels instead (1,700 triangles over 8 tiles: bin count 28 and list write 27
+// us spread, 6 and 5 not; 4,000 over 576: 28 and 41 us not spread, a third of
+// it spread).
+inline int vct_lanes_log2(uint32_t ntri, uint32_t targets) {
+  if (ntri > 16ull * targets) return 0;
   int l = 0;
   while (l < 6 && ((uint64_t)ntri << (l + 1)) <= (1ull << 18)) ++l;
   return l;

@@ -122,7 +122,7 @@ struct Tex<VCT_FP32> {
 // the next line's first again, so the 4 corners of an (x, y) cell are always
 // 16 consecutive bytes of one line: 2 loads fetch the 8 corners (16 bytes at
 // an alignment of 8).  As x-paired entries (4 loads of 8 bytes) the marcher
-// took 1.86 ms of the 2560x1440 frame at 256^3 and 0.83 of the 960x720 one at
+// took 1.86 ms of the 2560x1440 frame at 256^3 and 0.83 of the 1280x720 one at
 // 128^3; tiled 1.68 and 0.72, for 2.7 times the volume written where the pairs
 // were 2 (entries of the four texels, 4 times: 1.71 and 0.73).
 template <int DT>

@@ -346,9 +346,9 @@ __device__ __forceinline__ bool shade_w(const Rec& c, const TriRec* sp, const Vo
 }
 
 // ---- exact mean: bricks of the grid accumulated in LDS ----------------------
-// The grid is cut into cubes of kBrick^3 voxels (the whole grid when smaller);
+// The grid is cut into cubes of kBrick^3 voxels (4^3 on small grids, brick_edge);
 // a brick is one contiguous run of the Morton-ordered level 0, and the low
-// 3 * log2(kBrick) bits of a voxel's Morton index are its index inside the
+// 3 * log2(edge) bits of a voxel's Morton index are its index inside the
 // brick.  Triangles are binned to the bricks their voxel bounding box
 // overlaps; one workgroup per brick rasterises its triangles' pixels inside
 // the brick's footprint on the projection plane, keeps the fragments whose
@@ -367,6 +367,13 @@ constexpr int kBrickThreads = 256;
 // workgroup per CU (the registers' limit) where 256 allowed 6
 constexpr int kBrickItems = 128;
 
+// Grids up to 32^3 would be 64 bricks or fewer of 8^3, a quarter of the CUs
+// with a workgroup each, and take bricks of 4^3: 103,000 triangles at 32^3
+// voxelize in 0.07 ms instead of 0.18 (8^3 bricks), 1,700 in 0.047 instead of
+// 0.10.  At 64^3 (512 bricks of 8^3) soups gain a fifth, but 34 triangles the
+// size of the grid lose 5 %: the larger edge stays.
+__host__ __device__ inline uint32_t brick_edge(uint32_t res) { return res <= 32u ? 4u : (uint32_t)kBrick; }
+
 struct BrickGeom {
   uint32_t bits;    // log2(brick edge)
   uint32_t per;     // bricks per grid edge
@@ -374,8 +381,7 @@ struct BrickGeom {
 
 __device__ __forceinline__ BrickGeom brick_geom(uint32_t res) {
   BrickGeom g;
-  const uint32_t edge = res < (uint32_t)kBrick ? res : (uint32_t)kBrick;
-  g.bits = 31u - __clz(edge);
+  g.bits = 31u - __clz(brick_edge(res));
   g.per = res >> g.bits;
   return g;
 }
@@ -837,7 +843,7 @@ __device__ __forceinline__ void vox_span(int64_t w, int32_t ey, int& lo, int& hi
 // Testing every pixel of the boxes, one per lane with its own three 64-bit
 // edge functions, cost a pixel inside or outside the triangle the same; a row
 // pays for its edges once and its pixels one queue entry each.  The voxelize
-// pass of the 10M-triangle soup at 512^3 4.85 -> 4.08 ms, of the 1M-triangle
+// pass of the 5M-triangle soup at 512^3 4.85 -> 4.08 ms, of the 1M-triangle
 // one at 256^3 0.40 -> 0.37; a walk that also tests each pixel of the span
 // exactly needs spills: 4.34 and 0.40.
 template <class Frag>
@@ -925,7 +931,7 @@ __device__ __forceinline__ uint32_t brick_of_block() {
 }
 
 // Exact mean: sums the brick's fragments and writes its texels.  On grids of
-// many small bricks' worth of fragments the vector ALUs bound it (10M triangles
+// many small bricks' worth of fragments the vector ALUs bound it (5M triangles
 // at 512^3: 2.3 G wave instructions in 3.55 ms, about all the issue slots), on
 // smaller ones the waits on LDS and L2 between its phases do, so it runs at 8
 // waves per SIMD: 64 registers, no spills, and LDS for 8 workgroups per CU.
@@ -1342,7 +1348,8 @@ static int launch_setup(vct_context* ctx, const std::vector<uint32_t>& q, const 
   if ((rc = vct_ensure(ctx->vox_shade, (size_t)(b.ntri ? b.ntri : 1) * sizeof(VoxShade), ctx))) return rc;
   const bool build = !(ctx->vox_shade_epoch == ctx->shade_epoch && ctx->vox_shade_models == q &&
                        ctx->vox_shade_ptr == ctx->vox_shade.p);
-  const int lsh = vct_lanes_log2(b.ntri);
+  const uint32_t per = ctx->res / brick_edge(ctx->res);
+  const int lsh = vct_lanes_log2(b.ntri, per * per * per);
   hipLaunchKernelGGL(vox_brick_count_kernel, dim3(vct_lane_blocks(b.ntri, lsh)), dim3(256), 0, ctx->stream, b, vp,
                      (TriRec*)ctx->setup.p, (const DevMaterial*)ctx->d_materials.p, (VoxShade*)ctx->vox_shade.p,
                      build, (uint2*)ctx->vox_box.p, bcount, lsh);
@@ -1354,8 +1361,9 @@ static int launch_setup(vct_context* ctx, const std::vector<uint32_t>& q, const 
 }
 
 // The list write, lists of `cap` entries in ctx->tri_off.
-static int launch_list(vct_context* ctx, uint32_t ntri, const uint32_t* off, uint32_t* cursor, uint32_t cap) {
-  const int lsh = vct_lanes_log2(ntri);
+static int launch_list(vct_context* ctx, uint32_t ntri, uint32_t nbricks, const uint32_t* off, uint32_t* cursor,
+                       uint32_t cap) {
+  const int lsh = vct_lanes_log2(ntri, nbricks);
   hipLaunchKernelGGL(vox_brick_write_kernel, dim3(vct_lane_blocks(ntri, lsh)), dim3(256), 0, ctx->stream, ntri,
                      ctx->res, (const TriRec*)ctx->setup.p, (const uint2*)ctx->vox_box.p, off, cursor,
                      (uint32_t*)ctx->tri_off.p, cap, lsh);
@@ -1381,9 +1389,7 @@ static void launch_brick(vct_context* ctx, uint32_t nbricks, const VoxParams& vp
 static int voxelize_exact(vct_context* ctx, const std::vector<uint32_t>& q, const VoxParams& vp, void* level0,
                           int phase) {
   const uint32_t res = ctx->res;
-  const uint32_t edge = res < (uint32_t)kBrick ? res : (uint32_t)kBrick;
-  const uint32_t per = res / edge;
-  const uint32_t nbricks = per * per * per;
+  const uint32_t per = res / brick_edge(res), nbricks = per * per * per;
   uint32_t* counters = (uint32_t*)ctx->counters.p;
   int rc;
   // [0, nbricks): counts, [nbricks, 2 nbricks): cursors; then offsets
@@ -1436,7 +1442,7 @@ static int voxelize_exact(vct_context* ctx, const std::vector<uint32_t>& q, cons
         const uint32_t cap = (uint32_t)std::min<uint64_t>(want, 0xffffffffull);
         if ((rc = vct_ensure(ctx->tri_off, (size_t)cap * 4, ctx))) return rc;
         ctx->vox_cap = cap;
-        if ((rc = launch_list(ctx, ntri, boff, cursor, cap))) return rc;
+        if ((rc = launch_list(ctx, ntri, nbricks, boff, cursor, cap))) return rc;
         ctx->vox_total_pending = true;
         ctx->vox_pairs_on_device = true;
         bricks((const uint32_t*)ctx->tri_off.p, ListCap{(const uint2*)ctx->vox_box.p, ntri, cap});
@@ -1449,7 +1455,7 @@ static int voxelize_exact(vct_context* ctx, const std::vector<uint32_t>& q, cons
   const uint32_t total = ntri ? ctx->h_readback[2] : 0u;
   if (total) {
     if ((rc = vct_ensure(ctx->tri_off, (size_t)total * 4 + (size_t)total / 4 * 4, ctx))) return rc;
-    if ((rc = launch_list(ctx, ntri, boff, cursor, total))) return rc;
+    if ((rc = launch_list(ctx, ntri, nbricks, boff, cursor, total))) return rc;
   } else {
     hipLaunchKernelGGL(zero_u32_kernel, dim3((nbricks + 255) / 256), dim3(256), 0, ctx->stream, boff,
                        (uint64_t)nbricks);
@@ -1473,9 +1479,7 @@ static int voxelize_exact(vct_context* ctx, const std::vector<uint32_t>& q, cons
 static int voxelize_reference(vct_context* ctx, const std::vector<uint32_t>& q, const VoxParams& vp, void* level0,
                               int phase) {
   const uint32_t res = ctx->res;
-  const uint32_t edge = res < (uint32_t)kBrick ? res : (uint32_t)kBrick;
-  const uint32_t per = res / edge;
-  const uint32_t nbricks = per * per * per;
+  const uint32_t per = res / brick_edge(res), nbricks = per * per * per;
   uint32_t* counters = (uint32_t*)ctx->counters.p;  // [2] pairs
   int rc;
   // per-brick counts + cursors (the cursors hold the fragment counts at the end), offsets
@@ -1515,7 +1519,7 @@ static int voxelize_reference(vct_context* ctx, const std::vector<uint32_t>& q, 
   }
   const size_t seg = ((size_t)pairs + pairs / 4 + 3) & ~(size_t)3;
   if ((rc = vct_ensure(ctx->tri_off, seg * 8, ctx))) return rc;
-  if ((rc = launch_list(ctx, ntri, boff, cursor, pairs))) return rc;
+  if ((rc = launch_list(ctx, ntri, nbricks, boff, cursor, pairs))) return rc;
   hipLaunchKernelGGL(vox_ref_kernel, dim3(nbricks), dim3(kBrickThreads), 0, ctx->stream, vp,
                      (const TriRec*)ctx->setup.p, (const VoxShade*)ctx->vox_shade.p, (const uint32_t*)bcount,
                      (const uint32_t*)boff, (uint32_t*)ctx->tri_off.p, (uint32_t*)ctx->tri_off.p + seg,
