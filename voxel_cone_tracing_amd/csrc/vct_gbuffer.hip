@@ -738,9 +738,8 @@ __device__ __forceinline__ uint32_t g_zmin_bits(const GRec& r) {
   return zmin > 0.0f ? __builtin_bit_cast(uint32_t, zmin) : 0u;
 }
 
-__device__ __forceinline__ bool g_hidden(const unsigned long long* s_depth, int li, int lj, uint32_t zmin_bits) {
-  const uint32_t cur = (uint32_t)(s_depth[lj * kTile + li] >> 32);
-  return zmin_bits > cur;
+__device__ __forceinline__ bool g_hidden(unsigned long long key, uint32_t zmin_bits) {
+  return zmin_bits > (uint32_t)(key >> 32);
 }
 
 __device__ __forceinline__ void g_depth_test(unsigned long long* s_depth, int li, int lj, float b0, float b1,
@@ -754,8 +753,6 @@ __device__ __forceinline__ void g_depth_test(unsigned long long* s_depth, int li
   }
 }
 
-// 6 waves per SIMD: the LDS of 6 workgroups fits a CU, and 80 registers
-// hold the kernel without spills.
 // Workgroups that share a tile's list.  A viewport of few tiles leaves most of
 // the chip idle if each tile has one workgroup, and the longest list decides;
 // so up to kShareMax workgroups take a tile's chunks in turn, each with its own
@@ -769,6 +766,8 @@ __device__ __forceinline__ void g_depth_test(unsigned long long* s_depth, int li
 constexpr uint32_t kShareTiles = 4096, kShareMax = 64;
 static uint32_t g_tile_share(uint32_t ntiles) { return std::min(std::max(kShareTiles / ntiles, 1u), kShareMax); }
 
+// 6 waves per SIMD: the LDS of 6 workgroups fits a CU.  Chunks of 64 and 7 or 8
+// waves were no faster (1M triangles at 2560x1440: 0.49 ms against 0.45).
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void g_tile_kernel(GParams p, const GRec* __restrict__ recs,
                                                      const GRec* __restrict__ fan_recs,
                                                      const GFan* __restrict__ fans,
@@ -844,9 +843,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void g
     __syncthreads();
     const uint32_t total = s_end[kChunk - 1];
     // Pixels in two phases.  1: each lane walks the span of its row with the
-    // edge signs and the early depth rejection only, and appends the pixels
-    // that pass to its wave's queue in LDS (ballot + popcount; no barrier:
-    // only the wave touches it).  2: whenever the queue holds 64, every lane
+    // early depth rejection only, and appends the pixels that pass to its
+    // wave's queue in LDS (ballot + popcount; no barrier: only the wave touches
+    // it).  Edge functions stepped along the span, which the exact test repeats,
+    // drop next to none of its pixels and cost the loop three 64-bit additions
+    // and compares (G-buffer of 5M triangles at 3840x2160 2.43 -> 2.06 ms, of 1M
+    // at 2560x1440 0.51 -> 0.45).  2: whenever the queue holds 64, every lane
     // takes one and runs the exact test (top-left rule), the barycentrics and
     // the depth test, so the expensive part runs with all lanes busy instead
     // of on the lanes whose rows are still long.  A pixel's key reaches its
@@ -891,58 +893,46 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void g
         if (k < 64u) break;
       }
       const uint32_t ek = own0 + (uint32_t)lane < (uint32_t)kChunk ? s_end[own0 + lane] : 0xffffffffu;
+      // the ends inside the window, a prefix of the lanes; few are read one by
+      // one into scalar registers instead of by dependent shuffles
+      const uint32_t nend = (uint32_t)__popcll(__ballot(ek < c0 + 64u));
       uint32_t past = 0;
-      for (uint32_t st = 32; st; st >>= 1)
-        if ((uint32_t)__shfl(ek, (int)(past + st - 1u), 64) <= c) past += st;
-      if ((uint32_t)__shfl(ek, (int)past, 64) <= c) ++past;
+      if (nend <= 8u) {
+        for (uint32_t k = 0; k < nend; ++k) past += (uint32_t)__builtin_amdgcn_readlane((int)ek, (int)k) <= c ? 1u : 0u;
+      } else {
+        for (uint32_t st = 32; st; st >>= 1)
+          if ((uint32_t)__shfl(ek, (int)(past + st - 1u), 64) <= c) past += st;
+        if ((uint32_t)__shfl(ek, (int)past, 64) <= c) ++past;
+      }
       // the lane's row and its span: for each edge w(i) = w_row + di * (i - ci0)
       // >= 0, bounded in float with a margin (the exact tests decide)
-      int len = 0, lo_i = 0, lj = 0;
-      uint32_t lo = 0, row = 0, zb = 0;
-      int64_t wa = 0, wb = 0, wc = 0, da = 0, db = 0, dc = 0;
+      int len = 0;
+      uint32_t desc = 0, zb = 0;
+      const unsigned long long* depth = s_depth;
       if (c < total) {
-        lo = own0 + past;
+        uint32_t lo = own0 + past;
         if (past == 64u)
           while (s_end[lo] <= c) ++lo;
-        row = c - (lo ? s_end[lo - 1] : 0u);
+        const uint32_t row = c - (lo ? s_end[lo - 1] : 0u);
         const GRowSetup& g = s_row[lo];
-        const int ci0 = g.ci0, ci1 = g.ci1;
-        lj = (int)g.cj0 + (int)row - y0;
-        const int64_t ra = g.w0[0] + g.dj[0] * (int64_t)row;
-        const int64_t rb = g.w0[1] + g.dj[1] * (int64_t)row;
-        const int64_t rc = g.w0[2] + g.dj[2] * (int64_t)row;
-        int hi_i = ci1;
-        lo_i = ci0;
+        const int ci0 = g.ci0;
+        int lo_i = ci0, hi_i = g.ci1;
         const GTileRec& tr = s_tr[lo];
-        g_span(ra, g.di[0], tr.inv[0], ci0, lo_i, hi_i);
-        g_span(rb, g.di[1], tr.inv[1], ci0, lo_i, hi_i);
-        g_span(rc, g.di[2], tr.inv[2], ci0, lo_i, hi_i);
-        if (lo_i <= hi_i) {
-          len = hi_i - lo_i + 1;
-          const int64_t k0 = lo_i - ci0;
-          da = g.di[0];
-          db = g.di[1];
-          dc = g.di[2];
-          wa = ra + da * k0;
-          wb = rb + db * k0;
-          wc = rc + dc * k0;
-          zb = tr.zb;
-        }
+        g_span(g.w0[0] + g.dj[0] * (int64_t)row, g.di[0], tr.inv[0], ci0, lo_i, hi_i);
+        g_span(g.w0[1] + g.dj[1] * (int64_t)row, g.di[1], tr.inv[1], ci0, lo_i, hi_i);
+        g_span(g.w0[2] + g.dj[2] * (int64_t)row, g.di[2], tr.inv[2], ci0, lo_i, hi_i);
+        len = hi_i - lo_i + 1;
+        zb = tr.zb;
+        const uint32_t li = (uint32_t)(lo_i - x0);
+        desc = lo | (row << 7) | (li << 12);
+        depth += ((int)g.cj0 + (int)row - y0) * kTile + (int)li;
       }
       // the wave walks its longest span; each lane stops at the end of its own
-      for (int k = 0; __ballot(k < len) != 0ull; ++k) {
-        bool hit = false;
-        uint32_t desc = 0;
-        if (k < len) {
-          const int li = lo_i + k - x0;
-          hit = wa >= 0 && wb >= 0 && wc >= 0 && !g_hidden(s_depth, li, lj, zb);
-          desc = lo | (row << 7) | ((uint32_t)li << 12);
-          wa += da;
-          wb += db;
-          wc += dc;
-        }
+      for (int k = 0;; ++k) {
+        if (__ballot(k < len) == 0ull) break;
+        const bool hit = k < len && !g_hidden(depth[k], zb);
         const unsigned long long m = __ballot(hit);
-        if (hit) q[qn + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = desc;
+        if (hit) q[qn + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = desc + ((uint32_t)k << 12);
         qn += (uint32_t)__popcll(m);
         if (qn >= 64u) {
           qn -= 64u;
