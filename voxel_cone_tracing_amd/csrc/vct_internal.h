@@ -120,11 +120,20 @@ VCT_HD float f16_to_f32(uint16_t h) {
 }
 
 // GL unorm8 -> float: c / 255 (the GL definition; correctly rounded divide).
-VCT_HD float unorm8_exact(uint32_t c) { return (float)c / 255.0f; }
+// Two terms of 1/255 give the correctly rounded quotient for every byte (all
+// 256 compared) in 2 operations where a division takes about 10.
+VCT_HD float unorm8_exact(uint32_t c) {
+  const float f = (float)c;
+  return __builtin_fmaf(f, 0x1.010102p-8f, f * -0x1.fdfdfep-33f);
+}
 // float -> GL unorm8: clamp to [0,1], scale by 255, round to nearest even.
 VCT_HD uint32_t to_unorm8(float f) {
+#ifdef __HIP_DEVICE_COMPILE__
+  f = __builtin_amdgcn_fmed3f(f, 0.0f, 1.0f);  // NaN: the lower bound
+#else
   f = f > 0.0f ? f : 0.0f;  // also maps NaN to 0
   f = f < 1.0f ? f : 1.0f;
+#endif
   return (uint32_t)__builtin_rintf(f * 255.0f);
 }
 
