@@ -447,6 +447,35 @@ def test_reference_average_rounds_bit_exact(gpu_available, orc, res, n, size):
     assert nfrag == int(want["count"].sum())
 
 
+@pytest.mark.parametrize("n", [2, 64, 65, 128, 129, 256, 257, 1024, 1025])
+def test_reference_average_one_brick_bit_exact(gpu_available, orc, n):
+    """n triangles inside one 8^3 brick of a 64^3 grid: the list sorted by rank
+    (1, 2 or 4 lanes a triangle), by a bitonic sort past 256 triangles and by
+    radix passes past 1024, and voxels with many fragments each."""
+    say(f"reference average, {n} triangles in one brick")
+    res = 64
+    rng = np.random.default_rng(n)
+    sc = SceneSpec("soup", ntri=n, res=res, W=16, H=16)
+    centre = 0.125 * sc.cube_size  # the middle of the brick after the grid's
+    p = centre * (1.0 + rng.uniform(-0.6, 0.6, (n, 1, 3))) + 0.02 * sc.cube_size * rng.uniform(-1.0, 1.0, (n, 3, 3))
+    nrm = np.cross(p[:, 1] - p[:, 0], p[:, 2] - p[:, 0])
+    nrm /= np.linalg.norm(nrm, axis=1, keepdims=True)
+    sc.pos = np.ascontiguousarray(p.reshape(n, 9).astype(np.float32))
+    sc.nrm = np.ascontiguousarray(np.repeat(nrm[:, None], 3, 1).reshape(n, 9).astype(np.float32))
+    want = orc.voxelize(res, sc.cube_size, sc.M, sc.pos, sc.nrm, sc.tri_mat, sc.mat_records, sc.lights,
+                        want=("ref", "count"))
+    z, y, x = np.nonzero(want["count"])
+    assert (np.stack([z, y, x]) // 8 == 4).all()
+    with Context(16, 16) as ctx:
+        sc.build(ctx, L.RGBA8, L.AVG_REFERENCE)
+        for _ in range(2):
+            ctx.voxelize()
+            assert np.array_equal(ctx.download_level(0), want["ref"])
+        nfrag, _ = ctx.voxelize_stats()
+    say(f"  {nfrag} fragments, up to {int(want['count'].max())} in a voxel")
+    assert nfrag == int(want["count"].sum())
+
+
 # ---- trace (kernel c) ----------------------------------------------------------------
 @pytest.mark.parametrize("kind,dtype,res,ntri", [("cornell", L.RGBA8, 64, 34), ("cornell", L.FP16, 64, 34),
                                                  ("soup", L.FP16, 64, 4000), ("soup", L.BF16, 64, 4000),

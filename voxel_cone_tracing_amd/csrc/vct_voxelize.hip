@@ -732,11 +732,21 @@ __device__ __forceinline__ uint32_t replay_step(uint32_t stored, float vx, float
   rz = rz * fn + vz;
   rw = rw * fn + vw;
   ++n;
+  // x / n correctly rounded for n = 1 .. 16: the rounded reciprocal (one
+  // Newton step from the approximation), the product and one correction by its
+  // exact remainder (compared for every n and mantissa); 4 divisions cost four
+  // times as many cycles
   const float fn1 = (float)n;
-  rx = rx / fn1;
-  ry = ry / fn1;
-  rz = rz / fn1;
-  rw = rw / fn1;
+  float inv = __builtin_amdgcn_rcpf(fn1);
+  inv = __builtin_fmaf(__builtin_fmaf(-fn1, inv, 1.0f), inv, inv);
+  auto div = [&](float x) {
+    const float q = x * inv;
+    return __builtin_fmaf(__builtin_fmaf(-fn1, q, x), inv, q);
+  };
+  rx = div(rx);
+  ry = div(ry);
+  rz = div(rz);
+  rw = div(rw);
   rx = __builtin_rintf(rx / 2.0f) * 2.0f;
   ry = __builtin_rintf(ry / 2.0f) * 2.0f;
   rz = __builtin_rintf(rz / 2.0f) * 2.0f;
@@ -1000,15 +1010,18 @@ __global__ __launch_bounds__(kBrickThreads) __attribute__((amdgpu_waves_per_eu(8
 // triangle index (in LDS up to kRefSort triangles, by a radix sort in global
 // memory past that), takes the triangles in rounds in that order, keeps a
 // round's fragments in LDS (colour and a 15-bit key: place of the triangle in
-// the round, pixel in the brick's footprint), groups them by voxel, and each
-// voxel's lane sorts its few by key and replays the packed RGBA8 + count
-// nibble recurrence on them.  A round whose fragments do not fit is taken
+// the round, pixel in the brick's footprint), groups them by voxel, ranks each
+// by its key among its voxel's, and each voxel's lane replays the packed RGBA8
+// + count nibble recurrence on them.  A round whose fragments do not fit is taken
 // again with half its triangles: three triangles always fit (a footprint has
 // 256 pixels).  A pass that counted the fragments of every voxel, a scan over
 // the voxels, a host wait for the number of fragments and a pass that stored
 // them in global memory, sorted and replayed them took the voxelize pass of
-// the 1M-triangle soup at 256^3 1.15 ms; this one pass 0.81 (voxels replayed
-// in their own order rather than the fullest first: 0.99).
+// the 1M-triangle soup at 256^3 1.15 ms; this one pass 0.76 (voxels replayed
+// in their own order rather than the fullest first: 0.99) and 0.61 since the
+// list and the fragments are ranked side by side (they were sorted by a bitonic
+// network, a barrier a stage, and by insertion, a chain of LDS reads) and the
+// recurrence divides by a reciprocal.
 constexpr int kRefFrags = 768;   // fragments of a round (512 at 6 waves per SIMD: no faster)
 constexpr int kRefSort = 1024;   // triangles sorted in LDS
 
@@ -1016,13 +1029,19 @@ struct RefLds {
   union {
     struct {
       float col[3][kRefFrags];
-      uint16_t key[kRefFrags], vox[kRefFrags], idx[kRefFrags];
+      // key << 9 | voxel of each fragment; then, voxel by voxel in order, its
+      // triangle's place in the round << 10 | fragment
+      uint32_t kv[kRefFrags];
+      uint32_t ent[kRefFrags];  // key << 10 | fragment, voxel by voxel
     };
     unsigned long long sort[kRefSort];  // original triangle << 32 | triangle
+    alignas(16) uint32_t otri[256];
     uint32_t hist[4][256];
   };
 };
 static_assert(sizeof(RefLds) >= kRefSort * 8, "the sort uses the fragments' space");
+static_assert(kRefFrags <= 1024 && kRefFrags % kBrickThreads == 0 && kBrickItems <= 128 && kBrick * kBrick * kBrick <= 512,
+              "packing of kv and ent");
 
 // Sorts the brick's list segment by original triangle index in global memory
 // (4 stable passes of 8 bits between the segment and its place in `other`; an
@@ -1106,6 +1125,26 @@ __global__ __launch_bounds__(kBrickThreads) __attribute__((amdgpu_waves_per_eu(5
   // ---- the list in order ---------------------------------------------------------
   if (n > (uint32_t)kRefSort) {
     ref_radix_sort(R, seg, list2 + base, n, recs);
+  } else if (n > 1u && n <= (uint32_t)kBrickThreads) {
+    // each triangle's rank, by comparing it with every other one: 256, 128 or
+    // 64 threads' worth of them by 1, 2 or 4 lanes each, with three barriers
+    // where a bitonic sort of 64 has 22
+    const uint32_t sh = n <= 64u ? 2u : (n <= 128u ? 1u : 0u);
+    const uint32_t k = (uint32_t)tid >> sh, h = (uint32_t)tid & ((1u << sh) - 1u);
+    uint32_t t = 0;
+    if ((uint32_t)tid < n) t = seg[tid];
+    R.otri[tid] = (uint32_t)tid < n ? recs[t].otri : 0xffffffffu;
+    __syncthreads();
+    const uint32_t mine = R.otri[k];
+    uint32_t rank = 0;
+    for (uint32_t j = 4u * h; j < n; j += 4u << sh) {
+      const uint4 o = *reinterpret_cast<const uint4*>(&R.otri[j]);
+      rank += (o.x < mine) + (o.y < mine) + (o.z < mine) + (o.w < mine);
+    }
+    for (uint32_t o = 1; o < (1u << sh); o <<= 1) rank += (uint32_t)__shfl_xor((int)rank, (int)o, 64);
+    const uint32_t own = k < n ? seg[k] : 0u;
+    __syncthreads();  // every lane has read the segment
+    if (h == 0u && k < n) seg[rank] = own;
   } else if (n > 1u) {
     uint32_t m = 64;  // a bitonic sort of the next power of two
     while (m < n) m <<= 1;
@@ -1144,7 +1183,7 @@ __global__ __launch_bounds__(kBrickThreads) __attribute__((amdgpu_waves_per_eu(5
     if ((uint32_t)tid < m) {
       const uint32_t t = seg[pos + tid];
       cnt = brick_stage(s_round, tid, t, recs, bc, span, lim);
-      s_alpha[tid] = shade[t].alpha;
+      s_alpha[tid] = fminf(fmaxf(shade[t].alpha, 0.0f), 1.0f) * 255.0f;
     }
     const uint32_t total = brick_prefix(s_round, cnt);
     brick_scan(s_round, total, [&](uint32_t d, bool on) {
@@ -1170,9 +1209,9 @@ __global__ __launch_bounds__(kBrickThreads) __attribute__((amdgpu_waves_per_eu(5
         R.col[1][slot] = color.y;
         R.col[2][slot] = color.z;
         // the order within a triangle: 2x2 quads row by row, each quad x then y
-        R.key[slot] = (uint16_t)((lo << 8) | (((uint32_t)j >> 1 & 7u) << 5) | (((uint32_t)i >> 1 & 7u) << 2) |
-                                 (((uint32_t)j & 1u) << 1) | ((uint32_t)i & 1u));
-        R.vox[slot] = (uint16_t)lv;
+        const uint32_t pix = (((uint32_t)j >> 1 & 7u) << 5) | (((uint32_t)i >> 1 & 7u) << 2) |
+                             (((uint32_t)j & 1u) << 1) | ((uint32_t)i & 1u);
+        R.kv[slot] = (((lo << 8) | pix) << 9) | lv;
         atomicAdd(&s_cnt[lv], 1u);
       }
     });
@@ -1200,9 +1239,14 @@ __global__ __launch_bounds__(kBrickThreads) __attribute__((amdgpu_waves_per_eu(5
     if (c0) atomicAdd(&s_place[min(c0, 63u)], 1u);
     if (c1) atomicAdd(&s_place[min(c1, 63u)], 1u);
     __syncthreads();
-    for (uint32_t f = tid; f < nf; f += kBrickThreads) {
-      const uint32_t lv = R.vox[f];
-      R.idx[s_off[lv] + atomicSub(&s_cnt[lv], 1u) - 1u] = (uint16_t)f;
+    constexpr int kMine = kRefFrags / kBrickThreads;  // fragments of a lane
+    uint32_t kv[kMine];
+#pragma unroll
+    for (int r = 0; r < kMine; ++r) {
+      const uint32_t f = (uint32_t)(tid + r * kBrickThreads);
+      kv[r] = f < nf ? R.kv[f] : 0u;
+      const uint32_t lv = kv[r] & 511u;
+      if (f < nf) R.ent[s_off[lv] + atomicSub(&s_cnt[lv], 1u) - 1u] = ((kv[r] >> 9) << 10) | f;
     }
     // voxels with fragments, most first: a wave's lanes then replay voxels of
     // like length, and voxels without fragments take no lanes
@@ -1220,27 +1264,29 @@ __global__ __launch_bounds__(kBrickThreads) __attribute__((amdgpu_waves_per_eu(5
     if (c0) s_ord[atomicAdd(&s_place[min(c0, 63u)], 1u)] = (uint16_t)v0;
     if (c1) s_ord[atomicAdd(&s_place[min(c1, 63u)], 1u)] = (uint16_t)v1;
     __syncthreads();
+    // each fragment's place among its voxel's: how many of them have a smaller key
+#pragma unroll
+    for (int r = 0; r < kMine; ++r) {
+      const uint32_t f = (uint32_t)(tid + r * kBrickThreads);
+      if (f >= nf) break;
+      const uint32_t v = kv[r] & 511u, key = kv[r] >> 9;
+      const uint32_t beg = s_off[v], end = v + 1u < nvox ? s_off[v + 1u] : nf;
+      uint32_t at = beg;
+      for (uint32_t a = beg; a < end; ++a) at += R.ent[a] >> 10 < key ? 1u : 0u;
+      R.kv[at] = ((key >> 8) << 10) | f;
+    }
+    __syncthreads();
     // ---- each voxel's fragments in order, through the recurrence -------------------
     const uint32_t nused = s_nfrag;
     for (uint32_t k = tid; k < nused; k += kBrickThreads) {
       const uint32_t v = s_ord[k], beg = s_off[v], end = v + 1u < nvox ? s_off[v + 1u] : nf;
-      for (uint32_t a = beg + 1u; a < end; ++a) {  // insertion sort by key
-        const uint16_t f = R.idx[a];
-        const uint32_t kf = R.key[f];
-        uint32_t b = a;
-        while (b > beg) {
-          const uint16_t p = R.idx[b - 1u];
-          if (R.key[p] <= kf) break;
-          R.idx[b] = p;
-          --b;
-        }
-        R.idx[b] = f;
-      }
       uint32_t st = s_state[v];
+      uint32_t o = R.kv[beg];
       for (uint32_t a = beg; a < end; ++a) {
-        const uint32_t f = R.idx[a];
-        const float al = fminf(fmaxf(s_alpha[R.key[f] >> 8], 0.0f), 1.0f);
-        st = replay_step(st, R.col[0][f] * 255.0f, R.col[1][f] * 255.0f, R.col[2][f] * 255.0f, al * 255.0f);
+        const uint32_t f = o & 1023u;
+        const float al = s_alpha[o >> 10];
+        o = R.kv[min(a + 1u, end - 1u)];
+        st = replay_step(st, R.col[0][f] * 255.0f, R.col[1][f] * 255.0f, R.col[2][f] * 255.0f, al);
       }
       s_state[v] = st;
     }
