@@ -978,23 +978,41 @@ struct VViewVol {
   int res, levels, dtype;
 };
 
-__device__ __forceinline__ float4 vv_texel(const VViewVol& V, int l, int map, int x, int y, int z) {
-  const char* lv = V.base + V.off[l][l == 0 ? 0 : map];
-  const uint32_t e = brick_index((uint32_t)x, (uint32_t)y, (uint32_t)z);
-  if (V.dtype == VCT_RGBA8) {
-    const uint32_t v = reinterpret_cast<const uint32_t*>(lv)[e];
-    return make_float4(unorm8_exact(v & 255u), unorm8_exact((v >> 8) & 255u), unorm8_exact((v >> 16) & 255u),
-                       unorm8_exact(v >> 24));
+__device__ __forceinline__ float4 vv_decode(int, uint32_t v) {
+  return make_float4(unorm8_exact(v & 255u), unorm8_exact((v >> 8) & 255u), unorm8_exact((v >> 16) & 255u),
+                     unorm8_exact(v >> 24));
+}
+__device__ __forceinline__ float4 vv_decode(int dtype, uint2 v) {
+  if (dtype == VCT_FP16)
+    return make_float4(f16_to_f32((uint16_t)(v.x & 0xffffu)), f16_to_f32((uint16_t)(v.x >> 16)),
+                       f16_to_f32((uint16_t)(v.y & 0xffffu)), f16_to_f32((uint16_t)(v.y >> 16)));
+  return make_float4(bf16_to_f32((uint16_t)(v.x & 0xffffu)), bf16_to_f32((uint16_t)(v.x >> 16)),
+                     bf16_to_f32((uint16_t)(v.y & 0xffffu)), bf16_to_f32((uint16_t)(v.y >> 16)));
+}
+__device__ __forceinline__ float4 vv_decode(int, float4 v) { return v; }
+
+// The weighted sum of the eight corners, corner k at element e[k]: all loads
+// go out before any is used.  A corner outside the level has weight 0 and an
+// element inside it, whose value is dropped rather than multiplied (an
+// uploaded level may hold infinities).
+template <typename T>
+__device__ __forceinline__ float4 vv_corners(int dtype, const T* lv, const uint32_t (&e)[8], const float (&wt)[8],
+                                             uint32_t inside) {
+#pragma clang fp contract(off)
+  T raw[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) raw[k] = lv[e[k]];
+  float4 out = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float4 t = vv_decode(dtype, raw[k]);
+    const bool in = (inside >> k) & 1u;
+    out.x = out.x + (in ? wt[k] * t.x : 0.0f);
+    out.y = out.y + (in ? wt[k] * t.y : 0.0f);
+    out.z = out.z + (in ? wt[k] * t.z : 0.0f);
+    out.w = out.w + (in ? wt[k] * t.w : 0.0f);
   }
-  if (V.dtype == VCT_FP16 || V.dtype == VCT_BF16) {
-    const uint2 v = reinterpret_cast<const uint2*>(lv)[e];
-    if (V.dtype == VCT_FP16)
-      return make_float4(f16_to_f32((uint16_t)(v.x & 0xffffu)), f16_to_f32((uint16_t)(v.x >> 16)),
-                         f16_to_f32((uint16_t)(v.y & 0xffffu)), f16_to_f32((uint16_t)(v.y >> 16)));
-    return make_float4(bf16_to_f32((uint16_t)(v.x & 0xffffu)), bf16_to_f32((uint16_t)(v.x >> 16)),
-                       bf16_to_f32((uint16_t)(v.y & 0xffffu)), bf16_to_f32((uint16_t)(v.y >> 16)));
-  }
-  return reinterpret_cast<const float4*>(lv)[e];
+  return out;
 }
 
 // One level, trilinear with a zero border (CLAMP_TO_BORDER, texture_3d.cpp:10-15).
@@ -1005,20 +1023,24 @@ __device__ __forceinline__ float4 vv_trilinear(const VViewVol& V, int l, int map
   const float fu = floorf(u), fv = floorf(v), fw = floorf(w);
   const int i0 = (int)fu, j0 = (int)fv, k0 = (int)fw;
   const float a = u - fu, b = v - fv, c = w - fw;
-  float4 out = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (int dz = 0; dz < 2; ++dz)
-    for (int dy = 0; dy < 2; ++dy)
-      for (int dx = 0; dx < 2; ++dx) {
-        const int x = i0 + dx, y = j0 + dy, z = k0 + dz;
-        if (x < 0 || y < 0 || z < 0 || x >= s || y >= s || z >= s) continue;
-        const float wt = (dx ? a : 1.0f - a) * (dy ? b : 1.0f - b) * (dz ? c : 1.0f - c);
-        const float4 t = vv_texel(V, l, map, x, y, z);
-        out.x = out.x + wt * t.x;
-        out.y = out.y + wt * t.y;
-        out.z = out.z + wt * t.z;
-        out.w = out.w + wt * t.w;
-      }
-  return out;
+  auto at = [s](int q) { return spread3((uint32_t)min(max(q, 0), s - 1)); };
+  const uint32_t sx[2] = {at(i0), at(i0 + 1)}, sy[2] = {at(j0) << 1, at(j0 + 1) << 1},
+                 sz[2] = {at(k0) << 2, at(k0 + 1) << 2};
+  uint32_t e[8], inside = 0;
+  float wt[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const int dx = k & 1, dy = (k >> 1) & 1, dz = k >> 2;
+    e[k] = sx[dx] | sy[dy] | sz[dz];
+    wt[k] = (dx ? a : 1.0f - a) * (dy ? b : 1.0f - b) * (dz ? c : 1.0f - c);
+    // (one unsigned compare: a negative coordinate is past the edge)
+    if ((uint32_t)(i0 + dx) < (uint32_t)s && (uint32_t)(j0 + dy) < (uint32_t)s && (uint32_t)(k0 + dz) < (uint32_t)s)
+      inside |= 1u << k;
+  }
+  const char* lv = V.base + V.off[l][l == 0 ? 0 : map];
+  if (V.dtype == VCT_RGBA8) return vv_corners(V.dtype, reinterpret_cast<const uint32_t*>(lv), e, wt, inside);
+  if (V.dtype == VCT_FP32) return vv_corners(V.dtype, reinterpret_cast<const float4*>(lv), e, wt, inside);
+  return vv_corners(V.dtype, reinterpret_cast<const uint2*>(lv), e, wt, inside);
 }
 
 // textureLod with LINEAR_MIPMAP_LINEAR, lod clamped to [0, levels - 1].
