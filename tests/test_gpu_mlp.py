@@ -407,3 +407,33 @@ def test_tile_check_and_refinement_hold_40db(gpu_available, half):
     assert p >= 40.0
     assert st["tiles"] == 10 * 6 and 0 <= st["tiles_full"] <= st["tiles_refined"] <= st["tiles"]
     assert st["probes"] >= 16 * st["tiles"]
+
+
+@pytest.mark.parametrize("W,H", [(96, 64), (324, 164)])
+def test_rgba8_traced_pixels_match_the_plain_frame(gpu_available, W, H):
+    """RGBA8 storage: the learned form's launches scale each texel by 1/255
+    before weighting it, the plain frame the weighted sum, so a traced pixel
+    differs from the plain frame's by rounding alone: 2^-24 in each of the ~20
+    operations from a texel to a pixel, over a sum of ten cones, is at most
+    1.2e-5."""
+    sc = SceneSpec("soup", res=64, ntri=20000, W=W, H=H, mu=-4.0)
+    with Context(W, H) as ctx:
+        sc.build(ctx, L.RGBA8)
+        ctx.mlp_set_params(np.zeros(L.MLP_PARAMS, np.float32))
+        ctx.set_fallback(0.0)
+        plain = _plain(ctx, sc)
+        sc_q(ctx, sc)
+        ctx.render_learned()
+        img = ctx.download_image()
+        traced = ctx.traced_pixels()
+        low = ctx.download_lowres()
+        gp, gn = ctx.download_gbuffer()
+    cov = gp[..., 3] != 0
+    mid = gn[..., 3].copy().view(np.uint32)
+    alb = sc.mat_records[np.where(cov, mid, 0)][..., 4:7]
+    _, st = _guided_numpy(gp, gn, low, alb, W, H)
+    t = st == 2
+    err = np.abs(img[t] - plain[t]).max()
+    say(f"traced {traced}, max-abs vs plain {err:.3e}")
+    assert traced == int(t.sum()) and traced > 0
+    assert err <= 1.2e-5

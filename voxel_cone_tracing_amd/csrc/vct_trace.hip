@@ -76,6 +76,17 @@ struct TraceArgs {
 
 // Storage types: raw texel as loaded (Raw) and its decode to float4; the
 // decode folds into the blend (v_fma_mix_f32 for the 16-bit types).
+// RGBA8 storage as the learned form's launches read it.  Its network rounds
+// what the trace gives it to BF16 and its tiles are picked by their errors, so
+// the last bit of a sample can move a pixel by 6e-4 (936x692, sixteen cones):
+// there each texel is scaled by 1/255 before it is weighted, as a texel fetch
+// rounds.  Plain frames scale the weighted sum instead: a byte then takes half
+// the vector cycles (quarter-resolution trace of that frame 0.16 ms against
+// 0.19, its tiles traced in full 0.30 against 0.38).
+constexpr int kRgba8Unorm = 4;
+template <int DT>
+constexpr bool kBytes = DT == VCT_RGBA8 || DT == kRgba8Unorm;
+
 template <int DT>
 struct Tex;
 template <>
@@ -87,6 +98,8 @@ struct Tex<VCT_RGBA8> {
                        (float)(v >> 24) * k);
   }
 };
+template <>
+struct Tex<kRgba8Unorm> : Tex<VCT_RGBA8> {};
 template <>
 struct Tex<VCT_FP16> {
   using Raw = uint2;
@@ -143,6 +156,8 @@ struct Pair16 {
   static __device__ __forceinline__ Raw make(uint2 a, uint2 b) { return pair_pack(a, b); }
 };
 template <>
+struct Pair<kRgba8Unorm> : Pair<VCT_RGBA8> {};
+template <>
 struct Pair<VCT_FP16> : Pair16<VCT_FP16> {};
 template <>
 struct Pair<VCT_BF16> : Pair16<VCT_BF16> {};
@@ -161,8 +176,14 @@ __device__ __forceinline__ uint32_t tile_z(uint32_t z) { return (spread3(z >> 1)
 __device__ __forceinline__ float4 f4(float x) { return make_float4(x, x, x, x); }
 // The four bytes of an RGBA8 texel, each masked in place and taken as the bits
 // of a (subnormal) float: byte * 2^-149, * 2^-141, * 2^-133 and, shifted down,
-// * 2^-149.
+// * 2^-149 (kRgba8Unorm: as byte / 255).
+template <int DT>
 __device__ __forceinline__ float4 bytes4(uint32_t v) {
+  if constexpr (DT == kRgba8Unorm) {
+    float k = 1.0f / 255.0f;
+    return make_float4((float)(v & 255u) * k, (float)((v >> 8) & 255u) * k, (float)((v >> 16) & 255u) * k,
+                       (float)(v >> 24) * k);
+  }
   return make_float4(__builtin_bit_cast(float, v & 0xffu), __builtin_bit_cast(float, v & 0xff00u),
                      __builtin_bit_cast(float, v & 0xff0000u), __builtin_bit_cast(float, v >> 24));
 }
@@ -197,9 +218,9 @@ template <int DT>
 __device__ __forceinline__ void sampler_init(const TraceArgs& A, SamplerLds* S) {
   for (uint32_t q = threadIdx.x; q < (uint32_t)kMaxEdge; q += blockDim.x) {
     const uint32_t v = spread3(q) << 4;  // a 16-bit pair or an FP32 texel has 16 bytes
-    S->sx[q] = DT == VCT_RGBA8 ? tile_x(q) : v;
-    S->sy[q] = DT == VCT_RGBA8 ? tile_y(q) : v << 1;
-    S->sz[q] = DT == VCT_RGBA8 ? tile_z(q) : v << 2;
+    S->sx[q] = kBytes<DT> ? tile_x(q) : v;
+    S->sy[q] = kBytes<DT> ? tile_y(q) : v << 1;
+    S->sz[q] = kBytes<DT> ? tile_z(q) : v << 2;
   }
   for (int q = threadIdx.x; q < 16 * 6; q += blockDim.x) S->off[q / 6][(q % 6) ^ 1] = (uint32_t)A.off[q / 6][q % 6];
 }
@@ -297,7 +318,7 @@ __device__ __forceinline__ void gather_pairs(const char* __restrict__ vol, uint3
 #pragma unroll
   for (int k = 0; k < n; ++k) {
     const char* p = vol + (base + c.ix[0] + c.iyz[k * (4 / n)]);
-    __builtin_memcpy(&r[k], __builtin_assume_aligned(p, DT == VCT_RGBA8 ? 8 : 16), sizeof(Raw));
+    __builtin_memcpy(&r[k], __builtin_assume_aligned(p, kBytes<DT> ? 8 : 16), sizeof(Raw));
   }
 }
 
@@ -368,8 +389,8 @@ __device__ __forceinline__ float4 blend4(const PairWeights<DT>& W, const typenam
   } else {
 #pragma unroll
     for (int k = 0; k < 2; ++k)
-      acc = acc + W.w[4 * k] * bytes4(r[k].x) + W.w[4 * k + 1] * bytes4(r[k].z) + W.w[4 * k + 2] * bytes4(r[k].y) +
-            W.w[4 * k + 3] * bytes4(r[k].w);
+      acc = acc + W.w[4 * k] * bytes4<DT>(r[k].x) + W.w[4 * k + 1] * bytes4<DT>(r[k].z) +
+            W.w[4 * k + 2] * bytes4<DT>(r[k].y) + W.w[4 * k + 3] * bytes4<DT>(r[k].w);
   }
   return acc;
 }
@@ -561,7 +582,7 @@ struct WideOf<VCT_BF16> {
 // FP32: 4 waves in 126 registers 0.367 ms, 5 waves and 24 bytes of scratch
 // 0.398; the 16-bit types hold 12 paired loads in flight and spill past 5).
 template <int DT>
-constexpr int kTraceWaves = DT == VCT_RGBA8 ? 6 : (DT == VCT_FP32 ? 4 : 5);
+constexpr int kTraceWaves = kBytes<DT> ? 6 : (DT == VCT_FP32 ? 4 : 5);
 
 // 32.32 fixed point of a non-negative cone colour channel (< 2^31): sums of
 // these are exact, so the diffuse cones of a pixel may finish in any order.
@@ -1447,7 +1468,10 @@ int vct_trace_select(vct_context* ctx, const float4* gpos, const float4* gnrm, f
   const int nshadow = (ctx->en_direct && ctx->en_shadow) ? n : 0;
   const bool wide = nshadow <= ShapeTile::NSHADOW;
   switch (ctx->dtype) {
-    case VCT_RGBA8: rc = launch_trace<VCT_RGBA8>(ctx, A, sel, W, H, wide); break;
+    case VCT_RGBA8:
+      if (demodulate || sel.pix_list || sel.tile_list) rc = launch_trace<kRgba8Unorm>(ctx, A, sel, W, H, wide);
+      else rc = launch_trace<VCT_RGBA8>(ctx, A, sel, W, H, wide);
+      break;
     case VCT_FP16: rc = launch_trace<VCT_FP16>(ctx, A, sel, W, H, wide); break;
     case VCT_BF16: rc = launch_trace<VCT_BF16>(ctx, A, sel, W, H, wide); break;
     default: rc = launch_trace<VCT_FP32>(ctx, A, sel, W, H, wide); break;
