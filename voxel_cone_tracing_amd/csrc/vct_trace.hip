@@ -1393,16 +1393,19 @@ static void launch_shape(vct_context* ctx, const TraceArgs& A, const TraceSelect
 template <int DT>
 static int launch_trace(vct_context* ctx, const TraceArgs& A, const TraceSelect& sel, int W, int H, bool wide) {
   if ((sel.pix_list && sel.npix_list == 0) || (!sel.pix_list && sel.tile_list && sel.max_tiles == 0)) return VCT_OK;
-  // A viewport (or pixel list) of at most 2^18 pixels is at most 2048
-  // workgroups of 128 pixels, under two rounds of the ~1280 that 256 CUs hold
-  // at once, so the last round runs part-empty; 64-pixel workgroups halve
-  // that tail.  Measured on the 1M-triangle soup: 640x360 0.384 -> 0.345 ms
-  // (no change at 1280x720 and above, where 128 pixels shorten each
-  // workgroup's drain instead); the learned frame's 57,600 probes beside it,
-  // 3.257 -> 3.244 ms for the frame.
-  if (wide && !sel.tile_list && (sel.pix_list ? (size_t)sel.npix_list : (size_t)W * H) <= (1u << 18))
+  // The 256 CUs hold about 1280 workgroups of any shape at once, so a viewport
+  // of few workgroups runs a part-empty last round whose length is that of one
+  // workgroup, all its pixels' cones: small viewports take small workgroups.
+  // Up to 2^19 pixels 64 (trace at 753x400, BF16, sixteen cones and two shadows
+  // a pixel: 0.78 ms in workgroups of 192 pixels, 0.53 of 128, 0.44 of 64;
+  // 855x512 FP16 0.69, 0.57, 0.50; 1001x563 FP32 0.35 of 128, 0.38 of 64), up to
+  // 3 * 2^18 128 (974x700 FP16: 0.182 of 64, 0.160 of 128, 0.162 of 192; 1363x767
+  // BF16: 1.26, 1.27, 1.24).  A pixel list runs beside other launches: 64 up to
+  // 2^18 pixels (the learned frame's 57,600 probes, 3.257 -> 3.244 ms).
+  const size_t npix = sel.pix_list ? (size_t)sel.npix_list : (size_t)W * H;
+  if (wide && !sel.tile_list && npix <= (sel.pix_list ? 1u << 18 : 1u << 19))
     launch_shape<DT, ShapeSmall>(ctx, A, sel, W, H);
-  else if (wide && (sel.pix_list || sel.tile_list)) launch_shape<DT, ShapeTile>(ctx, A, sel, W, H);
+  else if (wide && (sel.pix_list || sel.tile_list || npix <= 3u << 18)) launch_shape<DT, ShapeTile>(ctx, A, sel, W, H);
   else if (wide) launch_shape<DT, typename WideOf<DT>::type>(ctx, A, sel, W, H);
   else launch_shape<DT, ShapeFull>(ctx, A, sel, W, H);
   return VCT_OK;
