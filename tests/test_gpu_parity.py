@@ -211,6 +211,43 @@ def test_voxelize_follows_material_changes_bit_exact(gpu_available, orc, dtype, 
         check(every2, "the first model queued again")
 
 
+@pytest.mark.parametrize("dtype,average", [(L.FP16, L.AVG_EXACT), (L.RGBA8, L.AVG_REFERENCE)])
+@pytest.mark.parametrize("change", ["grid", "transform", "cube"])
+def test_voxelize_keeps_terms_of_undrawn_triangles(gpu_available, orc, dtype, average, change):
+    """The per-triangle material terms kept from the first frame hold for
+    every queued triangle, drawn then or not: triangles that the first frame
+    dropped (between the pixel centres of a coarse grid, off the grid by the
+    model matrix, or too small in a larger cube) and the second frame draws
+    have their own materials there."""
+    say(f"voxelize: undrawn, then drawn; dtype={dtype} average={average} change={change}")
+    res = 128
+    sc = SceneSpec("soup", res=res, ntri=6000, mu=-4.0, model="rot_scale")
+    with Context(32, 32) as ctx:
+        sc.build(ctx, dtype, average)
+        if change == "grid":
+            ctx.set_grid(8, 4, dtype, average)
+        elif change == "transform":
+            away = sc.M.copy().reshape(-1)
+            away[12:15] += 50.0
+            ctx.set_model_transform(sc.model, away.reshape(4, 4))
+        else:
+            ctx.set_grid_size(60.0)
+        ctx.voxelize()
+        if change == "grid":
+            ctx.set_grid(res, 7, dtype, average)
+        elif change == "transform":
+            ctx.set_model_transform(sc.model, sc.M)
+        else:
+            ctx.set_grid_size(sc.cube_size)
+        ctx.voxelize()
+        got = ctx.download_level(0)
+    want = orc.voxelize(res, sc.cube_size, sc.M, sc.pos, sc.nrm, sc.tri_mat, sc.mat_records, sc.lights,
+                        want=("ref", "q32", "count"))
+    assert want["count"].sum() > 6000
+    w = want["ref"] if average == L.AVG_REFERENCE else encode_level(want["q32"], dtype)
+    assert np.array_equal(bits(got), bits(w)), f"{np.count_nonzero(bits(got) != bits(w))} values differ"
+
+
 # ---- voxelize under a model matrix (voxelize.vert:24-30) ----------------------------
 @pytest.mark.parametrize("dtype,average", [(L.RGBA8, L.AVG_REFERENCE), (L.FP16, L.AVG_EXACT), (L.FP32, L.AVG_EXACT)])
 def test_voxelize_with_model_matrix_bit_exact(gpu_available, orc, dtype, average):

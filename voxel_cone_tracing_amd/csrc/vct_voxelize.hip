@@ -543,10 +543,8 @@ __global__ __launch_bounds__(256) void vox_brick_count_kernel(DrawTable b, VoxPa
     DevMaterial m;
     if (build_shade) m = mats[dr.mat[lt]];
     tri_setup(dr, lt, vp.res, vp.cube_size, s);
-    if (s.ok) {
-      rec = make_rec(dr, lt, s);
-      if (build_shade) h = make_shade(m);
-    }
+    if (s.ok) rec = make_rec(dr, lt, s);
+    if (build_shade) h = make_shade(m);  // also of a triangle that draws nothing in this frame
   }
   const BrickBox bb = brick_box(s, vp.res, g);
   uint4* w = s_out[wave];
