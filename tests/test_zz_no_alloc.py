@@ -82,3 +82,68 @@ def test_noalloc_forward_equals_forward(gpu_available):
         finally:
             dx.free()
             dy.free()
+
+
+@pytest.mark.parametrize("n,offset", [(1, 0), (33, 0), (5000, 0), (5000, -3), (5000, 33 * 5000), (5000, 34 * 5000 - 1),
+                                      (L.MLP_NOALLOC_MAX_ROWS, 0), (L.MLP_NOALLOC_MAX_ROWS, 17 * 100_001)])
+def test_noalloc_outputs_may_overlap_the_features(gpu_available, n, offset):
+    """out inside features (offset in floats from their start), at either end
+    and only 4-byte aligned: the outputs are vct_mlp_forward's, and what lies
+    outside them keeps its bits."""
+    say(f"no-alloc forward in place, n={n} offset={offset}")
+    rng = np.random.default_rng(n + offset)
+    p = (rng.standard_normal(L.MLP_PARAMS) * 0.2).astype(np.float32)
+    x = (rng.random((n, 34)) * 2 - 0.5).astype(np.float32)
+    pad = 4  # floats before the features and after the last output
+    flat = np.concatenate([np.zeros(pad, np.float32), x.reshape(-1), np.zeros(3 * n + pad, np.float32)])
+    with Context(16, 16) as ctx:
+        ctx.mlp_set_params(p)
+        ctx.sync()
+        want = ctx.mlp_forward(x)
+        d = DeviceBuffer(flat.nbytes)
+        try:
+            d.put(flat)
+            L.check(ctx.lib.vct_mlp_forward_noalloc(ctx.h, d.p.value + 4 * pad, n, d.p.value + 4 * (pad + offset), None))
+            ctx.sync()
+            got = d.get(np.zeros_like(flat))
+        finally:
+            d.free()
+    flat[pad + offset:pad + offset + 3 * n] = want.reshape(-1)
+    assert np.array_equal(got.view(np.uint32), flat.view(np.uint32))
+
+
+def test_noalloc_calls_on_two_streams(gpu_available):
+    """Calls in flight at the same time on two streams, with inputs and row
+    counts of their own, each give vct_mlp_forward's outputs."""
+    say("no-alloc forward on two streams")
+    rng = np.random.default_rng(6)
+    p = (rng.standard_normal(L.MLP_PARAMS) * 0.2).astype(np.float32)
+    xs = [(rng.random((n, 34)) * 2 - 0.5).astype(np.float32) for n in (200_003, 70_001)]
+    with Context(16, 16) as ctx:
+        ctx.mlp_set_params(p)
+        ctx.sync()
+        want = [ctx.mlp_forward(x) for x in xs]
+        dx = [DeviceBuffer(x.nbytes) for x in xs]
+        dy = [DeviceBuffer(w.nbytes) for w in want]
+        hip = DeviceBuffer.hip
+        streams = [C.c_void_p(), C.c_void_p()]
+        try:
+            for s in streams:
+                assert hip.hipStreamCreateWithFlags(C.byref(s), C.c_uint(1)) == 0  # non-blocking, default priority
+            for d, x in zip(dx, xs):
+                d.put(x)
+            for d, w in zip(dy, want):
+                d.put(np.full_like(w, np.nan))
+            for _ in range(8):
+                for s, x, a, b in zip(streams, xs, dx, dy):
+                    L.check(ctx.lib.vct_mlp_forward_noalloc(ctx.h, a.p, x.shape[0], b.p, s))
+            for s in streams:
+                assert hip.hipStreamSynchronize(s) == 0
+            for d, w in zip(dy, want):
+                assert np.array_equal(d.get(np.zeros_like(w)).view(np.uint32), w.view(np.uint32))
+        finally:
+            for s in streams:
+                if s.value:
+                    hip.hipStreamDestroy(s)
+            for d in dx + dy:
+                d.free()

@@ -459,6 +459,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
   }
 }
 
+__global__ __launch_bounds__(256) void copy_f32_kernel(const float* __restrict__ src, uint32_t n,
+                                                       float* __restrict__ dst) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i < n) dst[i] = src[i];
+}
+
 // ---- training: forward + backward, a wave per 32 samples --------------------------
 // The A and B operands of v_mfma_f32_16x16x32_bf16 have one layout, so
 // exchanging them yields the transposed tile: every activation and gradient
@@ -1148,7 +1154,7 @@ int mlp_ensure(vct_context* ctx) {
   if ((rc = vct_ensure(ctx->mlp_packed, kPacked * 2, ctx))) return rc;
   if ((rc = vct_ensure(ctx->mlp_bias, 144 * 4, ctx))) return rc;
   if ((rc = vct_ensure(ctx->mlp_grad, (kParams + 1) * 4, ctx))) return rc;
-  return VCT_OK;
+  return vct_ensure(ctx->mlp_stage, (size_t)VCT_MLP_NOALLOC_MAX_ROWS * kOut * 4, ctx);
 }
 
 int mlp_pack(vct_context* ctx) {
@@ -1604,7 +1610,17 @@ int vct_mlp_forward_noalloc(vct_ctx ctx, const float* features, uint32_t n, floa
     return vct_set_error(VCT_ERR_LIMIT, "vct_mlp_forward_noalloc takes at most VCT_MLP_NOALLOC_MAX_ROWS rows");
   int rc;
   if ((rc = need_mlp(ctx))) return rc;
-  return launch_forward(ctx, features, n, out, stream ? (hipStream_t)stream : ctx->stream);
+  const hipStream_t st = stream ? (hipStream_t)stream : ctx->stream;
+  // The kernel reads the rows and writes the outputs in no order of its own,
+  // so outputs that overlap the rows wait in mlp_stage until every row is read.
+  const uintptr_t f = (uintptr_t)features, o = (uintptr_t)out;
+  const bool overlap = f < o + (uintptr_t)n * (kOut * 4) && o < f + (uintptr_t)n * (kIn * 4);
+  if (!overlap) return launch_forward(ctx, features, n, out, st);
+  if ((rc = launch_forward(ctx, features, n, (float*)ctx->mlp_stage.p, st))) return rc;
+  hipLaunchKernelGGL(copy_f32_kernel, dim3((n * kOut + 255) / 256), dim3(256), 0, st, (const float*)ctx->mlp_stage.p,
+                     n * kOut, out);
+  VCT_HIP(hipGetLastError());
+  return VCT_OK;
 }
 
 int vct_mlp_loss_grad(vct_ctx ctx, const float* features, const float* albedo, const float* target, uint32_t n,
