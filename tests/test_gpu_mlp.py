@@ -437,3 +437,32 @@ def test_rgba8_traced_pixels_match_the_plain_frame(gpu_available, W, H):
     say(f"traced {traced}, max-abs vs plain {err:.3e}")
     assert traced == int(t.sum()) and traced > 0
     assert err <= 1.2e-5
+
+
+@pytest.mark.parametrize("n,bad", [(64, [(5, 3)]), (200, [(0, 33), (130, 17)]), (8192, [(4097, 0), (4099, 31), (8191, 32)])])
+def test_gradient_of_nonfinite_features_matches_oracle(gpu_available, orc, n, bad):
+    """A NaN, or an infinity that every unit of layer 1 cuts (negative
+    weights), leaves its sample without positive activations, so of the
+    gradient only the feature's own column is NaN (0 * NaN): the pattern is
+    the oracle's, and the rest holds the bars of test_gradient_matches_oracle."""
+    say(f"mlp gradient, non-finite features n={n} {bad}")
+    rng = np.random.default_rng(n)
+    x = rng.random((n, 34)).astype(np.float32)
+    a = rng.random((n, 3)).astype(np.float32)
+    t = rng.random((n, 3)).astype(np.float32)
+    p = _params(6)
+    w1 = p[:64 * 34].reshape(64, 34)
+    for k, (row, col) in enumerate(bad):
+        x[row, col] = np.inf if k & 1 else np.nan
+        w1[:, col] = -np.abs(w1[:, col])
+    with Context(16, 16) as ctx:
+        ctx.mlp_set_params(p)
+        loss, g = ctx.mlp_loss_grad(x, a, t)
+    wl, wg = orc.mlp_loss_grad(p, x, a, t, bf16=True)
+    nan = np.isnan(wg)
+    assert nan.sum() == 64 * len(bad)
+    assert np.array_equal(np.isnan(g), nan), f"NaN at {np.flatnonzero(np.isnan(g) != nan)[:8]}"
+    rel = np.linalg.norm(g[~nan] - wg[~nan]) / np.linalg.norm(wg[~nan])
+    say(f"  loss {loss:.6f} vs {wl:.6f}; gradient relative error {rel:.2e}")
+    assert abs(loss - wl) <= 1e-3 * wl
+    assert rel < 2e-2

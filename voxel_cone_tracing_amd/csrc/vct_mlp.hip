@@ -496,6 +496,13 @@ struct TrainArgs {
 constexpr uint32_t kTrainRows = 128;   // samples of a workgroup at a time, 32 per wave
 constexpr uint32_t kTrainBlocks = 256;
 
+// Carries into bits 15 and 31 where a word's BF16 halves are infinite or NaN.
+__device__ __forceinline__ uint32_t nonfinite(bf16x8 v) {
+  const uint4 w = __builtin_bit_cast(uint4, v);
+  auto carry = [](uint32_t u) { return (u & 0x7f807f80u) + 0x00800080u; };
+  return (carry(w.x) | carry(w.y) | carry(w.z) | carry(w.w)) & 0x80008000u;
+}
+
 __device__ __forceinline__ bf16x8 join(uint2 a, uint2 b) {
   return __builtin_bit_cast(bf16x8, make_uint4(a.x, a.y, b.x, b.y));
 }
@@ -554,6 +561,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     for (int t = 0; t < 2; ++t) {
 #pragma unroll
       for (int nt = 0; nt < 3; ++nt) xT[t][nt] = pack4(mfma32(x[t][nt >> 1], eye[nt & 1], z));
+      // the product would spread an infinite or NaN feature (0 * NaN) over its
+      // sample's others: such tiles are read from the rows instead
+      if (__ballot((nonfinite(x[t][0]) | nonfinite(x[t][1])) != 0u)) {
+#pragma unroll
+        for (int nt = 0; nt < 3; ++nt) {
+          uint32_t v[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const uint32_t r = (uint32_t)__shfl((int)row[t], 4 * q + i, 64);
+            v[i] = base + 16u * t + 4u * q + i < A.n ? A.X[(size_t)r * 64 + 16 * nt + col] : 0u;
+          }
+          xT[t][nt] = make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
+        }
+      }
       uint2 p[4];
 #pragma unroll
       for (int mt = 0; mt < 4; ++mt) {
