@@ -466,3 +466,19 @@ def test_gradient_of_nonfinite_features_matches_oracle(gpu_available, orc, n, ba
     say(f"  loss {loss:.6f} vs {wl:.6f}; gradient relative error {rel:.2e}")
     assert abs(loss - wl) <= 1e-3 * wl
     assert rel < 2e-2
+
+
+def test_infinite_activations_give_an_infinite_loss(gpu_available):
+    """An infinite unit of layer 2 makes every output, and so the loss,
+    infinite; the output tile's unused columns (zero weights) stay out of it."""
+    say("mlp loss, infinite activations")
+    rng = np.random.default_rng(2)
+    x, a, t = (rng.random((100, k)).astype(np.float32) + 0.1 for k in (34, 3, 3))
+    p = _params(7)
+    b2, w3 = 64 * 34 + 64 + 64 * 64, 64 * 34 + 64 + 64 * 64 + 64
+    p[b2 + 5] = np.inf
+    p[[w3 + 5, w3 + 64 + 5, w3 + 128 + 5]] = 0.5
+    with Context(16, 16) as ctx:
+        ctx.mlp_set_params(p)
+        loss, _ = ctx.mlp_loss_grad(x, a, t)
+    assert loss == np.inf

@@ -619,19 +619,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       hf[t][0] = next_frag(p[0], p[1]);
       hf[t][1] = next_frag(p[2], p[3]);
     }
-    // outputs (samples x outputs) and their gradient; lanes past the outputs hold zeros
+    // outputs (samples x outputs) and their gradient; lanes past the outputs
+    // and samples past the last hold zeros, whatever infinite activations
+    // make of them
     uint2 dyT[2];
     bf16x8 dy[2];
     {
       const bf16x8 w0 = ld_frag(pk + kPW3, 64), w1 = ld_frag(pk + kPW3 + 32, 64);
       const float b = A.P.b3[col];
+      const int left = col < kOut ? (int)min(A.n - base, 32u) - 4 * q : 0;  // samples from the lane's first on
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         const floatx4 y = mfma32(hf[t][1], w1, mfma32(hf[t][0], w0, z));
         floatx4 d;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float e = al[t][i] * ((y[i] + b) - tg[t][i]);
+          const float e = 16 * t + i < left ? al[t][i] * ((y[i] + b) - tg[t][i]) : 0.f;
           loss += e * e;
           d[i] = A.scale * al[t][i] * e;  // d(loss)/dy
           db3 += d[i];
