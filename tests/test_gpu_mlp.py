@@ -482,3 +482,53 @@ def test_infinite_activations_give_an_infinite_loss(gpu_available):
         ctx.mlp_set_params(p)
         loss, _ = ctx.mlp_loss_grad(x, a, t)
     assert loss == np.inf
+
+
+@pytest.mark.parametrize("half", [True, False])
+@pytest.mark.parametrize("dtype", [L.RGBA8, L.FP16, L.BF16, L.FP32])
+def test_traced_pixels_equal_the_plain_frame(gpu_available, dtype, half):
+    """Every pixel that the learned frame traces itself is the plain frame's bit
+    for bit, in every storage type: the pixels without a same-surface sample
+    and the probes and, at a bound that no interpolation meets, every covered
+    pixel but the half-resolution stage's."""
+    say(f"traced pixels against the plain frame, dtype={dtype} half={half}")
+    W, H = 324, 164
+    sc = SceneSpec("soup", res=64, ntri=20000, W=W, H=H, mu=-4.0)
+
+    def learned(ctx, db):
+        ctx.set_fallback(db)
+        sc_q(ctx, sc)
+        ctx.render_learned()
+        return ctx.download_image()
+
+    with Context(W, H) as ctx:
+        sc.build(ctx, dtype)
+        ctx.mlp_set_params(np.zeros(L.MLP_PARAMS, np.float32))
+        ctx.set_refine(half)
+        plain = _plain(ctx, sc)
+        unchecked, checked, full = learned(ctx, 0.0), learned(ctx, 40.0), learned(ctx, 120.0)
+        st = ctx.upsample_stats()
+        low = ctx.download_lowres()
+        gp, gn = ctx.download_gbuffer()
+    cov = gp[..., 3] != 0
+    mid = gn[..., 3].copy().view(np.uint32)
+    alb = sc.mat_records[np.where(cov, mid, 0)][..., 4:7]
+    _, status = _guided_numpy(gp, gn, low, alb, W, H)
+    traced = status == 2
+    assert traced.sum() > 0
+    same = [(img.view(np.uint32) == plain.view(np.uint32)).all(-1) for img in (unchecked, checked, full)]
+    assert same[0][traced].all(), f"{np.count_nonzero(~same[0][traced])} listed pixels differ"
+    probe = np.zeros((H, W), bool)
+    ty, tx = np.meshgrid(np.arange(-(-H // 32)), np.arange(-(-W // 32)), indexing="ij")
+    for o in (3, 11, 19, 27):
+        for b in (3, 11, 19, 27):
+            probe[np.minimum(ty * 32 + b, H - 1), np.minimum(tx * 32 + o, W - 1)] = True
+    if not half:  # (the half-resolution stage interpolates over the first probes)
+        assert same[1][probe & cov].all(), f"{np.count_nonzero(~same[1][probe & cov])} probes differ"
+
+    def tiles(a, fill):  # per 32x32 tile: every pixel true
+        return np.pad(a, ((0, -H % 32), (0, -W % 32)), constant_values=fill).reshape(-1, 32, -(-W // 32), 32).all((1, 3))
+
+    whole, empty = tiles(same[2] | ~cov, True), tiles(~cov, True)
+    say(f"  {st}, whole {int(whole.sum())}, empty {int(empty.sum())}")
+    assert st["tiles_full"] > 0 and (whole & ~empty).sum() >= st["tiles_full"]

@@ -76,13 +76,15 @@ struct TraceArgs {
 
 // Storage types: raw texel as loaded (Raw) and its decode to float4; the
 // decode folds into the blend (v_fma_mix_f32 for the 16-bit types).
-// RGBA8 storage as the learned form's launches read it.  Its network rounds
-// what the trace gives it to BF16 and its tiles are picked by their errors, so
-// the last bit of a sample can move a pixel by 6e-4 (936x692, sixteen cones):
-// there each texel is scaled by 1/255 before it is weighted, as a texel fetch
-// rounds.  Plain frames scale the weighted sum instead: a byte then takes half
-// the vector cycles (quarter-resolution trace of that frame 0.16 ms against
-// 0.19, its tiles traced in full 0.30 against 0.38).
+// RGBA8 storage as the learned form's demodulated launches read it: what they
+// trace is interpolated and goes into a network that rounds its inputs to BF16,
+// where the last bit of a sample can move a pixel by 6e-4 (936x692, sixteen
+// cones), so each texel is scaled by 1/255 before it is weighted, as a texel
+// fetch rounds.  Every launch that traces pixels of the image itself, plain or
+// learned, scales the weighted sum instead, so a traced pixel is the plain
+// frame's bit for bit: a byte then takes half the vector cycles
+// (quarter-resolution trace of that frame 0.16 ms against 0.19, its tiles
+// traced in full 0.30 against 0.38).
 constexpr int kRgba8Unorm = 4;
 template <int DT>
 constexpr bool kBytes = DT == VCT_RGBA8 || DT == kRgba8Unorm;
@@ -1472,7 +1474,7 @@ int vct_trace_select(vct_context* ctx, const float4* gpos, const float4* gnrm, f
   const bool wide = nshadow <= ShapeTile::NSHADOW;
   switch (ctx->dtype) {
     case VCT_RGBA8:
-      if (demodulate || sel.pix_list || sel.tile_list) rc = launch_trace<kRgba8Unorm>(ctx, A, sel, W, H, wide);
+      if (demodulate) rc = launch_trace<kRgba8Unorm>(ctx, A, sel, W, H, wide);
       else rc = launch_trace<VCT_RGBA8>(ctx, A, sel, W, H, wide);
       break;
     case VCT_FP16: rc = launch_trace<VCT_FP16>(ctx, A, sel, W, H, wide); break;
