@@ -484,6 +484,41 @@ def test_reference_average_rounds_bit_exact(gpu_available, orc, res, n, size):
     assert nfrag == int(want["count"].sum())
 
 
+@pytest.mark.parametrize("res,n,size", [(64, 2000, 1.0), (64, 1200, 0.3)])
+def test_reference_average_of_large_triangles_in_proportion(gpu_available, orc, res, n, size):
+    """Bricks of triangles that fill their footprint, a few of which fit in a
+    round, and of mixed sizes: the texels are the oracle's, and the average
+    takes at most 12 times as long as the exact mean, which tests the same
+    pixels once (a round that always starts from 128 triangles tests them 30
+    to 60 times: 28.6 times as long at 2,000 triangles, 5.3 when rounds follow
+    the fragments of the one before)."""
+    say(f"reference average, large triangles, res={res} n={n} size={size}")
+    rng = np.random.default_rng(n + res)
+    p = rng.uniform(-1.0, 1.0, (n, 1, 3)) + size * rng.standard_normal((n, 3, 3))
+    nrm = np.cross(p[:, 1] - p[:, 0], p[:, 2] - p[:, 0])
+    nrm /= np.linalg.norm(nrm, axis=1, keepdims=True)
+    sc = SceneSpec("soup", ntri=n, res=res, W=16, H=16)
+    sc.pos = np.ascontiguousarray(p.reshape(n, 9).astype(np.float32))
+    sc.nrm = np.ascontiguousarray(np.repeat(nrm[:, None], 3, 1).reshape(n, 9).astype(np.float32))
+    want = orc.voxelize(res, sc.cube_size, sc.M, sc.pos, sc.nrm, sc.tri_mat, sc.mat_records, sc.lights,
+                        want=("ref", "count"))
+    ms = {}
+    for average in (L.AVG_REFERENCE, L.AVG_EXACT):
+        with Context(16, 16) as ctx:
+            sc.build(ctx, L.RGBA8, average)
+            t = []
+            for _ in range(6):
+                ctx.voxelize()
+                ctx.sync()
+                t.append(float(ctx.pass_times()[0]))
+            ms[average] = min(t)
+            if average == L.AVG_REFERENCE:
+                assert np.array_equal(ctx.download_level(0), want["ref"])
+                assert ctx.voxelize_stats()[0] == int(want["count"].sum())
+    say(f"  reference {ms[L.AVG_REFERENCE]:.3f} ms, exact mean {ms[L.AVG_EXACT]:.3f} ms")
+    assert ms[L.AVG_REFERENCE] <= 12.0 * ms[L.AVG_EXACT]
+
+
 @pytest.mark.parametrize("n", [2, 64, 65, 128, 129, 256, 257, 1024, 1025])
 def test_reference_average_one_brick_bit_exact(gpu_available, orc, n):
     """n triangles inside one 8^3 brick of a 64^3 grid: the list sorted by rank
