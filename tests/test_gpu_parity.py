@@ -406,6 +406,45 @@ def test_gbuffer_many_models(gpu_available, orc):
     assert np.array_equal(bits(gn), bits(n32))
 
 
+def test_equal_draw_tables_on_both_streams(gpu_available):
+    """An unchanged draw table is copied once, for the frame's second stream or
+    the context's: passes called one by one and whole frames in turn, with the
+    table unchanged, changed and changed back, give the buffers of a context
+    that only runs that call."""
+    say("draw tables, frames and single passes in turn")
+    W, H = 320, 200
+    sc = SceneSpec("soup", res=64, ntri=4000, W=W, H=H, mu=-3.0)
+    moved = sc.M.copy().reshape(-1)
+    moved[12:15] += 0.2
+
+    def passes(ctx, whole, M):
+        ctx.set_model_transform(sc.model, M)
+        ctx.clear_queues()
+        ctx.queue_model(sc.model)
+        for (p, c, i, k) in sc.lights:
+            ctx.queue_light(p, c, i, k)
+        if whole:
+            ctx.render()
+        else:
+            ctx.gbuffer()
+            ctx.voxelize()
+        return [bits(a) for a in (*ctx.download_gbuffer(), ctx.download_level(0))]
+
+    want = {}
+    for key, M in (("home", sc.M), ("moved", moved.reshape(4, 4))):
+        with Context(W, H) as ctx:
+            sc.build(ctx, L.FP16)
+            want[key] = passes(ctx, False, M)
+    assert not np.array_equal(want["home"][0], want["moved"][0])
+    with Context(W, H) as ctx:
+        sc.build(ctx, L.FP16)
+        for whole, key in [(True, "home"), (False, "home"), (True, "home"), (True, "moved"), (False, "moved"),
+                           (False, "home"), (True, "home"), (False, "home")]:
+            got = passes(ctx, whole, sc.M if key == "home" else moved.reshape(4, 4))
+            for g, w in zip(got, want[key]):
+                assert np.array_equal(g, w), (whole, key)
+
+
 def large_triangles(n, seed):
     """Triangles of 0.01 to 3 world units around and across the grid, every
     fourth a sliver, every fifth flat in a coordinate plane."""

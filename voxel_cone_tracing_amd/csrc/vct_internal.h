@@ -206,12 +206,14 @@ struct VctBuf {
 // A per-frame table (the draws of a pass) copied to the device on a stream:
 // pinned host staging and the device copy.  The staging area is rewritten
 // only once the copy that last read it has completed (its event), and a table
-// equal to the last one is not copied again.
+// equal to the last one is not copied again: another stream than the copy's
+// waits for the event instead.
 struct VctUpload {
   void* host = nullptr;
   size_t cap = 0;
   size_t bytes = 0;  // of the table last copied (0: none)
   hipEvent_t ev = nullptr;
+  hipStream_t stream = nullptr;  // of the copy
   VctBuf dev;
 };
 

@@ -55,8 +55,13 @@ static void free_buf(VctBuf& b) {
 }
 
 int vct_upload(vct_context* ctx, VctUpload& u, const void* data, size_t bytes) {
-  // the same table as the last one (staging still holds it): the device copy stands
-  if (u.ev && bytes == u.bytes && u.dev.p && memcmp(u.host, data, bytes) == 0) return VCT_OK;
+  // The same table as the last one (staging still holds it): the device copy
+  // stands.  A frame front that returned early leaves its copy in flight on
+  // the second stream, which nothing else orders before this one.
+  if (u.ev && bytes == u.bytes && u.dev.p && memcmp(u.host, data, bytes) == 0) {
+    if (u.stream != ctx->stream) VCT_HIP(hipStreamWaitEvent(ctx->stream, u.ev, 0));
+    return VCT_OK;
+  }
   u.bytes = 0;
   if (!u.ev) VCT_HIP(hipEventCreateWithFlags(&u.ev, hipEventDisableTiming));
   else VCT_HIP(hipEventSynchronize(u.ev));  // the last copy out of the staging area has completed
@@ -73,6 +78,7 @@ int vct_upload(vct_context* ctx, VctUpload& u, const void* data, size_t bytes) {
   memcpy(u.host, data, bytes);
   VCT_HIP(hipMemcpyAsync(u.dev.p, u.host, bytes, hipMemcpyHostToDevice, ctx->stream));
   VCT_HIP(hipEventRecord(u.ev, ctx->stream));
+  u.stream = ctx->stream;
   u.bytes = bytes;
   return VCT_OK;
 }
