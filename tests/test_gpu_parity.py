@@ -759,6 +759,39 @@ def test_trace_wide_blocks_ragged_viewport_matches_oracle(gpu_available, orc, dt
     assert err <= 2e-3
 
 
+@pytest.mark.parametrize("dtype", [L.RGBA8, L.FP16, L.BF16, L.FP32])
+@pytest.mark.parametrize("W,H", [(811, 653), (1013, 781)])
+def test_trace_block_shapes_ragged_viewport_matches_oracle(gpu_available, orc, dtype, W, H):
+    """The shapes of viewports past 2^19 pixels (811 = 50 x 16 + 11, 653 = 81 x 8
+    + 5: 128-pixel blocks) and past 3 * 2^18 (1013 = 42 x 24 + 5 = 63 x 16 + 5,
+    781 = 97 x 8 + 5: 192-pixel blocks in the 16-bit types): partial blocks on
+    both edges, block rows past a multiple of 8, whole blocks inside."""
+    say(f"trace parity, ragged {W}x{H} viewport, dtype={dtype}")
+    assert (1 << 19) < W * H and (W * H <= 3 << 18) == (W == 811)
+    res = 64
+    sc = SceneSpec("cornell", res=res, W=W, H=H, glass=True, phases=(True, True, True, True),
+                   fovy_deg=40.0)  # the box fills the window, edges included
+    with Context(W, H) as ctx:
+        sc.build(ctx, dtype)
+        ctx.render()
+        img = ctx.download_image()
+        gp, gn = ctx.download_gbuffer()
+        l0 = decode_level(ctx.download_level(0), dtype)
+        mips = {(l, d): decode_level(ctx.download_level(l, d), dtype) for l in range(1, 7) for d in range(6)}
+    pick = np.zeros((H, W), bool)
+    pick[-6:, :] = True
+    pick[:, -6:] = True
+    pick[392:400, 480:528] = True  # two whole 24-pixel blocks, three 16-pixel ones
+    pick.reshape(-1)[np.random.default_rng(W).choice(W * H, 2000, replace=False)] = True
+    pix = np.flatnonzero(pick & (gp[..., 3] != 0)).astype(np.int64)
+    assert pix.size > 8000
+    want, _ = orc.trace(np.float32, res, 7, l0, mips, gp, gn, sc.mat_records, sc.lights, sc.cam, sc.cube_size,
+                        cone_set=sc.cone_set, phases=sc.phases, pixels=pix)
+    err = np.abs(img.reshape(-1, 4)[pix, :3] - want[:, :3]).max()
+    say(f"  {pix.size} pixels, max-abs vs FP32 oracle = {err:.3e}")
+    assert err <= 2e-3
+
+
 @pytest.mark.parametrize("view_dir,lod,extra,dtype", [
     (0, 0.0, {}, L.RGBA8), (3, 1.5, {}, L.RGBA8), (5, 4.0, {}, L.FP16),
     # the camera inside the box: clipped walls drawn as fans, in draw order
