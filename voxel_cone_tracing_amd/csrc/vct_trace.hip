@@ -1375,26 +1375,42 @@ int vct_trace_into(vct_context* ctx, const float4* gpos, const float4* gnrm, flo
   return vct_trace_select(ctx, gpos, gnrm, out, W, H, demodulate, step_counter, sel);
 }
 
-// Launches the marcher of one block shape: the viewport, or one workgroup
-// per chunk of the largest the list can be.
+// Launches the marcher over the viewport in blocks of one shape.
 template <int DT, class SH>
-static void launch_shape(vct_context* ctx, const TraceArgs& A, const TraceSelect& sel, int W, int H) {
+static void launch_frame(vct_context* ctx, const TraceArgs& A, int W, int H) {
   constexpr int bw = 8 * SH::BX, bh = 8 * (SH::NSUB / SH::BX);
-  dim3 grid((W + bw - 1) / bw, (H + bh - 1) / bh);
-  if (sel.pix_list) {
-    grid = dim3((sel.npix_list + SH::NPIX - 1) / SH::NPIX);
-    hipLaunchKernelGGL((trace_list_kernel<DT, SH>), grid, dim3(256), 0, ctx->stream, A);
-  } else if (sel.tile_list) {
-    grid = dim3((sel.grid_stride == 2 ? 4u : 16u) / SH::NSUB * sel.max_tiles);
-    hipLaunchKernelGGL((trace_list_kernel<DT, SH>), grid, dim3(256), 0, ctx->stream, A);
-  } else {
-    hipLaunchKernelGGL((trace_frame_kernel<DT, SH>), grid, dim3(256), 0, ctx->stream, A);
-  }
+  hipLaunchKernelGGL((trace_frame_kernel<DT, SH>), dim3((W + bw - 1) / bw, (H + bh - 1) / bh), dim3(256), 0,
+                     ctx->stream, A);
+}
+
+// Launches it over a list: one workgroup per chunk of the largest the list can be.
+template <int DT, class SH>
+static void launch_list(vct_context* ctx, const TraceArgs& A, const TraceSelect& sel) {
+  static_assert(4 % SH::NSUB == 0, "chunks of a listed tile's 16 sub-blocks, or of the 4 of its odd-odd pixels");
+  const uint32_t chunks = sel.pix_list ? (sel.npix_list + SH::NPIX - 1) / SH::NPIX
+                                       : (sel.grid_stride == 2 ? 4u : 16u) / SH::NSUB * sel.max_tiles;
+  hipLaunchKernelGGL((trace_list_kernel<DT, SH>), dim3(chunks), dim3(256), 0, ctx->stream, A);
 }
 
 template <int DT>
 static int launch_trace(vct_context* ctx, const TraceArgs& A, const TraceSelect& sel, int W, int H, bool wide) {
   if ((sel.pix_list && sel.npix_list == 0) || (!sel.pix_list && sel.tile_list && sel.max_tiles == 0)) return VCT_OK;
+  // A pixel list runs beside other launches: workgroups of 64 pixels up to 2^18
+  // of them (the learned frame's 57,600 probes, 3.257 -> 3.244 ms), else of 128.
+  if (sel.pix_list || sel.tile_list) {
+    if (!wide) {
+      launch_list<DT, ShapeFull>(ctx, A, sel);
+      return VCT_OK;
+    }
+    if constexpr (DT != kRgba8Unorm) {  // (the demodulated lists are lists of tiles)
+      if (sel.pix_list && sel.npix_list <= 1u << 18) {
+        launch_list<DT, ShapeSmall>(ctx, A, sel);
+        return VCT_OK;
+      }
+    }
+    launch_list<DT, ShapeTile>(ctx, A, sel);
+    return VCT_OK;
+  }
   // The 256 CUs hold about 1280 workgroups of any shape at once, so a viewport
   // of few workgroups runs a part-empty last round whose length is that of one
   // workgroup, all its pixels' cones: small viewports take small workgroups.
@@ -1402,14 +1418,12 @@ static int launch_trace(vct_context* ctx, const TraceArgs& A, const TraceSelect&
   // a pixel: 0.78 ms in workgroups of 192 pixels, 0.53 of 128, 0.44 of 64;
   // 855x512 FP16 0.69, 0.57, 0.50; 1001x563 FP32 0.35 of 128, 0.38 of 64), up to
   // 3 * 2^18 128 (974x700 FP16: 0.182 of 64, 0.160 of 128, 0.162 of 192; 1363x767
-  // BF16: 1.26, 1.27, 1.24).  A pixel list runs beside other launches: 64 up to
-  // 2^18 pixels (the learned frame's 57,600 probes, 3.257 -> 3.244 ms).
-  const size_t npix = sel.pix_list ? (size_t)sel.npix_list : (size_t)W * H;
-  if (wide && !sel.tile_list && npix <= (sel.pix_list ? 1u << 18 : 1u << 19))
-    launch_shape<DT, ShapeSmall>(ctx, A, sel, W, H);
-  else if (wide && (sel.pix_list || sel.tile_list || npix <= 3u << 18)) launch_shape<DT, ShapeTile>(ctx, A, sel, W, H);
-  else if (wide) launch_shape<DT, typename WideOf<DT>::type>(ctx, A, sel, W, H);
-  else launch_shape<DT, ShapeFull>(ctx, A, sel, W, H);
+  // BF16: 1.26, 1.27, 1.24).
+  const size_t npix = (size_t)W * H;
+  if (!wide) launch_frame<DT, ShapeFull>(ctx, A, W, H);
+  else if (npix <= 1u << 19) launch_frame<DT, ShapeSmall>(ctx, A, W, H);
+  else if (npix <= 3u << 18) launch_frame<DT, ShapeTile>(ctx, A, W, H);
+  else launch_frame<DT, typename WideOf<DT>::type>(ctx, A, W, H);
   return VCT_OK;
 }
 

@@ -258,15 +258,6 @@ __device__ __forceinline__ void vox_edges(const Rec& s, int i, int j, VEdges& e)
   e.ey[2] = by - ay;
 }
 
-// Coverage of a pixel from its edge values (top-left rule).
-__device__ __forceinline__ bool vox_covers(const VEdges& e) {
-  if (e.w[0] < 0 || e.w[1] < 0 || e.w[2] < 0) return false;
-  if (e.w[0] == 0 && !top_left(e.ex[0], e.ey[0])) return false;
-  if (e.w[1] == 0 && !top_left(e.ex[1], e.ey[1])) return false;
-  if (e.w[2] == 0 && !top_left(e.ex[2], e.ey[2])) return false;
-  return true;
-}
-
 // Fragment at pixel (i, j) of the triangle's 2res x 2res raster given its
 // edge values (wa, wb, wc): coverage, voxel (Morton index) and colour.
 // Returns false if the pixel is not covered or the voxel falls outside the
