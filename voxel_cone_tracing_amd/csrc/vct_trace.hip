@@ -539,10 +539,14 @@ __device__ __forceinline__ float3 refract3(float3 I, float3 N, float eta) {
 // job codes: 0..15 diffuse cone k, then:
 constexpr int kJobSpecular = 16, kJobRefraction = 17, kJobShadow = 18;  // kJobShadow + light
 constexpr int kMaxJobs = kJobShadow + VCT_MAX_LIGHTS;
-// idle lanes of a wave that trigger a refill: a refill costs the whole wave
-// its set-up; measured on the 1M-triangle soup at 2560x1440, FP16 / RGBA8:
-// 16 -> 1.90 / 2.02 ms, 24 -> 1.90 / 2.06, 32 -> 1.96 / 2.11, 40 -> 2.04 / 2.21
-constexpr int kRefillMin = 16;
+// Idle lanes of a wave that trigger a refill: a refill costs the whole wave its
+// set-up.  1M-triangle soup at 2560x1440, FP16 / RGBA8: 16 -> 1.90 / 2.02 ms, 24
+// -> 1.90 / 2.06, 32 -> 1.96 / 2.11, 40 -> 2.04 / 2.21.  FP32, whose step is the
+// longest, waits for more of them (50,000-triangle soup at 128^3; 16, 24, 32):
+// 1001x563 1.13, 1.10, 1.11 ms, 2560x1440 3.72, 3.71, 3.85; in blocks of 64
+// pixels 200x150 with two shadows 0.472, 0.458, 0.444, 640x360 0.810, 0.796, 0.780.
+template <int DT, int NPIX>
+constexpr int kRefillMin = DT != VCT_FP32 ? 16 : (NPIX == 64 ? 32 : 24);
 
 // Block shapes: pixels per workgroup and the shadow-light slots in LDS.
 // Cones are short in cluttered scenes (6.2 steps per cone of a covered pixel
@@ -838,7 +842,7 @@ __device__ __forceinline__ void shade_block(const TraceArgs& A, Where&& where, S
     for (;;) {
       const bool need = cur < 0 && !drained;
       const unsigned long long want = __ballot(need);
-      if (!want || (busy && __popcll(want) < kRefillMin)) break;
+      if (!want || (busy && __popcll(want) < kRefillMin<DT, SH::NPIX>)) break;
       const int first = __ffsll((long long)want) - 1;
       int base = 0;
       if (lane == first) base = atomicAdd(&L->next_item, __popcll(want));
