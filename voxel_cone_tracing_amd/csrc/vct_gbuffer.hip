@@ -313,7 +313,7 @@ struct alignas(16) GFan {
 };
 static_assert(sizeof(GFan) == 64, "GFan must be 64 bytes");
 
-constexpr int kTile = 32;  // screen tile edge in pixels (one workgroup per tile)
+constexpr int kTile = 32;  // screen tile edge in pixels
 
 __device__ __forceinline__ GSetup g_setup_of(const GRec& r) {
   GSetup s;
@@ -1427,7 +1427,7 @@ int vct_launch_gbuffer_phase(vct_context* ctx, int phase) {
 
 // The voxel view of the last rasterised G-buffer, blended in draw order: the
 // tile lists sorted by draw order (a segmented radix sort, one segment per
-// tile), then one workgroup per tile.
+// tile), then four workgroups per tile.
 int vct_launch_voxel_view(vct_context* ctx) {
   const auto& F = ctx->g_frame;
   const int W = F.W, H = F.H;

@@ -783,7 +783,7 @@ __device__ __forceinline__ void shade_block(const TraceArgs& A, Where&& where, S
   }
   __syncthreads();
   if (grp < SH::NSUB) {
-    // the block's shading pixels, compacted in sub-block order
+    // the block's shading pixels, compacted in the order of their keys
     int total = 0;
     bool refr = false;
 #pragma unroll
@@ -1001,10 +1001,10 @@ __device__ __forceinline__ void shade_block(const TraceArgs& A, Where&& where, S
 // Work of a launch: the whole viewport (trace_frame_kernel, one workgroup per
 // block of NSUB 8x8 sub-blocks side by side), or a device-side list of pixels
 // (NPIX per chunk) or tiles (16 sub-blocks of 8x8 pixels per tile, or 4 of
-// 8x8 odd-odd grid points, NSUB per chunk) for trace_list_kernel.  5 waves per
-// SIMD (96 VGPRs; the 8- and 16-bit storage paths fit without scratch, the
-// FP32 path keeps 20 bytes per lane in scratch at this occupancy): the 12
-// paired loads of a three-map level are in flight together.
+// 8x8 odd-odd grid points, NSUB per chunk) for trace_list_kernel.  At the waves
+// of kTraceWaves no storage type needs scratch: the 12 paired loads of a
+// three-map level (16-bit storage; 6 for RGBA8, FP32 one map's 8) are in flight
+// together.
 template <int DT, class SH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kTraceWaves<DT>))) void trace_frame_kernel(TraceArgs A) {
   __shared__ ShadeLds<SH> s_shade;
@@ -1312,9 +1312,10 @@ void vct_cone_set_table(int set, ConeSet& cs) {
   }
 }
 
-// Rebuilds the x-paired copy of the volume when the volume has changed since
-// it was last built (16-bit and RGBA8 storage).  The mip pass calls it last;
-// the marcher calls it again for volumes written since (uploads).
+// The marcher's copy of the volume (x-paired 16-bit, tiled RGBA8 storage): its
+// layout, the maps of its levels, and its rebuilding when the volume has changed
+// since it was last built.  The mip pass builds it last; the marcher calls
+// vct_ensure_pairs again for volumes written since (uploads).
 int vct_pair_layout(vct_context* ctx) {
   const uint64_t bpe = dtype_bytes(ctx->dtype);
   uint64_t bytes = 0;

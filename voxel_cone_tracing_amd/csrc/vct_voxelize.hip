@@ -745,7 +745,8 @@ __device__ __forceinline__ uint32_t replay_step(uint32_t stored, float vx, float
 
 // The brick lists' capacity: a brick whose range [off, off + count) runs past
 // `cap` entries walks the packed brick boxes of all `ntri` triangles and keeps
-// those that contain it (the same triangles its list would hold).
+// those that contain it: the triangles of its list, and ones that its list
+// leaves out because they do not reach it, which give no fragment in it.
 struct ListCap {
   const uint2* boxes;
   uint32_t ntri;
