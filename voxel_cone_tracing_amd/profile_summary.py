@@ -5,8 +5,8 @@ Kernel times (from `rocprofv3 --kernel-trace --stats --output-format csv`):
     python -m voxel_cone_tracing_amd.profile_summary times --trace DIR/run_kernel_trace.csv \\
         --cmd "<the profiled command>" --out profiles/kernel_times_soup256.md
 
-Counter ratios (VALU active, TA busy, stalls, instructions per wave) from
-`rocprofv3 --pmc` runs of SQ, TA and GRBM counters:
+Counter ratios (VALU active, TA busy, L1 lookups, stalls, instructions per wave)
+from `rocprofv3 --pmc` runs of SQ, TA, TCP and GRBM counters:
 
     python -m voxel_cone_tracing_amd.profile_summary counters --dirs DIR1 DIR2 ... \\
         --cmd "<the profiled commands>" --out profiles/kernel_counters_soup256.md
@@ -140,12 +140,13 @@ def cmd_traffic(a):
 
 
 def cmd_counters(a):
-    """Utilisation of the listed kernels from SQ / TA / GRBM counter runs.
+    """Utilisation of the listed kernels from SQ / TA / TCP / GRBM counter runs.
 
     SQ counters are sums over the shader engines, GRBM_GUI_ACTIVE a sum over
     the XCDs; with N CUs and X XCDs:
       VALU active = SQ_ACTIVE_INST_VALU / N / (GRBM_GUI_ACTIVE / X)
       TA busy   = TA_TA_BUSY_sum / N / (GRBM_GUI_ACTIVE / X)
+      L1 lookups / cycle = TCP_TOTAL_CACHE_ACCESSES_sum / N / (GRBM_GUI_ACTIVE / X)
       wait      = SQ_WAIT_ANY / SQ_WAVE_CYCLES (share of wave time stalled)
     and instructions per wave are the SQ_INSTS_* counts over SQ_WAVES.
     VALU active is a ratio of counter sums, not a utilisation bounded by 1:
@@ -162,11 +163,12 @@ def cmd_counters(a):
              f"over launches, {a.cus} CUs in {a.xcds} XCDs.  VALU active = SQ_ACTIVE_INST_VALU / CUs / "
              "(GRBM_GUI_ACTIVE / XCDs), a ratio of counter sums that can pass 100 %: it shows where VALU work "
              "fills the issue slots, not that the ALUs bound the kernel; TA busy = TA_TA_BUSY_sum / CUs / "
-             "(GRBM_GUI_ACTIVE / XCDs); stalled = SQ_WAIT_ANY / SQ_WAVE_CYCLES; per-wave counts = "
-             "SQ_INSTS_* / SQ_WAVES.", "",
-             "| kernel | grid (threads) | VALU active | TA busy | stalled | VALU / wave | SALU / wave | LDS / wave "
-             "| VMEM rd / wave | LDS bank conflicts / LDS instr |",
-             "|---|---:|---:|---:|---:|---:|---:|---:|---:|---:|"]
+             "(GRBM_GUI_ACTIVE / XCDs); L1 lookups (cache lines) per CU and cycle from "
+             "TCP_TOTAL_CACHE_ACCESSES_sum likewise, per wave load over SQ_INSTS_VMEM_RD; stalled = SQ_WAIT_ANY / "
+             "SQ_WAVE_CYCLES; per-wave counts = SQ_INSTS_* / SQ_WAVES.", "",
+             "| kernel | grid (threads) | VALU active | TA busy | L1 lookups / cycle | L1 lookups / load | stalled "
+             "| VALU / wave | SALU / wave | LDS / wave | VMEM rd / wave | LDS bank conflicts / LDS instr |",
+             "|---|---:|---:|---:|---:|---:|---:|---:|---:|---:|---:|---:|"]
 
     def mean(c, n):
         v = c.get(n)
@@ -190,7 +192,10 @@ def cmd_counters(a):
 
         wc, wa = mean(c, "SQ_WAVE_CYCLES"), mean(c, "SQ_WAIT_ANY")
         li, bc = mean(c, "SQ_INSTS_LDS"), mean(c, "SQ_LDS_BANK_CONFLICT")
+        tl, vr = mean(c, "TCP_TOTAL_CACHE_ACCESSES_sum"), mean(c, "SQ_INSTS_VMEM_RD")
         lines.append(f"| `{k}` | {g} | {frac('SQ_ACTIVE_INST_VALU')} | {frac('TA_TA_BUSY_sum')} | "
+                     f"{f'{tl / a.cus / (gui / a.xcds):.2f}' if tl is not None and gui else ''} | "
+                     f"{f'{tl / vr:.1f}' if tl is not None and vr else ''} | "
                      f"{f'{wa / wc:.0%}' if wc and wa is not None else ''} | {per_wave('SQ_INSTS_VALU')} | "
                      f"{per_wave('SQ_INSTS_SALU')} | {per_wave('SQ_INSTS_LDS')} | {per_wave('SQ_INSTS_VMEM_RD')} | "
                      f"{f'{bc / li:.2f}' if li and bc is not None else ''} |")
