@@ -558,12 +558,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     bf16x8 hf[2][2];
     uint32_t m1T[2] = {0u, 0u}, m2[2] = {0u, 0u}, m2T[2] = {0u, 0u};
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int nt = 0; nt < 3; ++nt) xT[t][nt] = pack4(mfma32(x[t][nt >> 1], eye[nt & 1], z));
-      // the product would spread an infinite or NaN feature (0 * NaN) over its
-      // sample's others: such tiles are read from the rows instead
-      if (__ballot((nonfinite(x[t][0]) | nonfinite(x[t][1])) != 0u)) {
+    // the product spreads an infinite or NaN feature over its sample's others
+    // (0 * NaN): such tiles are read from the rows instead
+    if (__ballot((nonfinite(x[0][0]) | nonfinite(x[0][1]) | nonfinite(x[1][0]) | nonfinite(x[1][1])) != 0u)) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int nt = 0; nt < 3; ++nt) {
           uint32_t v[4];
@@ -574,7 +576,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
           }
           xT[t][nt] = make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
         }
-      }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
       uint2 p[4];
 #pragma unroll
       for (int mt = 0; mt < 4; ++mt) {
