@@ -290,9 +290,9 @@ int vct_mlp_forward(vct_ctx ctx, const float* features, uint32_t n, float* out);
  * context's stream), after vct_mlp_set_params / vct_mlp_init has completed on
  * it (vct_sync).  The rows are read where they are, so calls may overlap in
  * time; n above VCT_MLP_NOALLOC_MAX_ROWS is rejected with VCT_ERR_LIMIT.  out
- * may overlap features: the outputs then pass through a staging array of the
- * context (3 MiB, allocated with its parameters), so two such calls on one
- * context must not run at the same time.  Outputs equal vct_mlp_forward's. */
+ * may overlap features: the outputs then pass through the library's staging
+ * array of that GPU, so two such calls on one GPU must not run at the same
+ * time.  Outputs equal vct_mlp_forward's. */
 #define VCT_MLP_NOALLOC_MAX_ROWS 262144
 int vct_mlp_forward_noalloc(vct_ctx ctx, const float* features, uint32_t n, float* out, void* stream);
 /* Loss mean((albedo * (y - target))^2) over n samples and 3 channels and its

@@ -311,7 +311,6 @@ struct vct_context {
 
   // learned upsampler
   VctBuf mlp_params, mlp_m1, mlp_m2, mlp_packed, mlp_bias, mlp_grad, mlp_partial;
-  VctBuf mlp_stage;  // vct_mlp_forward_noalloc: outputs of a call whose out overlaps its features
   bool mlp_ready = false;
   int mlp_step = 0;
   VctBuf low_gpos, low_gnrm, low_img, full_target, sample_pix;

@@ -430,9 +430,17 @@ constexpr uint32_t kRowsPerWave = 32;     // rows a wave takes at a time
 // 6.1 us with 256 workgroups, 7.7 with 512; 262,144: 14.8 and 13.7, 1024 16.3).
 constexpr uint32_t kForwardMin = 256, kForwardMax = 512;
 
+// Outputs of a no-allocation call that may not write its caller's buffer yet
+// (out overlaps features).  Part of the library on each GPU, so such a call
+// allocates nothing, nor does a context for it (3 MiB a context cost its
+// set-up 0.5 to 1.2 ms); the kernels name it, host code never does.
+static __device__ float staged_out[(size_t)VCT_MLP_NOALLOC_MAX_ROWS * kOut];
+
+// Y null: to staged_out.
 template <typename T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void mlp_forward_kernel(
     MlpDev P, const T* __restrict__ X, uint32_t n, float* __restrict__ Y) {
+  float* const out = Y ? Y : staged_out;
   const int lane = threadIdx.x & 63, col = lane & 15;
   const uint32_t first = (blockIdx.x * 4u + (threadIdx.x >> 6)) * kRowsPerWave, step = gridDim.x * 4u * kRowsPerWave;
   if (first >= n) return;
@@ -450,7 +458,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
       const floatx4 y = net_forward(N, x[t][0], x[t][1]);
       const uint32_t row = base + 16u * t + (uint32_t)lane;
       if (lane < 16 && row < n) {
-        float* o = Y + (size_t)row * 3;
+        float* o = out + (size_t)row * 3;
         o[0] = y[0];
         o[1] = y[1];
         o[2] = y[2];
@@ -459,10 +467,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
   }
 }
 
-__global__ __launch_bounds__(256) void copy_f32_kernel(const float* __restrict__ src, uint32_t n,
-                                                       float* __restrict__ dst) {
+__global__ __launch_bounds__(256) void mlp_unstage_kernel(uint32_t n, float* __restrict__ dst) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  if (i < n) dst[i] = src[i];
+  if (i < n) dst[i] = staged_out[i];
 }
 
 // ---- training: forward + backward, a wave per 32 samples --------------------------
@@ -1182,7 +1189,7 @@ int mlp_ensure(vct_context* ctx) {
   if ((rc = vct_ensure(ctx->mlp_packed, kPacked * 2, ctx))) return rc;
   if ((rc = vct_ensure(ctx->mlp_bias, 144 * 4, ctx))) return rc;
   if ((rc = vct_ensure(ctx->mlp_grad, (kParams + 1) * 4, ctx))) return rc;
-  return vct_ensure(ctx->mlp_stage, (size_t)VCT_MLP_NOALLOC_MAX_ROWS * kOut * 4, ctx);
+  return VCT_OK;
 }
 
 int mlp_pack(vct_context* ctx) {
@@ -1206,7 +1213,8 @@ int need_mlp(vct_context* ctx) {
   return VCT_OK;
 }
 
-// The forward pass of n rows on a stream; allocates nothing.
+// The forward pass of n rows on a stream (Y null: to staged_out, which holds
+// VCT_MLP_NOALLOC_MAX_ROWS of them); allocates nothing.
 template <typename T>
 int launch_forward(vct_context* ctx, const T* X, uint32_t n, float* Y, hipStream_t stream) {
   const uint32_t groups = (uint32_t)(((uint64_t)n + 4 * kRowsPerWave - 1) / (4 * kRowsPerWave));
@@ -1640,13 +1648,12 @@ int vct_mlp_forward_noalloc(vct_ctx ctx, const float* features, uint32_t n, floa
   if ((rc = need_mlp(ctx))) return rc;
   const hipStream_t st = stream ? (hipStream_t)stream : ctx->stream;
   // The kernel reads the rows and writes the outputs in no order of its own,
-  // so outputs that overlap the rows wait in mlp_stage until every row is read.
+  // so outputs that overlap the rows wait in staged_out until every row is read.
   const uintptr_t f = (uintptr_t)features, o = (uintptr_t)out;
   const bool overlap = f < o + (uintptr_t)n * (kOut * 4) && o < f + (uintptr_t)n * (kIn * 4);
   if (!overlap) return launch_forward(ctx, features, n, out, st);
-  if ((rc = launch_forward(ctx, features, n, (float*)ctx->mlp_stage.p, st))) return rc;
-  hipLaunchKernelGGL(copy_f32_kernel, dim3((n * kOut + 255) / 256), dim3(256), 0, st, (const float*)ctx->mlp_stage.p,
-                     n * kOut, out);
+  if ((rc = launch_forward(ctx, features, n, (float*)nullptr, st))) return rc;
+  hipLaunchKernelGGL(mlp_unstage_kernel, dim3((n * kOut + 255) / 256), dim3(256), 0, st, n * kOut, out);
   VCT_HIP(hipGetLastError());
   return VCT_OK;
 }

@@ -526,7 +526,7 @@ int vct_destroy(vct_ctx ctx) {
                     &ctx->scan_tmp, &ctx->g_scan_tmp, &ctx->counters, &ctx->setup, &ctx->g_list, &ctx->g_pos,
                     &ctx->g_nrm, &ctx->image, &ctx->g_count, &ctx->g_off, &ctx->g_recs, &ctx->g_merge,
                     &ctx->mlp_params, &ctx->mlp_m1, &ctx->mlp_m2, &ctx->mlp_packed, &ctx->mlp_bias,
-                    &ctx->mlp_grad, &ctx->mlp_partial, &ctx->mlp_stage, &ctx->low_gpos, &ctx->low_gnrm, &ctx->low_img,
+                    &ctx->mlp_grad, &ctx->mlp_partial, &ctx->low_gpos, &ctx->low_gnrm, &ctx->low_img,
                     &ctx->full_target, &ctx->sample_pix, &ctx->train_X, &ctx->train_A, &ctx->train_Y,
                     &ctx->train_valid, &ctx->probe_pix, &ctx->probe_val, &ctx->fb_list, &ctx->fb_pix,
                     &ctx->fb_list2, &ctx->fb_pix2, &ctx->fb_flag, &ctx->half_img, &ctx->probe_pix2,
