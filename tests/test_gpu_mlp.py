@@ -411,11 +411,12 @@ def test_tile_check_and_refinement_hold_40db(gpu_available, half):
 
 @pytest.mark.parametrize("W,H", [(96, 64), (324, 164)])
 def test_rgba8_traced_pixels_match_the_plain_frame(gpu_available, W, H):
-    """RGBA8 storage: the learned form's launches scale each texel by 1/255
-    before weighting it, the plain frame the weighted sum, so a traced pixel
-    differs from the plain frame's by rounding alone: 2^-24 in each of the ~20
-    operations from a texel to a pixel, over a sum of ten cones, is at most
-    1.2e-5."""
+    """RGBA8 storage: two roundings of a sample (each texel scaled by 1/255
+    before it is weighted, as the learned form's demodulated traces do, or the
+    weighted sum, as the plain frame does) differ by 2^-24 in each of the ~20
+    operations from a texel to a pixel, over a sum of ten cones at most 1.2e-5;
+    a traced pixel holds that bound
+    (test_traced_pixels_equal_the_plain_frame: it is the plain frame's)."""
     sc = SceneSpec("soup", res=64, ntri=20000, W=W, H=H, mu=-4.0)
     with Context(W, H) as ctx:
         sc.build(ctx, L.RGBA8)

@@ -2,10 +2,11 @@
 vct_mlp_forward, through the C ABI.
 
 Inputs and outputs are device buffers the test allocates itself (hipMalloc
-through ctypes); the entry point stages the BF16 rows in the library's fixed
-per-GPU array.  Two calls in a row, the second with fewer rows, must each
-equal vct_mlp_forward's output bit for bit (the second call must not see
-rows the first left behind); more rows than the array holds are rejected.
+through ctypes); the entry point reads the rows where they are.  Two calls in a
+row, the second with fewer rows, must each equal vct_mlp_forward's output bit
+for bit (the second call must not see rows the first left behind), as must
+calls whose output lies inside the features and calls in flight at the same
+time; more rows than VCT_MLP_NOALLOC_MAX_ROWS are rejected.
 """
 from __future__ import annotations
 

@@ -483,10 +483,10 @@ __global__ __launch_bounds__(256) void mlp_unstage_kernel(uint32_t n, float* __r
 // gradients up.  Partial sums go to `partial` [gridDim.x][kParams + 1] and
 // are reduced in a fixed order by mlp_adam_kernel (deterministic).  A step of
 // 8,192 samples (64 workgroups here) is one chain of dependent reads and
-// products per wave: 13.8 us, where every operand staged through LDS behind
-// ten barriers took 19.6 and the minibatch gather before it 5 (the weights
-// staged in LDS at once measured 13.0, the rows read ahead of them 14.5 with
-// spills).
+// products per wave: 14.6 us (14.5 without the look for non-finite features),
+// where every operand staged through LDS behind ten barriers took 19.6 and the
+// minibatch gather before it 5 (the weights staged in LDS at once measured
+// 13.0, the rows read ahead of them 14.5 with spills, both against 13.8).
 struct TrainArgs {
   MlpDev P;
   const uint16_t* X;  // [rows][64]
